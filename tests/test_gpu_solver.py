@@ -419,6 +419,33 @@ def test_coarse_solve_planes_wider_than_1024_dofs():
     assert its < 400 and true_res < 1.5e-6
 
 
+@pytest.mark.parametrize('shape, blocks', [((24, 48, 24), 1), ((32, 48, 32), 2), ((56, 64, 56), 3), ((56, 64, 64), 4),
+                                           ((128, 136, 128), 14)])
+def test_coarse_factorisation_at_block_edges(shape, blocks):
+    """The plane blocks' inverses with one 64-wide pivot block, with two, with three and no padding (192 DOFs per
+    plane), with four and the last one partly padding, and with fourteen: the coarsest solve's residual, the
+    product K_c x from the coarsest K*u.  An SPD block inverted without pivoting leaves a residual of
+    about its condition number (below 1e5 here) times the unit roundoff: bound 1e-10."""
+    import torch
+    from top_gpu_on_matlab_amd.model import cuboid_model
+    from top_gpu_on_matlab_amd.solver import Solver
+    s = Solver(cuboid_model(*shape, 1, precision='fp64'))
+    L = s.num_levels
+    c = s.levels[-1]
+    plane = 3 * (c['resY'] + 1) * (c['resZ'] + 1)
+    assert -(-plane // 64) == blocks
+    e = np.arange(int(np.prod(shape)))
+    ey, ex, ez = e % shape[0], (e // shape[0]) % shape[1], e // (shape[0] * shape[1])
+    x = 0.12 + 0.05 * np.sin(ex / 7.0) * np.cos(ey / 5.0) * np.sin(ez / 6.0 + 1)
+    s.set_modulus(1e-6 + x ** 3 * (1 - 1e-6))
+    s.assemble()
+    r = torch.randn(s.ndof(L), generator=torch.Generator().manual_seed(5), dtype=torch.float64).cuda()
+    for persistent in (True, False):
+        s.set_tuning(coarse_persistent=persistent)
+        res = float((s.kbyu(s.coarse_solve(r), L) - r).norm() / r.norm())
+        assert res < 1e-10, (persistent, res)
+
+
 def test_reassembly_is_bitwise_reproducible():
     """Assembling the same moduli again must give bitwise the same hierarchy: coarse element
     matrices, Jacobi diagonals, coarsest factorisation (checked through its solve) and V-cycle.

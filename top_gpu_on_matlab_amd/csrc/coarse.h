@@ -8,9 +8,9 @@
 //   chain A, p = 0 .. m-1:    S_p = A_pp - A_{p,p-1} N_{p-1},     N_p = S_p^-1 A_{p,p+1}
 //   chain B, q = P-1 .. m+1:  S_q = A_qq - A_{q,q+1} N_{q+1},     N_q = S_q^-1 A_{q,q-1}
 //   separator:                S_m = A_mm - A_{m,m-1} N_{m-1} - A_{m,m+1} N_{m+1}
-// Each S_p^-1 is formed in place by a blocked Gauss-Jordan sweep (64-wide pivot blocks: the pivot
-// block's inverse in LDS, the column panel, then a rank-64 update of the whole plane block on the
-// matrix cores); the two chains' planes of a step share every launch.  The solve operators are
+// Each S_p^-1 is formed by a blocked symmetric sweep (64-wide pivot blocks, one launch each: the rank-64
+// update of the plane block's lower triangle on the matrix cores, with the next pivot block's inverse
+// formed by the workgroup that updates it); the two chains' planes of a step share every launch.  The solve operators are
 //   forward  F_p = S_p^-1 A_{p,p-1} (chain A), S_q^-1 A_{q,q+1} (chain B), [S_m^-1 A_{m,m-1} | S_m^-1 A_{m,m+1}]
 //   backward B_p = N_p
 // and a solve is c = blockdiag(S_p^-1) b, the forward recurrences z_p = c_p - F_p z_{p-1|p+1} of both
@@ -53,7 +53,7 @@ struct CoarseSolver {
     DevBuf<double> dnV, upV;        // couplings to the previous / next plane, 27 per DOF row
     DevBuf<int32_t> dnC, upC;       // their column (local DOF in that plane)
     DevBuf<double> Fop, Bop;
-    DevBuf<double> T, Rw, Dk;       // sweep work: column panel, old pivot row, pivot inverse (2 planes)
+    DevBuf<double> W, Dk;           // sweep work: two step buffers and two pivot inverses for each of two planes
     DevBuf<double> bb, yy;
     DevBuf<double> xx;  // the persistent solve's separator and backward results (yy: its forward ones)
     DevBuf<int> info;

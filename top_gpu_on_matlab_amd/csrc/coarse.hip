@@ -1,6 +1,7 @@
 // Coarsest-level direct solver: twisted block-Schur-complement chain on the device (see coarse.h).
 #include "coarse.h"
 
+#include <climits>
 #include <cstring>
 
 namespace tg {
@@ -127,186 +128,408 @@ __global__ __launch_bounds__(256) void k_schur(const SchurProb A, const SchurPro
     q.S[i * q.np + j] -= acc;
 }
 
-// ---- blocked Gauss-Jordan sweep: S <- S^-1 in place, pivot blocks K = 0 .. nb-1 -------------------------
-// Per pivot block K (with D = S_KK^-1, computed from the current S):
-//   S_IJ -= S_IK D S_KJ (I, J != K),  S_IK <- S_IK D,  S_KJ <- -D S_KJ,  S_KK <- D,
-// which after the last block leaves the inverse (S is SPD, so every pivot block is the SPD Schur
-// complement of the blocks already swept and no pivoting is needed).  k_sweep_panel forms T_I = S_IK D
-// and copies the old pivot row Rw_I = S_KI; k_sweep_update then writes every block from T, Rw and D, so
-// no block is read after another workgroup has overwritten it.
+// ---- blocked symmetric sweep: S <- S^-1 in place of an SPD plane block, pivot blocks K = 0 .. nb-1 --------
+// Per pivot block K, with D = S_KK^-1 of the current S:
+//     S_IJ -= S_IK D S_KJ (I, J != K),  S_IK <- S_IK D,  S_KJ <- D S_KJ,  S_KK <- -D,
+// which leaves -S^-1 after the last block.  S is SPD, so every pivot block is the SPD Schur complement of
+// the blocks already swept and no pivoting is needed; and the matrix stays symmetric after every pivot
+// block, so only its lower block triangle is kept (210 instead of 392 workgroups for the two chains of
+// 896-wide planes: at most one per CU) and a block above the diagonal is read as its mirror's transpose.
+// One launch per pivot block (k_sweep_step): each workgroup forms its own part of D S_KI and updates its
+// block from it, reading the previous launch's buffer and writing the other one, so that no block is read
+// after it was overwritten; and the workgroup of the next pivot block goes on to invert it, while the others
+// finish, so the next launch finds its D ready.  The chain of pivot blocks is what bounds the factorisation
+// (a step moves 10 MB and multiplies 0.2 GFLOP): the latency of one step, 17 x 14 times at 128 x 256 x 128.
+// A block is 16 tiles in the matrix instructions' register layout (below), so that a wavefront's loads are
+// whole cache lines and its LDS reads 16 bytes wide (row-major blocks, 64 rows 7 KB apart, took 10 us to load).
+// Measured there: 15.4 us per step (of which the inverse's chain of 64 pivots takes 7.5, the products 3 to 4
+// -- the FP64 matrix rate -- and the loads and the launch 2 to 3 each), 5.2 ms per assembly's 17 chain steps,
+// against 11.4 ms for a panel launch, every workgroup of which inverted the pivot block scalar by scalar (31 us),
+// and an update launch (17 us) per pivot block.
 struct SweepProb {
-    double *S;      // npad x npad, row-major
-    int64_t np;     // npad
-    int nb;         // npad / CB
-    double *T;      // npad x CB   (T_I = S_IK D)
-    double *Rw;     // CB x npad   (old pivot row block)
-    double *D;      // CB x CB
-    int *info;      // first non-positive pivot (1-based, 0 = none)
+    double *S;       // npad x npad, row-major: the block on entry, its inverse after the last step
+    double *W0, *W1; // the steps' buffers, in turn: the lower triangle's blocks one after the other, in tiles
+    int64_t np;      // npad
+    int nb;          // npad / CB
+    double *D;       // 2 x (CB x CB): inverses of the even and of the odd pivot blocks
+    int *info;       // INT_MAX - the first non-positive pivot (1-based); 0 = none
 };
 
-// 1 / x for a positive normal x: the hardware reciprocal estimate refined by two Newton-Raphson steps
-// (p <- p + p (1 - x p)), each of which squares the relative error.
-__device__ __forceinline__ double recip_nr(double x) {
-    double p = __builtin_amdgcn_rcp(x);
-    double e = fma(-x, p, 1.0);
-    p = fma(p, e, p);
-    e = fma(-x, p, 1.0);
-    return fma(p, e, p);
+// 1 / x for a positive normal x: the hardware reciprocal estimate p refined once, p (1 + e + e^2) with
+// e = 1 - x p, which cubes the relative error (three dependent operations; two Newton steps take four).
+__device__ __forceinline__ double recip_refined(double x) {
+    const double p = __builtin_amdgcn_rcp(x), e = fma(-x, p, 1.0);
+    return fma(p, fma(e, e, e), p);
 }
 
-// 64 x 64 SPD inverse by Gauss-Jordan in registers: thread t holds the 4 x 4 block at rows 4 (t / 16),
-// columns 4 (t % 16); each pivot's row and column pass through LDS (double-buffered, one barrier per
-// pivot).  Pivots go four at a time so that the pivot's place in a thread's block is static.  Every
-// entry takes the rank-1 update, and the threads holding row k or column k then overwrite those
-// entries (row k: -a_kj / a_kk, column k: a_ik / a_kk, pivot: 1 / a_kk).  Returns 1 + the first
-// non-positive pivot index (0 if none; such a pivot is replaced by 1).
-__device__ int gj_inverse64(double (&r)[4][4], double (*rowb)[CB], double (*colb)[CB]) {
-    const int t = threadIdx.x, ti = t >> 4, tj = t & 15, bi = 4 * ti, bj = 4 * tj;
+// MFMA f64 16x16x4 and the 16 x 16 tiles it works on.  Lane l = 16 q + c (q < 4, c < 16) holds, in the
+// result's registers r = 0..3, the entries (4 r + q, c).  That register layout is also the B operand's
+// for the four steps of a 16-deep product (step r takes B(4 r + q, c)), and as the A operand (step r
+// takes A(c, 4 r + q)) a tile X in it acts as X transposed.  So products chain without moving data.
+typedef double tg_tile __attribute__((ext_vector_type(4)));
+
+__device__ __forceinline__ tg_tile tile_fma(const tg_tile &xt, const tg_tile &b, tg_tile acc) {  // acc + X' B
+#pragma unroll
+    for (int r = 0; r < 4; ++r) acc = __builtin_amdgcn_mfma_f64_16x16x4f64(xt[r], b[r], acc, 0, 0, 0);
+    return acc;
+}
+
+// acc[j] += X' B_j for four tiles, the dependent steps of one tile apart by the other three's
+__device__ __forceinline__ void tile_fma4(const tg_tile &xt, const tg_tile (&b)[4], tg_tile (&acc)[4]) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc[j] = __builtin_amdgcn_mfma_f64_16x16x4f64(xt[r], b[j][r], acc[j], 0, 0, 0);
+}
+
+// The value of lane N of each row of 16 lanes, in every lane of that row.
+template <int N>
+__device__ __forceinline__ double row_lane(double x) {
+    return __builtin_amdgcn_update_dpp(0.0, x, 0x150 + N, 0xf, 0xf, true);
+}
+
+// The four rows of 16 lanes of x, each in all four rows: y[q] = the value of lane (q, c) in every lane
+// (., c).  Halves, then rows, swapped between two copies.
+__device__ __forceinline__ void row_copies(double x, double (&y)[4]) {
+    unsigned v[2][4];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        const unsigned u = h ? (unsigned)__double2hiint(x) : (unsigned)__double2loint(x);
+        const auto s = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+        const auto a = __builtin_amdgcn_permlane16_swap(s[0], s[0], false, false);
+        const auto b = __builtin_amdgcn_permlane16_swap(s[1], s[1], false, false);
+        v[h][0] = a[0];
+        v[h][1] = a[1];
+        v[h][2] = b[0];
+        v[h][3] = b[1];
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) y[i] = __hiloint2double((int)v[1][i], (int)v[0][i]);
+}
+
+// Pivot row I of the four rows y (rows 4 B .. 4 B + 3 of the tile, each lane's column), pivot 4 B + I.  In the
+// pivot's column, -1 in place of the pivot row's entry and 0 in place of the others' make the one update
+// right there too.  The products with the pivot row come before its scaling, so they do not wait for the
+// reciprocal.  bad: lanes that saw a pivot that is not positive.
+template <int B, int I>
+__device__ __forceinline__ void sweep_row4(double (&y)[4], int c, unsigned long long (&bad)[16]) {
+    constexpr int P = 4 * B + I;
+    const double piv = row_lane<P>(y[I]);
+    bad[P] = __ballot(!(piv > 0.0));
+    const double d = recip_refined(piv), yi = c == P ? -1.0 : y[I];
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+        if (j != I) y[j] = fma(-(row_lane<P>(y[j]) * yi), d, c == P ? 0.0 : y[j]);
+    y[I] = yi * d;
+}
+
+// Pivots 4 B .. 4 B + 3 of the tile's sweep: their rows (register B of the four rows of lanes) are swept in
+// copies that every lane has of its column, so that no pivot's step crosses lanes but by the row
+// broadcast; the other rows take the four pivots as one MFMA, S_r. - S_rB (D S_B.) and S_rB D in the
+// pivots' columns.
+template <int B>
+__device__ __forceinline__ void sweep_block4(tg_tile &t, int q, int c, unsigned long long (&bad)[16]) {
+    const double old = t[B];
+    double y[4];
+    row_copies(old, y);
+    sweep_row4<B, 0>(y, c, bad);
+    sweep_row4<B, 1>(y, c, bad);
+    sweep_row4<B, 2>(y, c, bad);
+    sweep_row4<B, 3>(y, c, bad);
+    const double fresh = q < 2 ? (q == 0 ? y[0] : y[1]) : (q == 2 ? y[2] : y[3]);
+    const bool in = (c >> 2) == B;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) t[r] = in ? 0.0 : t[r];
+    t = __builtin_amdgcn_mfma_f64_16x16x4f64(old, -fresh, t, 0, 0, 0);
+    t[B] = fresh;
+}
+
+// t <- t^-1 of an SPD 16 x 16 tile, in one wavefront; returns 1 + the first pivot that is not positive (or
+// NaN), 0 if there is none.
+__device__ __forceinline__ int inverse16(tg_tile &t) {
+    const int lane = threadIdx.x & 63, q = lane >> 4, c = lane & 15;
+    unsigned long long bad[16];
+    sweep_block4<0>(t, q, c, bad);
+    sweep_block4<1>(t, q, c, bad);
+    sweep_block4<2>(t, q, c, bad);
+    sweep_block4<3>(t, q, c, bad);
+    t = -t;
+    unsigned long long any = 0;
+#pragma unroll
+    for (int p = 0; p < 16; ++p) any |= bad[p];
+    if (any) {
+        for (int p = 0; p < 16; ++p)
+            if (bad[p]) return p + 1;
+    }
+    return 0;
+}
+
+// A tile in memory: registers 0 and 1 of the 64 lanes, then registers 2 and 3 (16 bytes a lane).
+constexpr int TILE = 256;  // doubles
+__device__ __forceinline__ tg_tile get_tile(const double *p) {
+    const double2 *v = reinterpret_cast<const double2 *>(p) + (threadIdx.x & 63);
+    const double2 x = v[0], y = v[64];
+    return tg_tile{x.x, x.y, y.x, y.y};
+}
+__device__ __forceinline__ void put_tile(double *p, const tg_tile &t) {
+    double2 *v = reinterpret_cast<double2 *>(p) + (threadIdx.x & 63);
+    v[0] = make_double2(t[0], t[1]);
+    v[64] = make_double2(t[2], t[3]);
+}
+// The transposed tile: a product with the unit tile (exact).
+__device__ __forceinline__ tg_tile transposed(const tg_tile &t, const tg_tile &unit) {
+    return tile_fma(t, unit, tg_tile{0.0, 0.0, 0.0, 0.0});
+}
+
+// The inverse of an SPD 64 x 64 block held by a workgroup of four wavefronts: wavefront w has rows 16 w ..
+// 16 w + 15 as tiles a[0..3].  The same sweep over four 16 x 16 pivot tiles.  At stage k wavefront k inverts
+// its diagonal tile in registers (no barrier inside) while the others pass S_kw, the transpose of
+// their own tile, through LDS; then each updates its row with MFMA.  Wavefront k + 1 updates its diagonal tile alone and
+// goes on to invert it: the rest of its row follows after that, when the next wavefront is the one that all wait for.
+// (Its row's tiles are needed by nobody else.)  late() runs in wavefront 0 after its first inverse.
+// Returns 1 + the first non-positive pivot (0 if none) in the wavefront that met it.
+constexpr int INV64_LDS = 4 * 5 * TILE;  // doubles: five tiles a stage, so one barrier a stage suffices
+template <class Late>
+__device__ __forceinline__ int inverse64(tg_tile (&a)[4], double *lds, const tg_tile &unit, Late late) {
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const tg_tile zero = {0.0, 0.0, 0.0, 0.0};
     int bad = 0;
-    for (int k4 = 0; k4 < CB / 4; ++k4) {
+    tg_tile u = zero, sk = zero;
+    // S_wj -= S_wk D S_kj and S_wk <- S_wk D, from u = -D S_kw; skip: a tile that was done before
+    auto update = [&](int k, int skip) {
+        const double *buf = lds + k * (5 * TILE);
+        const tg_tile Dk = get_tile(buf + 4 * TILE);
+        tg_tile s[4];
 #pragma unroll
-        for (int kk = 0; kk < 4; ++kk) {
-            const int k = 4 * k4 + kk, b = kk & 1;
-            if (ti == k4) {
+        for (int j = 0; j < 4; ++j)
+            if (j != k && j != skip) s[j] = get_tile(buf + j * TILE);
+        a[k] = zero;
 #pragma unroll
-                for (int jj = 0; jj < 4; ++jj) rowb[b][bj + jj] = r[kk][jj];
-            }
-            if (tj == k4) {
+        for (int r = 0; r < 4; ++r)
 #pragma unroll
-                for (int ii = 0; ii < 4; ++ii) colb[b][bi + ii] = r[ii][kk];
-            }
+            for (int j = 0; j < 4; ++j)
+                if (j != skip)
+                    a[j] = __builtin_amdgcn_mfma_f64_16x16x4f64(j == k ? sk[r] : u[r], j == k ? Dk[r] : s[j][r], a[j], 0, 0, 0);
+    };
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        double *buf = lds + k * (5 * TILE);
+        if (w == k) {
+            tg_tile d = a[k];
+            const int b = inverse16(d);
+            if (b) bad = 16 * k + b;
+            put_tile(buf + 4 * TILE, d);
             __syncthreads();
-            double piv = colb[b][k];
-            if (!(piv > 0.0)) {
-                if (!bad) bad = k + 1;
-                piv = 1.0;
+            if (k == 0) late();
+            else update(k - 1, k);  // the rest of the previous stage
+            tg_tile s[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                s[j] = a[j];
+                a[j] = zero;
             }
-            const double p = recip_nr(piv);
-            double ap[4], kb[4];
 #pragma unroll
-            for (int ii = 0; ii < 4; ++ii) ap[ii] = colb[b][bi + ii] * p;
+            for (int r = 0; r < 4; ++r)
 #pragma unroll
-            for (int jj = 0; jj < 4; ++jj) kb[jj] = rowb[b][bj + jj];
-#pragma unroll
-            for (int ii = 0; ii < 4; ++ii)
-#pragma unroll
-                for (int jj = 0; jj < 4; ++jj) r[ii][jj] = fma(-ap[ii], kb[jj], r[ii][jj]);
-            if (tj == k4) {
-#pragma unroll
-                for (int ii = 0; ii < 4; ++ii) r[ii][kk] = ap[ii];
-            }
-            if (ti == k4) {
-#pragma unroll
-                for (int jj = 0; jj < 4; ++jj) r[kk][jj] = -p * kb[jj];
-                if (tj == k4) r[kk][kk] = p;
+                for (int j = 0; j < 4; ++j)
+                    if (j != k) a[j] = __builtin_amdgcn_mfma_f64_16x16x4f64(d[r], s[j][r], a[j], 0, 0, 0);
+            a[k] = -d;
+        } else {
+            sk = transposed(a[k], unit);
+            put_tile(buf + w * TILE, sk);
+            __syncthreads();
+            u = -tile_fma(get_tile(buf + 4 * TILE), sk, zero);  // -D S_kw
+            if (w == k + 1) {
+                if (k < 3) a[k < 3 ? k + 1 : 3] = tile_fma(u, sk, a[k < 3 ? k + 1 : 3]);
+            } else {
+                update(k, -1);
             }
         }
     }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) a[j] = -a[j];
     return bad;
 }
 
-__global__ __launch_bounds__(256) void k_sweep_panel(const SweepProb A, const SweepProb B, int K) {
-    __shared__ double dl[CB][CB + 1];   // D
-    __shared__ double sl[CB][CB + 1];   // S_IK
-    __shared__ double rowb[2][CB], colb[2][CB];
-    const SweepProb &q = blockIdx.y ? B : A;
-    const int I = blockIdx.x;
-    if (K >= q.nb || I >= q.nb) return;
-    const int t = threadIdx.x, bi = 4 * (t / 16), bj = 4 * (t % 16);
-    const int64_t np = q.np, k0 = (int64_t)K * CB, i0 = (int64_t)I * CB;
-    double r[4][4];
+// A workgroup's 64 x 64 block (wavefront w: rows 16 w .., tiles a[0..3]) at p, row-major with stride ld.
+__device__ __forceinline__ void store64(double *p, int64_t ld, const tg_tile (&a)[4]) {
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, q = lane >> 4, c = lane & 15;
 #pragma unroll
-    for (int ii = 0; ii < 4; ++ii)
+    for (int j = 0; j < 4; ++j)
 #pragma unroll
-        for (int jj = 0; jj < 4; ++jj) r[ii][jj] = q.S[(k0 + bi + ii) * np + k0 + bj + jj];
-    const int bad = gj_inverse64(r, rowb, colb);
-    if (I == K) {
-#pragma unroll
-        for (int ii = 0; ii < 4; ++ii)
-#pragma unroll
-            for (int jj = 0; jj < 4; ++jj) q.D[(bi + ii) * CB + bj + jj] = r[ii][jj];
-        if (t == 0 && bad && *q.info == 0) *q.info = (int)k0 + bad;
-        return;
-    }
-#pragma unroll
-    for (int ii = 0; ii < 4; ++ii)
-#pragma unroll
-        for (int jj = 0; jj < 4; ++jj) {
-            dl[bi + ii][bj + jj] = r[ii][jj];
-            sl[bi + ii][bj + jj] = q.S[(i0 + bi + ii) * np + k0 + bj + jj];
-            q.Rw[(int64_t)(bi + ii) * np + i0 + bj + jj] = q.S[(k0 + bi + ii) * np + i0 + bj + jj];
-        }
-    __syncthreads();
-    double acc[4][4] = {};
-    for (int k = 0; k < CB; ++k) {
-        double a[4], b[4];
-#pragma unroll
-        for (int ii = 0; ii < 4; ++ii) a[ii] = sl[bi + ii][k];
-#pragma unroll
-        for (int jj = 0; jj < 4; ++jj) b[jj] = dl[k][bj + jj];
-#pragma unroll
-        for (int ii = 0; ii < 4; ++ii)
-#pragma unroll
-            for (int jj = 0; jj < 4; ++jj) acc[ii][jj] += a[ii] * b[jj];
-    }
-#pragma unroll
-    for (int ii = 0; ii < 4; ++ii)
-#pragma unroll
-        for (int jj = 0; jj < 4; ++jj) q.T[(i0 + bi + ii) * CB + bj + jj] = acc[ii][jj];
+        for (int r = 0; r < 4; ++r) p[(16 * w + 4 * r + q) * ld + 16 * j + c] = a[j][r];
 }
 
-// Every 64 x 64 block (I, J) of the plane block from T, Rw and D.  The products run on the matrix cores
-// (MFMA f64 16x16x4: lane l holds A(l % 16, l / 16), B(l / 16, l % 16), result register r at
-// (4 r + l / 16, l % 16)); wave w computes the 32 x 32 quadrant (w / 2, w % 2) of the block.
-typedef double tg_cdbl4 __attribute__((ext_vector_type(4)));
-__global__ __launch_bounds__(256) void k_sweep_update(const SweepProb A, const SweepProb B, int K) {
-    __shared__ double al[CB][CB + 1];
-    __shared__ double bl[CB][CB + 1];
+// The block (I, J) of the lower triangle that workgroup b of a plane has.
+__device__ __forceinline__ void tri_block(int b, int &I, int &J) {
+    I = (int)((sqrtf(8.0f * (float)b + 1.0f) - 1.0f) * 0.5f);
+    while (I * (I + 1) / 2 > b) --I;
+    while ((I + 1) * (I + 2) / 2 <= b) ++I;
+    J = b - I * (I + 1) / 2;
+}
+__device__ __forceinline__ double *tri_tiles(double *W, int I, int J) {
+    return W + ((int64_t)I * (I + 1) / 2 + J) * (CB * CB);
+}
+
+__device__ __forceinline__ tg_tile unit_tile() {
+    const int lane = threadIdx.x & 63, q = lane >> 4, c = lane & 15;
+    tg_tile u;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) u[r] = 4 * r + q == c ? 1.0 : 0.0;
+    return u;
+}
+// A workgroup's block into the step buffers: as it is, or (tr) transposed, as the blocks below the next
+// pivot block are, so that step's S_KX has the same tiles on either side of the diagonal.
+__device__ __forceinline__ void put_block(double *p, const tg_tile (&a)[4], bool tr, const tg_tile &unit) {
+    const int w = threadIdx.x >> 6;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        if (tr) put_tile(p + (4 * j + w) * TILE, transposed(a[j], unit));
+        else put_tile(p + (4 * w + j) * TILE, a[j]);
+    }
+}
+
+// D of the first pivot block (a plane of one block is then done), and the other blocks in tiles, meanwhile.
+__global__ __launch_bounds__(256, 2) void k_sweep_first(const SweepProb A, const SweepProb B) {
+    __shared__ double lds[INV64_LDS];
     const SweepProb &q = blockIdx.y ? B : A;
-    if (K >= q.nb) return;
-    const int I = blockIdx.x / q.nb, J = blockIdx.x % q.nb;
-    if (I >= q.nb) return;
-    const int t = threadIdx.x;
-    const int64_t np = q.np, i0 = (int64_t)I * CB, j0 = (int64_t)J * CB;
-    if (J == K) {  // S_IK <- T_I, S_KK <- D
-        for (int idx = t; idx < CB * CB; idx += 256) {
-            const int ii = idx / CB, jj = idx % CB;
-            q.S[(i0 + ii) * np + j0 + jj] = I == K ? q.D[ii * CB + jj] : q.T[(i0 + ii) * CB + jj];
-        }
+    if ((int)blockIdx.x >= q.nb * (q.nb + 1) / 2) return;
+    int I, J;
+    tri_block(blockIdx.x, I, J);
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, qq = lane >> 4, c = lane & 15;
+    const double *p = q.S + (int64_t)I * CB * q.np + J * CB;
+    const tg_tile unit = unit_tile();
+    tg_tile a[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) a[j][r] = p[(16 * w + 4 * r + qq) * q.np + 16 * j + c];
+    if (I > 0) {
+        put_block(tri_tiles(q.W1, I, J), a, J == 0, unit);
         return;
     }
-    // S_IJ -= T_I Rw_J  (I != K),  S_KJ = -D Rw_J
-    for (int idx = t; idx < CB * CB; idx += 256) {
-        const int ii = idx / CB, jj = idx % CB;
-        al[ii][jj] = I == K ? q.D[ii * CB + jj] : q.T[(i0 + ii) * CB + jj];
-        bl[ii][jj] = q.Rw[(int64_t)ii * np + j0 + jj];
-    }
-    __syncthreads();
-    const int w = t >> 6, lane = t & 63, li = lane & 15, lk = lane >> 4;
-    const int R0 = 32 * (w >> 1), C0 = 32 * (w & 1);
-    tg_cdbl4 acc[2][2];
+    const int bad = inverse64(a, lds, unit, [] {});
+    if (q.nb == 1) store64(q.S, q.np, a);
+    else put_block(q.D, a, false, unit);
+    if (bad && lane == 0) atomicMax(q.info, INT_MAX - bad);
+}
+
+__global__ __launch_bounds__(256, 2) void k_sweep_step(const SweepProb A, const SweepProb B, int K) {
+    __shared__ double lD[INV64_LDS], lQ[CB * CB];  // D, then the inverse's LDS
+    const SweepProb &q = blockIdx.y ? B : A;
+    const int nb = q.nb;
+    if (K >= nb || nb == 1) return;  // a single block was done by k_sweep_first
+    int b = blockIdx.x;
+    if (b >= nb * (nb + 1) / 2) return;
+    const bool last = K == nb - 1;
+    // the next pivot block's workgroup has the longest way to go: it comes first in the launch
+    const int nxt = (K + 1) * (K + 2) / 2 + K + 1;
+    if (!last) b = b == 0 ? nxt : (b == nxt ? 0 : b);
+    int I, J;
+    tri_block(b, I, J);
+    double *src = (K & 1) ? q.W0 : q.W1, *dst = (K & 1) ? q.W1 : q.W0;
+    const double *Dk = q.D + (K & 1) * (CB * CB);
+    const int t = threadIdx.x, lane = t & 63, w = __builtin_amdgcn_readfirstlane(t >> 6);
+    const tg_tile zero = {0.0, 0.0, 0.0, 0.0}, unit = unit_tile();
+    const bool next = I == K + 1 && J == K + 1;
+    tg_tile a[4], u[4] = {zero, zero, zero, zero};
+    auto updated = [&](int j0, int j1) {  // a[j] -= S_IK D S_KJ, from u = -D S_KI of this wavefront's columns
 #pragma unroll
-    for (int a = 0; a < 2; ++a)
+        for (int k = 0; k < 4; ++k) {
+            tg_tile qk[4];
 #pragma unroll
-        for (int b = 0; b < 2; ++b) acc[a][b] = tg_cdbl4{0.0, 0.0, 0.0, 0.0};
-#pragma unroll 4
-    for (int kk = 0; kk < CB / 4; ++kk) {
-        const double x0 = al[R0 + li][4 * kk + lk], x1 = al[R0 + 16 + li][4 * kk + lk];
-        const double y0 = bl[4 * kk + lk][C0 + li], y1 = bl[4 * kk + lk][C0 + 16 + li];
-        acc[0][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(x0, y0, acc[0][0], 0, 0, 0);
-        acc[0][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(x0, y1, acc[0][1], 0, 0, 0);
-        acc[1][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(x1, y0, acc[1][0], 0, 0, 0);
-        acc[1][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(x1, y1, acc[1][1], 0, 0, 0);
-    }
+            for (int j = 0; j < 4; ++j)
+                if (j >= j0 && j < j1) qk[j] = get_tile(lQ + (4 * k + j) * TILE);
 #pragma unroll
-    for (int a = 0; a < 2; ++a)
+            for (int r = 0; r < 4; ++r)
 #pragma unroll
-        for (int b = 0; b < 2; ++b)
+                for (int j = 0; j < 4; ++j)
+                    if (j >= j0 && j < j1) a[j] = __builtin_amdgcn_mfma_f64_16x16x4f64(u[k][r], qk[j][r], a[j], 0, 0, 0);
+        }
+    };
+    if (I == K && J == K) {
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                double *dst = q.S + (i0 + R0 + 16 * a + 4 * r + lk) * np + j0 + C0 + 16 * b + li;
-                *dst = I == K ? -acc[a][b][r] : *dst - acc[a][b][r];
+        for (int j = 0; j < 4; ++j) a[j] = -get_tile(Dk + (4 * w + j) * TILE);
+    } else {
+        // D in LDS; P = S_KI, this wavefront's columns, in registers; Q = S_KJ in LDS (P where I = J).
+        // S_KX is the block (K, X), or (X, K) in transposed tiles.
+        double2 dv[8];
+        tg_tile p[4], qv[4];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) dv[i] = reinterpret_cast<const double2 *>(Dk)[256 * i + t];
+        if (I != K) {
+            const double *s = I > K ? tri_tiles(src, I, K) : tri_tiles(src, K, I);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) p[k] = get_tile(s + (4 * k + w) * TILE);
+        }
+        if (J != K && I != J) {
+            const double *s = J > K ? tri_tiles(src, J, K) : tri_tiles(src, K, J);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) qv[k] = get_tile(s + (4 * k + w) * TILE);
+        }
+        if (I != K && J != K) {
+            const double *s = tri_tiles(src, I, J);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) a[j] = get_tile(s + (4 * w + j) * TILE);
+        } else {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) a[j] = zero;
+        }
+#pragma unroll
+        for (int i = 0; i < 8; ++i) reinterpret_cast<double2 *>(lD)[256 * i + t] = dv[i];
+        if (J != K) {
+#pragma unroll
+            for (int k = 0; k < 4; ++k) put_tile(lQ + (4 * k + w) * TILE, I == J ? p[k] : qv[k]);
+        }
+        __syncthreads();
+        if (I == K || J == K) {  // D S_KJ, or S_IK D
+            const double *y = I == K ? lQ : lD;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                tg_tile yk[4];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) yk[j] = get_tile(y + (4 * k + j) * TILE);
+                tile_fma4(I == K ? get_tile(lD + (4 * k + w) * TILE) : p[k], yk, a);
             }
+        } else {
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                tg_tile dk[4];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) dk[j] = get_tile(lD + (4 * k + j) * TILE);
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+#pragma unroll
+                    for (int j = 0; j < 4; ++j)
+                        u[j] = __builtin_amdgcn_mfma_f64_16x16x4f64(dk[j][r], -p[k][r], u[j], 0, 0, 0);
+            }
+            // wavefront 0 of the next pivot block: its diagonal tile first, the others once that is inverted
+            if (next && w == 0) updated(0, 1);
+            else updated(0, 4);
+        }
+    }
+    if (last) {  // S^-1, row-major, the upper triangle from the lower one
+#pragma unroll
+        for (int j = 0; j < 4; ++j) a[j] = -a[j];
+        store64(q.S + (int64_t)I * CB * q.np + J * CB, q.np, a);
+        if (I != J) {
+            const int qq = lane >> 4, c = lane & 15;
+            double *m = q.S + (int64_t)J * CB * q.np + I * CB;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const tg_tile v = transposed(a[j], unit);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) m[(16 * j + 4 * r + qq) * q.np + 16 * w + c] = v[r];
+            }
+        }
+    } else if (next) {  // (the block itself is D's from here on)
+        __syncthreads();  // every wavefront has read lD
+        const int bad = inverse64(a, lD, unit, [&] { updated(1, 4); });
+        put_block(q.D + ((K + 1) & 1) * (CB * CB), a, false, unit);
+        if (bad && lane == 0) atomicMax(q.info, INT_MAX - ((K + 1) * CB + bad));
+    } else {
+        put_block(tri_tiles(dst, I, J), a, J == K + 1, unit);
+    }
 }
 
 // ---- solve operators:  Out(i, col0 + 3 jn + c) = sum_k S(i, C(3 jn, k)) V(3 jn + c, k) ----------------
@@ -804,9 +1027,8 @@ void CoarseSolver::setup(const HostLevel &L, const Grid &grid, hipStream_t st) {
     Bop.alloc(std::max<int64_t>(bOff[P], 1));
     Fop.zero(st);  // row padding stays zero
     Bop.zero(st);
-    T.alloc(2 * maxpad * CB);
-    Rw.alloc(2 * maxpad * CB);
-    Dk.alloc(2 * CB * CB);
+    W.alloc(maxpad > CB ? 4 * maxpad * maxpad : 1);
+    Dk.alloc(4 * CB * CB);
     bb.alloc(std::max<int64_t>(ntot, 1));
     yy.alloc(std::max<int64_t>(ntot, 1));
     xx.alloc(std::max<int64_t>(ntot, 1));
@@ -857,14 +1079,14 @@ void CoarseSolver::factor(const double *Ks, int64_t ldk, const uint8_t *eleMask,
         const int pl[2] = {p, q};
         for (int y = 0; y < 2; ++y) {
             if (!has(pl[y])) continue;
-            pr[y] = SweepProb{S_of(pl[y]), npad[pl[y]], (int)(npad[pl[y]] / CB), T.p + y * maxpad * CB,
-                              Rw.p + y * maxpad * CB, Dk.p + y * CB * CB, info.p + pl[y]};
+            pr[y] = SweepProb{S_of(pl[y]), W.p + 2 * y * maxpad * maxpad, W.p + (2 * y + 1) * maxpad * maxpad,
+                              npad[pl[y]], (int)(npad[pl[y]] / CB), Dk.p + 2 * y * CB * CB, info.p + pl[y]};
             nbmax = std::max(nbmax, pr[y].nb);
         }
-        for (int K = 0; K < nbmax; ++K) {
-            k_sweep_panel<<<dim3(nbmax, 2), 256, 0, st>>>(pr[0], pr[1], K);
-            k_sweep_update<<<dim3(nbmax * nbmax, 2), 256, 0, st>>>(pr[0], pr[1], K);
-        }
+        if (nbmax) k_sweep_first<<<dim3(nbmax * (nbmax + 1) / 2, 2), 256, 0, st>>>(pr[0], pr[1]);
+        if (nbmax > 1)
+            for (int K = 0; K < nbmax; ++K)
+                k_sweep_step<<<dim3(nbmax * (nbmax + 1) / 2, 2), 256, 0, st>>>(pr[0], pr[1], K);
         TG_LAUNCH_CHECK(id);
     };
     // solve operators: Out = S_p^-1 A_{p,r} for neighbour plane r, from r's coupling rows towards p
@@ -930,7 +1152,7 @@ void CoarseSolver::factor(const double *Ks, int64_t ldk, const uint8_t *eleMask,
         if (hinfo[p] != 0)
             fail(TG_ERR_NUMERIC, "tg_solver:coarse",
                  "coarsest-level factorisation failed on plane block %d (pivot %d): matrix not positive definite",
-                 p, hinfo[p]);
+                 p, INT_MAX - hinfo[p]);
     factored = true;
 }
 
