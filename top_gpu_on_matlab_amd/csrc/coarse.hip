@@ -209,8 +209,7 @@ __device__ __forceinline__ void row_copies(double x, double (&y)[4]) {
 
 // Pivot row I of the four rows y (rows 4 B .. 4 B + 3 of the tile, each lane's column), pivot 4 B + I.  In the
 // pivot's column, -1 in place of the pivot row's entry and 0 in place of the others' make the one update
-// right there too.  The products with the pivot row come before its scaling, so they do not wait for the
-// reciprocal.  bad: lanes that saw a pivot that is not positive.
+// right there too.  bad: lanes that saw a pivot that is not positive.
 template <int B, int I>
 __device__ __forceinline__ void sweep_row4(double (&y)[4], int c, unsigned long long (&bad)[16]) {
     constexpr int P = 4 * B + I;
@@ -219,7 +218,7 @@ __device__ __forceinline__ void sweep_row4(double (&y)[4], int c, unsigned long 
     const double d = recip_refined(piv), yi = c == P ? -1.0 : y[I];
 #pragma unroll
     for (int j = 0; j < 4; ++j)
-        if (j != I) y[j] = fma(-(row_lane<P>(y[j]) * yi), d, c == P ? 0.0 : y[j]);
+        if (j != I) y[j] = fma(-(row_lane<P>(y[j]) * d), yi, c == P ? 0.0 : y[j]);
     y[I] = yi * d;
 }
 

@@ -59,7 +59,9 @@ struct Solver {
     DevBuf<float> K0_32, E32;
     DevBuf<int32_t> fullUid;
     DevBuf<double> Gl2, Ech;               // level-2 Galerkin GEMM: G_s (nCh x 576, entry fastest), children moduli
-    DevBuf<int64_t> bndList;               // coarse elements with a boundary (fixed-DOF) child
+    DevBuf<int64_t> bndList;               // coarse elements with boundary (fixed-DOF) children, ...
+    DevBuf<int32_t> bndPtr;                // ... where each one's children start in bndChild (BndChild records)
+    DevBuf<unsigned char> bndChild;
     int64_t nBnd = 0;
     DevBuf<double> b, y;        // PCG right-hand side and iterate (full fine grid)
     PcgWork pw;                 // PCG work vectors

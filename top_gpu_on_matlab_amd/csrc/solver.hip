@@ -30,16 +30,6 @@ struct ChildGrid {
     }
 };
 
-struct SrcDevL2 : ChildGrid {
-    const double *E, *K0, *uf, *ux;
-    const int32_t *uid;
-    __device__ double kch(int f, int i) const {
-        const int32_t u = uid[f];
-        if (u > 0) return uf[(size_t)(u - 1) * 576 + i] * E[f] + ux[(size_t)(u - 1) * 576 + i];
-        return K0[i] * E[f];
-    }
-};
-
 struct SrcDevHigher : ChildGrid {
     const double *prev;
     int64_t ldp;
@@ -76,22 +66,80 @@ __global__ __launch_bounds__(GK_THREADS) void k_galerkin_dev(Src src, const uint
     for (int i = 0; i < 9; ++i) Ks[(int64_t)galerkin_entry(i) * ldk + ce] = acc[i];
 }
 
-// The same product restricted to a list of coarse elements (those with boundary children).
-template <class Src>
-__global__ __launch_bounds__(GK_THREADS) void k_galerkin_list(Src src, const int64_t *__restrict__ list, int nCh,
-                                                              const double *__restrict__ P, double *__restrict__ Ks,
-                                                              int64_t ldk) {
-    __shared__ double sB[576], sK[576], sT[576];
-    const int64_t ce = list[blockIdx.x];
-    src.ce = ce;
-    double acc[9];
-    galerkin_block(acc, src, nCh, P, sB, sK, sT);
+// Level 2, standard voxels: the children with fixed DOFs, which the moduli product (k_galerkin_l2_mfma) leaves
+// out, added to their coarse elements: Ks_e += sum P_s' (E_f Ufree_u + Ufixed_u) P_s over the listed children of
+// the element (slot s, fine element f, boundary matrices u).  P_s = W_s (x) I_3 with the 8 x 8 trilinear
+// weights W_s, so both products run over vertices only, a third of the dense operations.  One workgroup
+// per coarse element, its four wavefronts taking the children in turn (an element on a clamped face
+// has 16), and their sums added in wavefront order.  Bound by the chain of a child's loads and its two
+// products; recomputing all 64 children of such an element in one wavefront took 460 us at 96 x 192 x 96 and 510
+// at 128 x 256 x 128, this 45 and 86.
+struct BndChild {
+    int32_t slot, fine, uid;
+};
+constexpr int GB_WAVES = 4;
+__global__ __launch_bounds__(64 * GB_WAVES) void k_galerkin_bnd(const int64_t *__restrict__ list,
+                                                                const int32_t *__restrict__ ptr,
+                                                                const BndChild *__restrict__ child,
+                                                                const double *__restrict__ E,
+                                                                const double *__restrict__ uf,
+                                                                const double *__restrict__ ux,
+                                                                const double *__restrict__ P, double *__restrict__ Ks,
+                                                                int64_t ldk) {
+    __shared__ double sK[GB_WAVES][576], sT[GB_WAVES][576];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int a = lane & 7, j = lane >> 3;  // this lane's row and column vertex
+    const int c0 = ptr[blockIdx.x], c1 = ptr[blockIdx.x + 1];
+    double acc[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
+    for (int cb = c0; cb < c1; cb += GB_WAVES) {  // uniform over the workgroup
+        const bool on = cb + w < c1;
+        const BndChild ch = child[on ? cb + w : c0];
+        const double e = on ? E[ch.fine] : 0.0;
+        double wj[8], wi[8];  // W_s(b, j), W_s(b, a)
 #pragma unroll
-    for (int i = 0; i < 9; ++i) Ks[(int64_t)galerkin_entry(i) * ldk + ce] = acc[i];
+        for (int b = 0; b < 8; ++b) {
+            wj[b] = P[(size_t)576 * ch.slot + 3 * b + 72 * j];
+            wi[b] = P[(size_t)576 * ch.slot + 3 * b + 72 * a];
+        }
+        __syncthreads();  // the previous child's sT has been read
+#pragma unroll
+        for (int k = 0; k < 9; ++k) {
+            const size_t i = (size_t)ch.uid * 576 + 64 * k + lane;
+            sK[w][64 * k + lane] = on ? uf[i] * e + ux[i] : 0.0;
+        }
+        __syncthreads();
+        double t[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};  // t(d, f) = sum_b K(3 a + d, 3 b + f) W(b, j)
+#pragma unroll
+        for (int b = 0; b < 8; ++b)
+#pragma unroll
+            for (int f = 0; f < 3; ++f)
+#pragma unroll
+                for (int d = 0; d < 3; ++d) t[d + 3 * f] += sK[w][3 * a + d + 24 * (3 * b + f)] * wj[b];
+#pragma unroll
+        for (int k = 0; k < 9; ++k) sT[w][64 * k + lane] = t[k];
+        __syncthreads();
+#pragma unroll
+        for (int b = 0; b < 8; ++b)
+#pragma unroll
+            for (int k = 0; k < 9; ++k) acc[k] += wi[b] * sT[w][64 * k + b + 8 * j];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < 9; ++k) sK[w][64 * k + lane] = acc[k];
+    __syncthreads();
+    const int64_t ce = list[blockIdx.x];
+    for (int i = threadIdx.x; i < 576; i += 64 * GB_WAVES) {
+        double v = sK[0][i];
+        for (int k = 1; k < GB_WAVES; ++k) v += sK[k][i];
+        const int l = i & 63, k = i >> 6, row = 3 * (l & 7) + k % 3, col = 3 * (l >> 3) + k / 3;
+        Ks[(int64_t)(row + 24 * col) * ldk + ce] += v;
+    }
 }
 
-// Children moduli of every coarse element, child-major: Ech[ce + ldk * s] = E(child s) (0 when void).
-__global__ void k_gather_children(const double *__restrict__ E, const uint8_t *__restrict__ fineSolid, int span,
+// Children moduli of every coarse element, child-major: Ech[ce + ldk * s] = E(child s), 0 when void and for a
+// child with boundary matrices (uid > 0; k_galerkin_bnd adds those).
+__global__ void k_gather_children(const double *__restrict__ E, const uint8_t *__restrict__ fineSolid,
+                                  const int32_t *__restrict__ uid, int span,
                                   int cEY, int cEX, int64_t nC, int fEY, int fEX, int nCh, double *__restrict__ Ech,
                                   int64_t ldk) {
     const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -101,7 +149,7 @@ __global__ void k_gather_children(const double *__restrict__ E, const uint8_t *_
     const int a = s % span, b = (s / span) % span, c = s / (span * span);
     const int cy = (int)(ce % cEY), cx = (int)((ce / cEY) % cEX), cz = (int)(ce / ((int64_t)cEY * cEX));
     const int64_t f = (int64_t)(span * cy + a) + (int64_t)fEY * ((span * cx + b) + (int64_t)fEX * (span * cz + c));
-    Ech[ce + ldk * s] = fineSolid[f] ? E[f] : 0.0;
+    Ech[ce + ldk * s] = fineSolid[f] && uid[f] <= 0 ? E[f] : 0.0;
 }
 
 // Level-2 Galerkin product on the matrix cores: Ks[j * ldk + e] = sum_k Ech[e + ldk * k] G[k * 576 + j]
@@ -110,14 +158,18 @@ __global__ void k_gather_children(const double *__restrict__ E, const uint8_t *_
 // Ech', so its 16 x 16 result is entries x elements and every store row is 16 consecutive elements.
 // Lane layouts of that instruction: lane l holds A(l % 16, l / 16), B(l / 16, l % 16) and result registers
 // r = 0..3 at D(4 r + l / 16, l % 16).  A
-// wavefront owns 16 NG consecutive elements, keeps their children moduli in registers and walks the 36
-// entry tiles; each G value loaded feeds NG MFMAs.  e ranges over the padded count ldk (a multiple of
-// 64; padded elements have zero moduli).
+// wavefront owns 16 NG consecutive elements, keeps their children moduli in registers and walks `tiles` of the 36
+// entry tiles (blockIdx.y says which); each G value loaded feeds NG MFMAs.  e ranges over the padded
+// count ldk (a multiple of 64; padded elements have zero moduli).  A wavefront's walk is a serial chain of
+// 2.5 us per tile (FP64 MFMA), so where the elements alone do not fill the chip the tiles are shared
+// out: all 36 in one wavefront took 88 us at any size below 65,536 elements; shared out 7 us at 432 elements
+// and 60 at 27,648 (from 93); at 65,536 it stays at 100, the result's 302 MB and 4.8 GFLOP.
 typedef double tg_dbl4 __attribute__((ext_vector_type(4)));
 template <int KS, int NG>
 __global__ __launch_bounds__(256) void k_galerkin_l2_mfma(const double *__restrict__ Ech, const double *__restrict__ G,
-                                                          double *__restrict__ Ks, int64_t ldk) {
+                                                          double *__restrict__ Ks, int64_t ldk, int tiles) {
     const int lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4;
+    const int t0 = blockIdx.y * tiles, t1 = min(t0 + tiles, 36);
     const int64_t e0 = ((int64_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * (16 * NG);
     if (e0 >= ldk) return;
     double b[NG][KS];
@@ -128,13 +180,13 @@ __global__ __launch_bounds__(256) void k_galerkin_l2_mfma(const double *__restri
     const double *gp = G + (int64_t)lk * 576 + li;
     double a[KS];
 #pragma unroll
-    for (int kk = 0; kk < KS; ++kk) a[kk] = gp[(int64_t)4 * kk * 576];
-    for (int t = 0; t < 36; ++t) {
+    for (int kk = 0; kk < KS; ++kk) a[kk] = gp[(int64_t)4 * kk * 576 + 16 * t0];
+    for (int t = t0; t < t1; ++t) {
         tg_dbl4 acc[NG];
 #pragma unroll
         for (int g = 0; g < NG; ++g) acc[g] = tg_dbl4{0.0, 0.0, 0.0, 0.0};
         double an[KS];  // next tile's G values, loaded while this tile's MFMAs run
-        const int tn = t + 1 < 36 ? t + 1 : t;
+        const int tn = t + 1 < t1 ? t + 1 : t;
 #pragma unroll
         for (int kk = 0; kk < KS; ++kk) an[kk] = gp[(int64_t)4 * kk * 576 + 16 * tn];
 #pragma unroll
@@ -371,20 +423,28 @@ Solver::Solver(const tg_model &m, hipStream_t s) : model(m), st(s) {
                 }
         }
         Gl2.upload(gt, st);
-        std::vector<int64_t> bnd;
+        std::vector<int64_t> bnd;  // coarse elements with children that have fixed DOFs, and those children
+        std::vector<int32_t> ptr(1, 0);
+        std::vector<BndChild> kids;
         const Grid &cgd = C.g, &fgd = F.g;
         for (int64_t ce = 0; ce < cgd.elems(); ++ce) {
             const int cy = (int)(ce % cgd.EY), cx = (int)((ce / cgd.EY) % cgd.EX), cz = (int)(ce / ((int64_t)cgd.EY * cgd.EX));
-            bool b = false;
-            for (int sc = 0; sc < nCh && !b; ++sc) {
+            for (int sc = 0; sc < nCh; ++sc) {
                 const int a = sc % span, bb2 = (sc / span) % span, c = sc / (span * span);
                 const int64_t f = (int64_t)(span * cy + a) + (int64_t)fgd.EY * ((span * cx + bb2) + (int64_t)fgd.EX * (span * cz + c));
-                b = uid[f] > 0;
+                if (uid[f] > 0 && m.lv[0].solid[f]) kids.push_back(BndChild{sc, (int32_t)f, uid[f] - 1});
             }
-            if (b) bnd.push_back(ce);
+            if ((int32_t)kids.size() > ptr.back()) {
+                bnd.push_back(ce);
+                ptr.push_back((int32_t)kids.size());
+            }
         }
         nBnd = (int64_t)bnd.size();
-        if (nBnd) bndList.upload(bnd, st);
+        if (nBnd) {
+            bndList.upload(bnd, st);
+            bndPtr.upload(ptr, st);
+            bndChild.upload((const unsigned char *)kids.data(), kids.size() * sizeof(BndChild), st);
+        }
         Ech.alloc((size_t)nCh * C.ldk);
         Ech.zero(st);
     }
@@ -474,22 +534,21 @@ void Solver::assemble() {
         ChildGrid cg{C.span, C.g.EY, C.g.EX, Fi.g.EY, Fi.g.EX, Fi.eleMask.p, 0};
         const unsigned grid = (unsigned)C.g.elems();
         if (i == 1 && !super) {
-            SrcDevL2 src;
-            static_cast<ChildGrid &>(src) = cg;
-            src.E = E64; src.K0 = K0_64; src.uf = uFree; src.ux = uFixed; src.uid = fullUid;
             const int64_t nC = C.g.elems();
-            k_gather_children<<<grid_for(nC * nCh, 256), 256, 0, st>>>(E64, Fi.eleMask, C.span, C.g.EY, C.g.EX, nC,
-                                                                      Fi.g.EY, Fi.g.EX, nCh, Ech, C.ldk);
+            k_gather_children<<<grid_for(nC * nCh, 256), 256, 0, st>>>(E64, Fi.eleMask, fullUid, C.span, C.g.EY, C.g.EX,
+                                                                      nC, Fi.g.EY, Fi.g.EX, nCh, Ech, C.ldk);
             TG_LAUNCH_CHECK(id);
-            // ldk is a multiple of 64: 64 elements per wavefront, 256 per workgroup
-            if (nCh == 64)
-                k_galerkin_l2_mfma<16, 4><<<grid_for(C.ldk, 256), 256, 0, st>>>(Ech, Gl2, C.Ks64, C.ldk);
-            else if (nCh == 8)
-                k_galerkin_l2_mfma<2, 4><<<grid_for(C.ldk, 256), 256, 0, st>>>(Ech, Gl2, C.Ks64, C.ldk);
-            else
-                fail(TG_ERR_ARGS, id, "level-2 Galerkin: %d children per coarse element", nCh);
+            // ldk is a multiple of 64: 64 elements per wavefront, 256 per workgroup; entry tiles shared out until
+            // there are four wavefronts for each of the 1024 SIMDs
+            const int tiles = (int)std::max<int64_t>(1, std::min<int64_t>(36, 36 * (C.ldk / 64) / 4096));
+            const dim3 gg(grid_for(C.ldk, 256), grid_for(36, tiles));
+            if (nCh == 64) k_galerkin_l2_mfma<16, 4><<<gg, 256, 0, st>>>(Ech, Gl2, C.Ks64, C.ldk, tiles);
+            else if (nCh == 8) k_galerkin_l2_mfma<2, 4><<<gg, 256, 0, st>>>(Ech, Gl2, C.Ks64, C.ldk, tiles);
+            else fail(TG_ERR_ARGS, id, "level-2 Galerkin: %d children per coarse element", nCh);
             TG_LAUNCH_CHECK(id);
-            if (nBnd) k_galerkin_list<<<(unsigned)nBnd, GK_THREADS, 0, st>>>(src, bndList, nCh, C.P, C.Ks64, C.ldk);
+            if (nBnd)
+                k_galerkin_bnd<<<(unsigned)nBnd, 64 * GB_WAVES, 0, st>>>(bndList, bndPtr, (const BndChild *)bndChild.p, E64,
+                                                                        uFree, uFixed, C.P, C.Ks64, C.ldk);
         } else if (i == 1) {
             SrcDevSuper src;
             static_cast<ChildGrid &>(src) = cg;
