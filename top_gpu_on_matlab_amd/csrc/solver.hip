@@ -30,12 +30,6 @@ struct ChildGrid {
     }
 };
 
-struct SrcDevHigher : ChildGrid {
-    const double *prev;
-    int64_t ldp;
-    __device__ double kch(int f, int i) const { return prev[(int64_t)i * ldp + f]; }
-};
-
 struct SrcDevSuper : ChildGrid {
     const double *Kmat, *Esub, *uf, *ux;
     int64_t ldk;
@@ -199,6 +193,75 @@ __global__ __launch_bounds__(256) void k_galerkin_l2_mfma(const double *__restri
             for (int r = 0; r < 4; ++r) Ks[(int64_t)(16 * t + 4 * r + lk) * ldk + e0 + 16 * g + li] = acc[g][r];
 #pragma unroll
         for (int kk = 0; kk < KS; ++kk) a[kk] = an[kk];
+    }
+}
+
+// Levels 3 and up (span 2): Ks_e = sum over the 8 children of P_s' K_s P_s, P_s = W_s (x) I_3.  For one pair (d, f)
+// of components that is 64 outputs (i, j) from 8 x 64 inputs, sum W_s(a, i) W_s(b, j) K_s(3 a + d, 3 b + f), with
+// the same coefficients for every element: a product on the matrix cores, 16 elements to a tile's columns.
+// A workgroup has 16 consecutive coarse elements and one pair; its wavefronts take two children each and add
+// up through LDS in wavefront order.  The matrices are symmetric, so the pairs d < f give the entries (f, d)
+// too.  Lanes load 16 neighbouring elements' entries (every second one: the other child reads those
+// between), and products whose weights are all zero (7 of 16) are left out.  Children outside the mesh
+// have zero matrices.  Bound by reading the finer level's matrices: at 128 x 256 x 128 (201 MB of them) 188
+// us, against 714 for one wavefront per element that gathered each child's 576 entries singly.
+__global__ __launch_bounds__(256) void k_galerkin_half(const double *__restrict__ prev, int64_t ldp, int cEY, int cEX,
+                                                       int64_t nC, int fEY, int fEX, const double *__restrict__ P,
+                                                       double *__restrict__ Ks, int64_t ldk) {
+    __shared__ double2 red[4][4][128];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, li = lane & 15, lk = lane >> 4;
+    const int pair = blockIdx.y, d = pair < 3 ? pair : (pair == 5 ? 1 : 0), f = pair < 3 ? pair : (pair == 3 ? 1 : 2);
+    const int64_t e0 = (int64_t)blockIdx.x * 16 + li, ce = e0 < nC ? e0 : 0;
+    const int cy = (int)(ce % cEY), cx = (int)((ce / cEY) % cEX), cz = (int)(ce / ((int64_t)cEY * cEX));
+    tg_dbl4 acc[4];
+#pragma unroll
+    for (int t = 0; t < 4; ++t) acc[t] = tg_dbl4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+        const int s = 2 * w + c, sy = s & 1, sx = (s >> 1) & 1, sz = s >> 2;
+        const double *src = prev + (2 * cy + sy) + (int64_t)fEY * ((2 * cx + sx) + (int64_t)fEX * (2 * cz + sz));
+        const double *Ps = P + 576 * s;
+        double v[16], wa[2], wb[8][4];
+#pragma unroll
+        for (int k = 0; k < 16; ++k)  // K_s(3 a + d, 3 b + f), a = 4 (k % 2) + lk, b = k / 2
+            v[k] = src[(int64_t)(3 * (4 * (k & 1) + lk) + d + 24 * (3 * (k >> 1) + f)) * ldp];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) wa[h] = Ps[3 * (4 * h + lk) + 72 * (li & 7)];
+#pragma unroll
+        for (int b = 0; b < 8; ++b)
+#pragma unroll
+            for (int t = 0; t < 4; ++t) wb[b][t] = Ps[3 * b + 72 * (2 * t + (li >> 3))];
+#pragma unroll
+        for (int b = 0; b < 8; ++b)
+#pragma unroll
+            for (int t = 0; t < 4; ++t)
+                if (__ballot(wb[b][t] != 0.0))
+#pragma unroll
+                    for (int h = 0; h < 2; ++h)
+                        acc[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(wa[h] * wb[b][t], v[2 * b + h], acc[t], 0, 0, 0);
+    }
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+        red[w][t][lane] = make_double2(acc[t][0], acc[t][1]);
+        red[w][t][64 + lane] = make_double2(acc[t][2], acc[t][3]);
+    }
+    __syncthreads();
+    double2 x = red[0][w][lane], y = red[0][w][64 + lane];  // tile w's sum
+#pragma unroll
+    for (int k = 1; k < 4; ++k) {
+        const double2 x1 = red[k][w][lane], y1 = red[k][w][64 + lane];
+        x.x += x1.x;
+        x.y += x1.y;
+        y.x += y1.x;
+        y.y += y1.y;
+    }
+    if (e0 >= nC) return;
+    const double o[4] = {x.x, x.y, y.x, y.y};
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        const int m = 4 * r + lk, i = m & 7, j = 2 * w + (m >> 3);
+        Ks[(int64_t)(3 * i + d + 24 * (3 * j + f)) * ldk + e0] = o[r];
+        if (d != f) Ks[(int64_t)(3 * j + f + 24 * (3 * i + d)) * ldk + e0] = o[r];
     }
 }
 
@@ -555,10 +618,9 @@ void Solver::assemble() {
             src.Kmat = F.Ks64; src.ldk = F.ldk; src.Esub = Esub; src.uf = uFree; src.ux = uFixed; src.uid = fullUid;
             k_galerkin_dev<<<grid, GK_THREADS, 0, st>>>(src, C.eleMask, nCh, C.P, C.Ks64, C.ldk);
         } else {
-            SrcDevHigher src;
-            static_cast<ChildGrid &>(src) = cg;
-            src.prev = Fi.Ks64; src.ldp = Fi.ldk;
-            k_galerkin_dev<<<grid, GK_THREADS, 0, st>>>(src, C.eleMask, nCh, C.P, C.Ks64, C.ldk);
+            if (nCh != 8) fail(TG_ERR_ARGS, id, "Galerkin level %d: %d children per coarse element", i + 1, nCh);
+            k_galerkin_half<<<dim3(grid_for(C.g.elems(), 16), 6), 256, 0, st>>>(Fi.Ks64, Fi.ldk, C.g.EY, C.g.EX, C.g.elems(),
+                                                                            Fi.g.EY, Fi.g.EX, C.P, C.Ks64, C.ldk);
         }
         TG_LAUNCH_CHECK(id);
     }
