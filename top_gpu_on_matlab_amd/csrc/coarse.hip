@@ -107,25 +107,31 @@ struct SchurProb {
     SchurTerm t[2];
 };
 
+// The three DOF rows of a node share their column pattern, so a thread forms one column of all three from the
+// same 27 entries of N; the couplings are uniform over the workgroup.  Only the lower block triangle is formed,
+// which is what the sweep reads.  Bound by reading N from the cache: 30 us per launch at 128 x 256 x 128 with a
+// thread per row and column over the whole square, 16 this way.
 __global__ __launch_bounds__(256) void k_schur(const SchurProb A, const SchurProb B) {
     const SchurProb &q = blockIdx.z ? B : A;
-    const int64_t i = blockIdx.y, j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= q.n || j >= q.n) return;
-    double acc = 0.0;
+    const int64_t i = 3 * (int64_t)blockIdx.y, j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= q.n || j >= q.n || j / CB > (i + 2) / CB) return;
+    double acc[3] = {0.0, 0.0, 0.0};
     for (int s = 0; s < q.nt; ++s) {
         const double *V = q.t[s].V + i * NCPL;
         const int32_t *C = q.t[s].C + i * NCPL;
         const double *N = q.t[s].N + j;
-        double a0 = 0.0, a1 = 0.0, a2 = 0.0;
+        double a[3][3] = {};
 #pragma unroll
-        for (int k = 0; k < NCPL; k += 3) {
-            a0 += V[k] * N[(int64_t)C[k] * q.t[s].ldN];
-            a1 += V[k + 1] * N[(int64_t)C[k + 1] * q.t[s].ldN];
-            a2 += V[k + 2] * N[(int64_t)C[k + 2] * q.t[s].ldN];
+        for (int k = 0; k < NCPL; ++k) {
+            const double v = N[(int64_t)C[k] * q.t[s].ldN];
+#pragma unroll
+            for (int d = 0; d < 3; ++d) a[d][k % 3] += V[d * NCPL + k] * v;
         }
-        acc += (a0 + a1) + a2;
+#pragma unroll
+        for (int d = 0; d < 3; ++d) acc[d] += (a[d][0] + a[d][1]) + a[d][2];
     }
-    q.S[i * q.np + j] -= acc;
+#pragma unroll
+    for (int d = 0; d < 3; ++d) q.S[(i + d) * q.np + j] -= acc[d];
 }
 
 // ---- blocked symmetric sweep: S <- S^-1 in place of an SPD plane block, pivot blocks K = 0 .. nb-1 --------
@@ -543,35 +549,43 @@ struct DSProb {
     int64_t ld, col0;
 };
 
-// One thread per output column 3 jn + c and run of DS_ROWS rows: the column's 27 couplings and their
-// columns stay in registers over the run, the rows' gathered entries come from the cache (the lanes of
-// a wavefront share the row), and lanes write consecutive columns.  (A thread per row and column node
-// re-read the couplings for every row: 167 us per launch at 128 x 256 x 128.)
-constexpr int DS_ROWS = 16;
+// S is symmetric, so S(i, C_k) is read as S(C_k, i), along the rows i of a wavefront's lanes: 27 coalesced loads
+// give a node's three columns for 64 rows, with the node's couplings uniform over the wavefront.  A workgroup
+// has 64 rows and DS_NODES nodes; its columns turn through LDS so that they are written along the rows of Out.
+// Bound by reading S from the cache: 46 us per launch at 128 x 256 x 128 with gathered entries (a thread per column
+// and run of 16 rows), 22 this way.
+constexpr int DS_NODES = 16, DS_LD = 3 * DS_NODES + 1;
 __global__ __launch_bounds__(256) void k_dense_sparse(const DSProb P0, const DSProb P1, const DSProb P2,
                                                       const DSProb P3) {
+    __shared__ double out[64 * DS_LD];
     const DSProb &q = blockIdx.y == 0 ? P0 : (blockIdx.y == 1 ? P1 : (blockIdx.y == 2 ? P2 : P3));
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int64_t ncol = 3 * q.ncn, nruns = (q.nrows + DS_ROWS - 1) / DS_ROWS;
-    if (t >= ncol * nruns) return;
-    const int64_t jc = t % ncol, i0 = (t / ncol) * DS_ROWS;
-    const int64_t jn = jc / 3;
-    const int32_t *C = q.C + 3 * jn * NCPL;  // the three DOFs of node jn share their column pattern
-    const double *V = q.V + jc * NCPL;
-    int32_t ck[NCPL];
-    double vk[NCPL];
+    const int64_t runs = (q.nrows + 63) / 64;
+    if ((int64_t)blockIdx.x >= runs * ((q.ncn + DS_NODES - 1) / DS_NODES)) return;
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int64_t i0 = 64 * (blockIdx.x % runs), j0 = DS_NODES * (blockIdx.x / runs);
+    const double *S = q.S + (i0 + lane < q.nrows ? i0 + lane : q.nrows - 1);
 #pragma unroll
-    for (int k = 0; k < NCPL; ++k) {
-        ck[k] = C[k];
-        vk[k] = V[k];
+    for (int t = 0; t < DS_NODES / 4; ++t) {
+        const int64_t jn = j0 + 4 * t + w;
+        if (jn < q.ncn) {
+            const int32_t *C = q.C + 3 * jn * NCPL;  // the three DOFs of node jn share their column pattern
+            const double *V = q.V + 3 * jn * NCPL;
+            double o[3] = {0.0, 0.0, 0.0};
+#pragma unroll
+            for (int k = 0; k < NCPL; ++k) {
+                const double v = S[(int64_t)C[k] * q.np];
+#pragma unroll
+                for (int c = 0; c < 3; ++c) o[c] += v * V[c * NCPL + k];
+            }
+#pragma unroll
+            for (int c = 0; c < 3; ++c) out[lane * DS_LD + 3 * (4 * t + w) + c] = o[c];
+        }
     }
-    const int64_t i1 = i0 + DS_ROWS < q.nrows ? i0 + DS_ROWS : q.nrows;
-    for (int64_t i = i0; i < i1; ++i) {
-        const double *srow = q.S + i * q.np;
-        double o = 0.0;
-#pragma unroll
-        for (int k = 0; k < NCPL; ++k) o += srow[ck[k]] * vk[k];
-        q.Out[i * q.ld + q.col0 + jc] = o;
+    __syncthreads();
+    const int ncol = (int)(3 * (q.ncn - j0 < DS_NODES ? q.ncn - j0 : DS_NODES));
+    for (int idx = threadIdx.x; idx < 64 * 3 * DS_NODES; idx += 256) {
+        const int r = idx / (3 * DS_NODES), c = idx % (3 * DS_NODES);
+        if (c < ncol && i0 + r < q.nrows) q.Out[(i0 + r) * q.ld + q.col0 + 3 * j0 + c] = out[r * DS_LD + c];
     }
 }
 
@@ -1068,7 +1082,7 @@ void CoarseSolver::factor(const double *Ks, int64_t ldk, const uint8_t *eleMask,
     auto launch_schur = [&](const SchurProb &A, const SchurProb &B) {
         if (!A.nt && !B.nt) return;
         const int64_t n = std::max(A.nt ? A.n : 0, B.nt ? B.n : 0);
-        k_schur<<<dim3(grid_for(n, 256), (unsigned)n, 2), 256, 0, st>>>(A.nt ? A : noneS, B.nt ? B : noneS);
+        k_schur<<<dim3(grid_for(n, 256), grid_for(n, 3), 2), 256, 0, st>>>(A.nt ? A : noneS, B.nt ? B : noneS);
         TG_LAUNCH_CHECK(id);
     };
     // S_p <- S_p^-1 for up to two planes together
@@ -1112,9 +1126,9 @@ void CoarseSolver::factor(const double *Ks, int64_t ldk, const uint8_t *eleMask,
             const int cnt = (int)std::min<size_t>(4, ops.size() - i0);
             for (int y = 0; y < cnt; ++y) {
                 q[y] = ops[i0 + y];
-                work = std::max(work, 3 * q[y].ncn * ((q[y].nrows + DS_ROWS - 1) / DS_ROWS));
+                work = std::max(work, ((q[y].ncn + DS_NODES - 1) / DS_NODES) * ((q[y].nrows + 63) / 64));
             }
-            if (work) k_dense_sparse<<<dim3(grid_for(work, 256), cnt), 256, 0, st>>>(q[0], q[1], q[2], q[3]);
+            if (work) k_dense_sparse<<<dim3((unsigned)work, cnt), 256, 0, st>>>(q[0], q[1], q[2], q[3]);
         }
         TG_LAUNCH_CHECK(id);
         ops.clear();
