@@ -419,6 +419,28 @@ def test_coarse_solve_planes_wider_than_1024_dofs():
     assert its < 400 and true_res < 1.5e-6
 
 
+@pytest.mark.parametrize('shape', [(6, 9, 7), (24, 48, 24), (45, 83, 37), (64, 128, 64)])
+def test_finest_product_chunk_chosen_by_grid(shape):
+    """The tiled finest product with its planes per workgroup chosen by the grid (1 to 4 at these sizes) against
+    chunks of 12: a node's value does not depend on the chunk, so K*u in FP64 and the mixed V-cycle are
+    the same bit for bit."""
+    import torch
+    from top_gpu_on_matlab_amd.model import cuboid_model
+    from top_gpu_on_matlab_amd.solver import Solver
+    out = []
+    for zchunk in (None, 12):
+        s = Solver(cuboid_model(*shape, 1, precision='mixed'))
+        if zchunk:
+            s.set_tuning(kfine_zchunk=zchunk)
+        g = torch.Generator().manual_seed(7)
+        s.set_modulus(0.1 + torch.rand(s.model.num_elements, generator=g, dtype=torch.float64).cuda())
+        s.assemble()
+        u = (2 * torch.rand(s.ndof(), generator=g, dtype=torch.float64) - 1).cuda()
+        out.append((s.kbyu(u), s.vcycle(u)))
+    assert torch.equal(out[0][0], out[1][0])
+    assert torch.equal(out[0][1], out[1][1])
+
+
 @pytest.mark.parametrize('shape, blocks', [((24, 48, 24), 1), ((32, 48, 32), 2), ((56, 64, 56), 3), ((56, 64, 64), 4),
                                            ((128, 136, 128), 14)])
 def test_coarse_factorisation_at_block_edges(shape, blocks):

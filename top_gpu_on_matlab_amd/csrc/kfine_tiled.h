@@ -109,6 +109,34 @@ inline KTiles ktiles_for(const Grid &g, int zchunk) {
     return t;
 }
 
+// Node planes per workgroup where none are asked for.  A workgroup marches through zchunk + 1 element layers
+// in turn, so few long chunks leave the chip idle on small grids (24 x 48 x 24 in chunks of 12: 24 workgroups),
+// and a last round of few workgroups on larger ones; short chunks compute more layers twice.  The chip holds
+// `waves` (3 in FP64, 4 in FP32) workgroups per CU at once; the time of a layer with k of them on each CU, and
+// what a last round of k adds to full ones, are measured (us, plain product, 21 x 10 grids and chunks from
+// 8 x 16 x 8 to 128 x 256 x 128).  The chunk of the least sum (zchunk + 1) x (rounds) is within 3% of the
+// best measured one in FP64 and 9% in FP32.  Against chunks of 12: 5.9 from 21.9 us in FP64 at 24 x 48 x 24,
+// 17.6 from 29.4 at 64 x 128 x 64, 38.8 from 50.2 at 96 x 192 x 96 (FP32 4.9 from 17.1, 12.2 from 19.7, 22.8 from 27.5);
+// at 128 x 256 x 128 it is 12 again.
+inline int kfine_chunk_for(const Grid &g, int waves, int cus) {
+    constexpr double alone[2][5] = {{0, 1.45, 2.1, 2.7, 2.7}, {0, 1.07, 1.45, 1.75, 2.0}};
+    constexpr double after[2][5] = {{0, 1.1, 1.75, 2.6, 2.6}, {0, 0.8, 0.95, 1.4, 2.0}};
+    constexpr double round[2] = {2.6, 2.0};
+    const int v = waves >= 4 ? 1 : 0, slots = v ? 4 : 3;
+    int best = 1;
+    double least = 1e300;
+    for (int z = 1; z <= g.NZ && z <= 4096; ++z) {
+        const int64_t n = ktiles_for(g, z).count(), full = n / (slots * cus), rest = n % (slots * cus);
+        const int k = (int)((rest + cus - 1) / cus);
+        const double t = 2.5 + (z + 1) * (full ? full * round[v] + after[v][k] : alone[v][k]);
+        if (t < least) {
+            least = t;
+            best = z;
+        }
+    }
+    return best;
+}
+
 // 8-point Walsh butterflies over q: forward m = W^T x, inverse x = W g.
 template <typename T>
 __device__ __forceinline__ void walsh_fwd(T x[8]) {

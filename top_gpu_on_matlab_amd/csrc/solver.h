@@ -49,7 +49,8 @@ struct Solver {
     std::vector<TimedLaunch> tpool;
     size_t tused = 0;
     hipEvent_t *timing_slot(int key);
-    int kfine_zchunk = 12;  // node planes per workgroup of the tiled kernel
+    int kfine_zchunk = 0;   // node planes per workgroup of the tiled kernel (0: by the grid, kfine_chunk_for)
+    int kfine_auto[2] = {12, 12};  // that choice in FP64 and FP32
     int kfine_mfma = 0;     // FP32 tiled finest K*u: 0 Walsh form, 1 / 2 element products on MFMA (FP32 / BF16)
     int kelem_parts = 1;    // threads per element in the FP64 per-element-matrix K*u (1: packed symmetric)
     bool has_modulus = false, assembled = false;
@@ -77,6 +78,10 @@ struct Solver {
     template <typename T>
     bool kbyu_level(int i, const T *u, T *out, int epi, const T *rr, const T *dg, int dot_slot = -1,
                     T *xout = nullptr);
+    // the finest product's tiles; products on the matrix cores keep as few waves as FP64
+    KTiles fine_tiles(bool f64) const {
+        return ktiles_for(lv[0].g, kfine_zchunk ? kfine_zchunk : kfine_auto[f64 || kfine_mfma ? 0 : 1]);
+    }
     bool fine_tiled() const { return !super && kfine_kernel == 0 && walsh_ok; }
     template <typename T>
     // pk (optional): also write the coarsest level's plane-order copy for its persistent solve

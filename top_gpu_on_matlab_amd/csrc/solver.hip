@@ -437,6 +437,10 @@ Solver::Solver(const tg_model &m, hipStream_t s) : model(m), st(s) {
         }
     }
     DevLevel &F = lv[0];
+    int dev = 0, cus = 0;
+    TG_HIP(hipGetDevice(&dev), id);
+    TG_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev), id);
+    for (int v = 0; v < 2; ++v) kfine_auto[v] = kfine_chunk_for(F.g, 3 + v, std::max(cus, 1));
     K0_64.upload(m.Ke, st);
     {
         // Walsh-basis form of the finest element matrix for the tiled K*u (isotropic: 45 entries)
@@ -762,7 +766,7 @@ bool Solver::kbyu_level(int i, const T *u, T *out, int epi, const T *rr, const T
         const T *K0 = f64 ? (const T *)K0_64.p : (const T *)K0_32.p;
         const T cs = (T)model.prm.cell_size;
         if (kfine_kernel == 0 && walsh_ok) {
-            const KTiles kt = ktiles_for(D.g, kfine_zchunk);
+            const KTiles kt = fine_tiles(f64);
             const unsigned gt = (unsigned)kt.count();
             hipEvent_t *ev = (time_fine == 1 || (time_fine == 2 && epi == EPI_KU)) ? timing_slot((f64 ? 0 : 4) + epi) : nullptr;
             double *dp = nullptr;
@@ -907,7 +911,7 @@ void Solver::vcycle_t(const T *r0, T *z0) {
         T *out = (i == 0) ? z0 : vec<T>(D, 2);
         if (i == 0 && sizeof(T) == 4 && r64_dot) {
             // mixed: z = x + omega (r - K x) ./ d in FP32, with z.r against the FP64 r
-            const KTiles kt = ktiles_for(D.g, kfine_zchunk);
+            const KTiles kt = fine_tiles(false);
             const unsigned gt = (unsigned)kt.count();
             if ((int64_t)dotp.n < (int64_t)gt) dotp.alloc(gt);
             const float *x32 = (const float *)xx[0], *r32 = (const float *)rr[0], *d32 = D.diag32.p;
