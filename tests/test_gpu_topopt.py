@@ -76,6 +76,38 @@ def test_convolution_filter():
     assert _rel(gf.adjoint(_t(x)).cpu().numpy(), cf.adjoint(x).reshape(-1, order='F')) < 1e-13
 
 
+@pytest.mark.parametrize('r', [0.9, 1.5, 4 * math.sqrt(3), 9.0, 12.5, 13.2])
+@pytest.mark.parametrize('dims, num', [((1, 1, 1), 1), ((3, 17, 5), 1), ((2, 9, 3), 4), ((13, 2, 7), 3)])
+def test_convolution_filter_reach_and_edges(r, dims, num):
+    """Every reach class of the cone (a single voxel, up to 12 voxels in the tiled form, beyond it) on grids that are
+    smaller than a tile or end inside one, against scipy's zero-padded correlation of the same cone; sums
+    of at most 25^3 positive terms in FP64, so 1e-12 is far above their rounding.  A NaN reaches exactly
+    the voxels within the cone."""
+    import ctypes
+    import scipy.ndimage
+    import torch
+    from top_gpu_on_matlab_amd import top_gpu as G
+    nelx, nely, nelz = dims
+    gf = G.ConvolutionFilter(nelx, nely, nelz, r, num)
+    c = math.ceil(r)
+    v = np.arange(-c + 1, c)
+    dy, dx, dz = np.meshgrid(v, v, v, indexing='ij')
+    h = np.maximum(0.0, r - np.sqrt(dx ** 2 + dy ** 2 + dz ** 2))
+    shape = (num * nely, num * nelx, num * nelz)
+    conv = lambda a: scipy.ndimage.correlate(a, h, mode='constant', cval=0.0)
+    def grid(vec):  # element-major -> [y, x, z]
+        a = vec.reshape(nelz, nelx, nely, num, num, num).transpose(2, 5, 1, 4, 0, 3)
+        return np.ascontiguousarray(a.reshape(shape))
+    rng = np.random.default_rng(4)
+    x = rng.random(num ** 3 * nelx * nely * nelz)
+    Hs = conv(np.ones(shape))
+    assert _rel(grid(gf.forward(_t(x)).cpu().numpy()), conv(grid(x)) / Hs) < 1e-12
+    assert _rel(grid(gf.adjoint(_t(x)).cpu().numpy()), conv(grid(x) / Hs)) < 1e-12
+    x[x.size // 2] = np.nan
+    hit = conv(np.isnan(grid(x)).astype(float)) > 0
+    assert np.array_equal(np.isnan(grid(gf.forward(_t(x)).cpu().numpy())), hit)
+
+
 def test_oc_update_matches_bisection():
     from top_gpu_on_matlab_amd import top_gpu as G
     rng = np.random.default_rng(3)
