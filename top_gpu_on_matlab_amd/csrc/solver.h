@@ -63,6 +63,7 @@ struct Solver {
     DevBuf<int64_t> bndList;               // coarse elements with boundary (fixed-DOF) children, ...
     DevBuf<int32_t> bndPtr;                // ... where each one's children start in bndChild (BndChild records)
     DevBuf<unsigned char> bndChild;
+    DevBuf<double> Gpart;                  // partial sums of a Galerkin product in slices
     int64_t nBnd = 0;
     DevBuf<double> b, y;        // PCG right-hand side and iterate (full fine grid)
     PcgWork pw;                 // PCG work vectors

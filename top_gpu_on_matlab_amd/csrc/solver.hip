@@ -7,7 +7,6 @@
 #include <cmath>
 
 #include "coarse.h"
-#include "galerkin.h"
 #include "kernels.h"
 #include "kfine_tiled.h"
 #include "model.h"
@@ -17,49 +16,7 @@
 namespace tg {
 namespace {
 
-// ---- Galerkin sources, structured layouts -------------------------------------------------
-struct ChildGrid {
-    int span, cEY, cEX, fEY, fEX;
-    const uint8_t *fineSolid;
-    int64_t ce;
-    __device__ int child(int s) const {
-        const int a = s % span, b = (s / span) % span, c = s / (span * span);
-        const int cy = (int)(ce % cEY), cx = (int)((ce / cEY) % cEX), cz = (int)(ce / ((int64_t)cEY * cEX));
-        const int64_t f = (int64_t)(span * cy + a) + (int64_t)fEY * ((span * cx + b) + (int64_t)fEX * (span * cz + c));
-        return fineSolid[f] ? (int)f : -1;
-    }
-};
-
-struct SrcDevSuper : ChildGrid {
-    const double *Kmat, *Esub, *uf, *ux;
-    int64_t ldk;
-    const int32_t *uid;
-    __device__ double kch(int f, int i) const {
-        const int32_t u = uid[f];
-        if (u > 0) {
-            const size_t fb = (size_t)(u - 1) * 576 * 64, mb = (size_t)f * 64;
-            double acc = 0;
-            for (int q = 0; q < 64; ++q) acc += uf[fb + (size_t)q * 576 + i] * Esub[mb + q];
-            return acc + ux[(size_t)(u - 1) * 576 + i];
-        }
-        return Kmat[(int64_t)i * ldk + f];
-    }
-};
-
-template <class Src>
-__global__ __launch_bounds__(GK_THREADS) void k_galerkin_dev(Src src, const uint8_t *__restrict__ cSolid,
-                                                             int nCh, const double *__restrict__ P,
-                                                             double *__restrict__ Ks, int64_t ldk) {
-    __shared__ double sB[576], sK[576], sT[576];
-    const int64_t ce = blockIdx.x;
-    if (!cSolid[ce]) return;
-    src.ce = ce;
-    double acc[9];
-    galerkin_block(acc, src, nCh, P, sB, sK, sT);
-#pragma unroll
-    for (int i = 0; i < 9; ++i) Ks[(int64_t)galerkin_entry(i) * ldk + ce] = acc[i];
-}
-
+// ---- Galerkin products, structured layouts ---------------------------------------------------
 // Level 2, standard voxels: the children with fixed DOFs, which the moduli product (k_galerkin_l2_mfma) leaves
 // out, added to their coarse elements: Ks_e += sum P_s' (E_f Ufree_u + Ufixed_u) P_s over the listed children of
 // the element (slot s, fine element f, boundary matrices u).  P_s = W_s (x) I_3 with the 8 x 8 trilinear
@@ -68,10 +25,12 @@ __global__ __launch_bounds__(GK_THREADS) void k_galerkin_dev(Src src, const uint
 // has 16), and their sums added in wavefront order.  Bound by the chain of a child's loads and its two
 // products; recomputing all 64 children of such an element in one wavefront took 460 us at 96 x 192 x 96 and 510
 // at 128 x 256 x 128, this 45 and 86.
+// SUPER: super-element children, sum_q Esub(q, f) Ufree_u,q + Ufixed_u over their 64 sub-voxels.
 struct BndChild {
     int32_t slot, fine, uid;
 };
 constexpr int GB_WAVES = 4;
+template <bool SUPER>
 __global__ __launch_bounds__(64 * GB_WAVES) void k_galerkin_bnd(const int64_t *__restrict__ list,
                                                                 const int32_t *__restrict__ ptr,
                                                                 const BndChild *__restrict__ child,
@@ -88,7 +47,7 @@ __global__ __launch_bounds__(64 * GB_WAVES) void k_galerkin_bnd(const int64_t *_
     for (int cb = c0; cb < c1; cb += GB_WAVES) {  // uniform over the workgroup
         const bool on = cb + w < c1;
         const BndChild ch = child[on ? cb + w : c0];
-        const double e = on ? E[ch.fine] : 0.0;
+        const double e = !SUPER && on ? E[ch.fine] : 0.0;
         double wj[8], wi[8];  // W_s(b, j), W_s(b, a)
 #pragma unroll
         for (int b = 0; b < 8; ++b) {
@@ -99,7 +58,16 @@ __global__ __launch_bounds__(64 * GB_WAVES) void k_galerkin_bnd(const int64_t *_
 #pragma unroll
         for (int k = 0; k < 9; ++k) {
             const size_t i = (size_t)ch.uid * 576 + 64 * k + lane;
-            sK[w][64 * k + lane] = on ? uf[i] * e + ux[i] : 0.0;
+            double v = 0.0;
+            if (SUPER && on) {
+                const double *u = uf + (size_t)ch.uid * (576 * 64) + 64 * k + lane, *es = E + (size_t)ch.fine * 64;
+#pragma unroll 16
+                for (int q = 0; q < 64; ++q) v += u[(size_t)q * 576] * es[q];
+                v += ux[i];
+            } else if (on) {
+                v = uf[i] * e + ux[i];
+            }
+            sK[w][64 * k + lane] = v;
         }
         __syncthreads();
         double t[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};  // t(d, f) = sum_b K(3 a + d, 3 b + f) W(b, j)
@@ -158,8 +126,11 @@ __global__ void k_gather_children(const double *__restrict__ E, const uint8_t *_
 // 2.5 us per tile (FP64 MFMA), so where the elements alone do not fill the chip the tiles are shared
 // out: all 36 in one wavefront took 88 us at any size below 65,536 elements; shared out 7 us at 432 elements
 // and 60 at 27,648 (from 93); at 65,536 it stays at 100, the result's 302 MB and 4.8 GFLOP.
+// EMAJOR: the moduli element by element, Ech[4 KS e + k], and G = I_mat: K_mat = I_mat * E_sub of every
+// super-element (TOP_GPU.m:1101-1103), 4 KS = 64 sub-voxels; 762 us at 16,384 elements with a thread per entry that
+// read both operands for each product, 57 here.
 typedef double tg_dbl4 __attribute__((ext_vector_type(4)));
-template <int KS, int NG>
+template <int KS, int NG, bool EMAJOR = false>
 __global__ __launch_bounds__(256) void k_galerkin_l2_mfma(const double *__restrict__ Ech, const double *__restrict__ G,
                                                           double *__restrict__ Ks, int64_t ldk, int tiles) {
     const int lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4;
@@ -170,7 +141,8 @@ __global__ __launch_bounds__(256) void k_galerkin_l2_mfma(const double *__restri
 #pragma unroll
     for (int g = 0; g < NG; ++g)
 #pragma unroll
-        for (int kk = 0; kk < KS; ++kk) b[g][kk] = Ech[(e0 + 16 * g + li) + ldk * (lk + 4 * kk)];
+        for (int kk = 0; kk < KS; ++kk)
+            b[g][kk] = EMAJOR ? Ech[4 * KS * (e0 + 16 * g + li) + lk + 4 * kk] : Ech[(e0 + 16 * g + li) + ldk * (lk + 4 * kk)];
     const double *gp = G + (int64_t)lk * 576 + li;
     double a[KS];
 #pragma unroll
@@ -196,18 +168,23 @@ __global__ __launch_bounds__(256) void k_galerkin_l2_mfma(const double *__restri
     }
 }
 
-// Levels 3 and up (span 2): Ks_e = sum over the 8 children of P_s' K_s P_s, P_s = W_s (x) I_3.  For one pair (d, f)
-// of components that is 64 outputs (i, j) from 8 x 64 inputs, sum W_s(a, i) W_s(b, j) K_s(3 a + d, 3 b + f), with
-// the same coefficients for every element: a product on the matrix cores, 16 elements to a tile's columns.
-// A workgroup has 16 consecutive coarse elements and one pair; its wavefronts take two children each and add
-// up through LDS in wavefront order.  The matrices are symmetric, so the pairs d < f give the entries (f, d)
-// too.  Lanes load 16 neighbouring elements' entries (every second one: the other child reads those
-// between), and products whose weights are all zero (7 of 16) are left out.  Children outside the mesh
-// have zero matrices.  Bound by reading the finer level's matrices: at 128 x 256 x 128 (201 MB of them) 188
-// us, against 714 for one wavefront per element that gathered each child's 576 entries singly.
-__global__ __launch_bounds__(256) void k_galerkin_half(const double *__restrict__ prev, int64_t ldp, int cEY, int cEX,
-                                                       int64_t nC, int fEY, int fEX, const double *__restrict__ P,
-                                                       double *__restrict__ Ks, int64_t ldk) {
+// Coarse element matrices from the finer level's: Ks_e = sum over the SPAN^3 children of P_s' K_s P_s,
+// P_s = W_s (x) I_3.  For one pair (d, f) of components that is 64 outputs (i, j) from 64 inputs a child,
+// sum W_s(a, i) W_s(b, j) K_s(3 a + d, 3 b + f), with the same coefficients for every element: a product on the
+// matrix cores, 16 elements to a tile's columns.  A workgroup has 16 consecutive coarse elements, one pair and
+// (blockIdx.z) a slice of the children; its wavefronts take `per` children each and add up through LDS in
+// wavefront order.  Slices (few elements, many children) leave partial sums for k_sum_slices.  The matrices are
+// symmetric, so the pairs d < f give the entries (f, d) too.  Lanes load 16 neighbouring elements' entries
+// (at a stride of SPAN: the other children read those between), and products whose weights are all zero are
+// left out.  Children outside the mesh have zero matrices; children with boundary matrices (uid > 0, super-element
+// level 2) are left to k_galerkin_bnd.  Bound by reading the finer level's matrices: levels 3 and up at 128 x 256 x 128
+// (201 MB of them) 188 us, against 714 for one wavefront per element that gathered each child's 576 entries
+// singly; super-element level 2 of a 64 x 16 x 16 grid 63 with the slices' sum, against 477.
+template <int SPAN>
+__global__ __launch_bounds__(256) void k_galerkin_children(const double *__restrict__ prev, int64_t ldp,
+                                                           const int32_t *__restrict__ uid, int cEY, int cEX, int64_t nC,
+                                                           int fEY, int fEX, const double *__restrict__ P, int per,
+                                                           double *__restrict__ Ks, int64_t ldk) {
     __shared__ double2 red[4][4][128];
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, li = lane & 15, lk = lane >> 4;
     const int pair = blockIdx.y, d = pair < 3 ? pair : (pair == 5 ? 1 : 0), f = pair < 3 ? pair : (pair == 3 ? 1 : 2);
@@ -216,15 +193,18 @@ __global__ __launch_bounds__(256) void k_galerkin_half(const double *__restrict_
     tg_dbl4 acc[4];
 #pragma unroll
     for (int t = 0; t < 4; ++t) acc[t] = tg_dbl4{0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-    for (int c = 0; c < 2; ++c) {
-        const int s = 2 * w + c, sy = s & 1, sx = (s >> 1) & 1, sz = s >> 2;
-        const double *src = prev + (2 * cy + sy) + (int64_t)fEY * ((2 * cx + sx) + (int64_t)fEX * (2 * cz + sz));
-        const double *Ps = P + 576 * s;
+#pragma unroll 2
+    for (int c = 0; c < per; ++c) {
+        const int s = ((int)blockIdx.z * 4 + w) * per + c, sy = s % SPAN, sx = (s / SPAN) % SPAN, sz = s / (SPAN * SPAN);
+        const int64_t fe = (SPAN * cy + sy) + (int64_t)fEY * ((SPAN * cx + sx) + (int64_t)fEX * (SPAN * cz + sz));
+        const double *src = prev + fe, *Ps = P + 576 * s;
+        const bool out = uid && uid[fe] > 0;
         double v[16], wa[2], wb[8][4];
 #pragma unroll
-        for (int k = 0; k < 16; ++k)  // K_s(3 a + d, 3 b + f), a = 4 (k % 2) + lk, b = k / 2
+        for (int k = 0; k < 16; ++k) {  // K_s(3 a + d, 3 b + f), a = 4 (k % 2) + lk, b = k / 2
             v[k] = src[(int64_t)(3 * (4 * (k & 1) + lk) + d + 24 * (3 * (k >> 1) + f)) * ldp];
+            v[k] = out ? 0.0 : v[k];
+        }
 #pragma unroll
         for (int h = 0; h < 2; ++h) wa[h] = Ps[3 * (4 * h + lk) + 72 * (li & 7)];
 #pragma unroll
@@ -257,23 +237,22 @@ __global__ __launch_bounds__(256) void k_galerkin_half(const double *__restrict_
     }
     if (e0 >= nC) return;
     const double o[4] = {x.x, x.y, y.x, y.y};
+    double *K = Ks + (int64_t)blockIdx.z * 576 * ldk + e0;
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
         const int m = 4 * r + lk, i = m & 7, j = 2 * w + (m >> 3);
-        Ks[(int64_t)(3 * i + d + 24 * (3 * j + f)) * ldk + e0] = o[r];
-        if (d != f) Ks[(int64_t)(3 * j + f + 24 * (3 * i + d)) * ldk + e0] = o[r];
+        K[(int64_t)(3 * i + d + 24 * (3 * j + f)) * ldk] = o[r];
+        if (d != f) K[(int64_t)(3 * j + f + 24 * (3 * i + d)) * ldk] = o[r];
     }
 }
 
-// K_mat = I_mat * E_sub per element (TOP_GPU.m:1101-1103), entry-major output.
-__global__ void k_kmat(const double *__restrict__ Imat, const double *__restrict__ Esub, double *__restrict__ Km,
-                       int64_t ldk, int64_t nE) {
+// Ks = sum of the slices' partial sums, in order (entries of elements past the grid are not written by them).
+__global__ void k_sum_slices(const double *__restrict__ part, int slices, int64_t ldk, int64_t nC, double *__restrict__ Ks) {
     const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= nE * 576) return;
-    const int64_t e = t % nE, i = t / nE;
-    double acc = 0;
-    for (int q = 0; q < 64; ++q) acc += Imat[i + 576 * q] * Esub[q + 64 * e];
-    Km[i * ldk + e] = acc;
+    if (t >= 576 * ldk || t % ldk >= nC) return;
+    double s = part[t];
+    for (int k = 1; k < slices; ++k) s += part[(int64_t)k * 576 * ldk + t];
+    Ks[t] = s;
 }
 
 // Jacobi diagonal: sum over solid elements around the node of the element matrix diagonal.
@@ -465,31 +444,34 @@ Solver::Solver(const tg_model &m, hipStream_t s) : model(m), st(s) {
     std::vector<int32_t> uid(nEf, 0);
     for (int64_t k = 0; k < F.Ne; ++k) uid[m.lv[0].eleMapBack[k] - 1] = m.mapUniqueKes[k];
     fullUid.upload(uid, st);
-    if (!super && L >= 2) {
-        // Level-2 Galerkin as a GEMM on the matrix cores: Ks_e = sum_s E_s G_s with G_s = Pch_s' K0 Pch_s
-        // (linear in the children moduli) for children without fixed DOFs; coarse elements with a
-        // boundary child are recomputed child by child.
+    if (L >= 2) {
         DevLevel &C = lv[1];
         const int span = C.span, nCh = span * span * span;
-        std::vector<double> Ph;
-        build_pch(span, Ph);
-        std::vector<double> gt((size_t)nCh * 576, 0.0), tmp(576);
-        for (int sc = 0; sc < nCh; ++sc) {
-            const double *Pc = Ph.data() + (size_t)576 * sc;
-            for (int c = 0; c < 24; ++c)          // tmp = K0 Pch_s
-                for (int a = 0; a < 24; ++a) {
-                    double v = 0;
-                    for (int b = 0; b < 24; ++b) v += m.Ke[a + 24 * b] * Pc[b + 24 * c];
-                    tmp[a + 24 * c] = v;
-                }
-            for (int c = 0; c < 24; ++c)          // G_s = Pch_s' tmp
-                for (int r = 0; r < 24; ++r) {
-                    double v = 0;
-                    for (int a = 0; a < 24; ++a) v += Pc[a + 24 * r] * tmp[a + 24 * c];
-                    gt[(size_t)576 * sc + (r + 24 * c)] = v;
-                }
+        if (!super) {
+            // Level-2 Galerkin as a GEMM on the matrix cores: Ks_e = sum_s E_s G_s with G_s = Pch_s' K0 Pch_s
+            // (linear in the children moduli) over the children without fixed DOFs
+            std::vector<double> Ph;
+            build_pch(span, Ph);
+            std::vector<double> gt((size_t)nCh * 576, 0.0), tmp(576);
+            for (int sc = 0; sc < nCh; ++sc) {
+                const double *Pc = Ph.data() + (size_t)576 * sc;
+                for (int c = 0; c < 24; ++c)          // tmp = K0 Pch_s
+                    for (int a = 0; a < 24; ++a) {
+                        double v = 0;
+                        for (int b = 0; b < 24; ++b) v += m.Ke[a + 24 * b] * Pc[b + 24 * c];
+                        tmp[a + 24 * c] = v;
+                    }
+                for (int c = 0; c < 24; ++c)          // G_s = Pch_s' tmp
+                    for (int r = 0; r < 24; ++r) {
+                        double v = 0;
+                        for (int a = 0; a < 24; ++a) v += Pc[a + 24 * r] * tmp[a + 24 * c];
+                        gt[(size_t)576 * sc + (r + 24 * c)] = v;
+                    }
+            }
+            Gl2.upload(gt, st);
+            Ech.alloc((size_t)nCh * C.ldk);
+            Ech.zero(st);
         }
-        Gl2.upload(gt, st);
         std::vector<int64_t> bnd;  // coarse elements with children that have fixed DOFs, and those children
         std::vector<int32_t> ptr(1, 0);
         std::vector<BndChild> kids;
@@ -512,14 +494,12 @@ Solver::Solver(const tg_model &m, hipStream_t s) : model(m), st(s) {
             bndPtr.upload(ptr, st);
             bndChild.upload((const unsigned char *)kids.data(), kids.size() * sizeof(BndChild), st);
         }
-        Ech.alloc((size_t)nCh * C.ldk);
-        Ech.zero(st);
     }
     uFree.upload(m.uniqueFree, st);
     uFixed.upload(m.uniqueFixed, st);
     if (super) {
         Imat.upload(m.Imat, st);
-        Esub.alloc(64 * nEf);
+        Esub.alloc(64 * F.ldk);  // with the padding that k_galerkin_l2_mfma reads (zero)
         Esub.zero(st);
         F.Ks64.alloc(576 * F.ldk);  // K_mat on the finest level
         F.fv64.alloc(24 * F.ldk);
@@ -587,44 +567,64 @@ void Solver::set_modulus(const double *dE) {
     assembled = false;
 }
 
+// Entry tiles per wavefront of k_galerkin_l2_mfma (64 elements each, 256 per workgroup): shared out until there are
+// four wavefronts for each of the 1024 SIMDs.
+static int l2_tiles(int64_t ldk) { return (int)std::max<int64_t>(1, std::min<int64_t>(36, 36 * (ldk / 64) / 4096)); }
+
 void Solver::assemble() {
     const char *id = "tg_solver_assemble:State";
     if (!has_modulus) fail(TG_ERR_STATE, id, "set the element moduli first");
     DevLevel &F = lv[0];
     if (super) {
-        k_kmat<<<grid_for(F.g.elems() * 576, 256), 256, 0, st>>>(Imat, Esub, F.Ks64, F.ldk, F.g.elems());
+        const int tiles = l2_tiles(F.ldk);
+        k_galerkin_l2_mfma<16, 4, true><<<dim3(grid_for(F.ldk, 256), grid_for(36, tiles)), 256, 0, st>>>(Esub, Imat, F.Ks64,
+                                                                                                F.ldk, tiles);
         TG_LAUNCH_CHECK(id);
     }
     for (int i = 1; i < L; ++i) {
         DevLevel &C = lv[i], &Fi = lv[i - 1];
         const int nCh = C.span * C.span * C.span;
-        ChildGrid cg{C.span, C.g.EY, C.g.EX, Fi.g.EY, Fi.g.EX, Fi.eleMask.p, 0};
-        const unsigned grid = (unsigned)C.g.elems();
         if (i == 1 && !super) {
             const int64_t nC = C.g.elems();
             k_gather_children<<<grid_for(nC * nCh, 256), 256, 0, st>>>(E64, Fi.eleMask, fullUid, C.span, C.g.EY, C.g.EX,
                                                                       nC, Fi.g.EY, Fi.g.EX, nCh, Ech, C.ldk);
             TG_LAUNCH_CHECK(id);
-            // ldk is a multiple of 64: 64 elements per wavefront, 256 per workgroup; entry tiles shared out until
-            // there are four wavefronts for each of the 1024 SIMDs
-            const int tiles = (int)std::max<int64_t>(1, std::min<int64_t>(36, 36 * (C.ldk / 64) / 4096));
+            const int tiles = l2_tiles(C.ldk);
             const dim3 gg(grid_for(C.ldk, 256), grid_for(36, tiles));
             if (nCh == 64) k_galerkin_l2_mfma<16, 4><<<gg, 256, 0, st>>>(Ech, Gl2, C.Ks64, C.ldk, tiles);
             else if (nCh == 8) k_galerkin_l2_mfma<2, 4><<<gg, 256, 0, st>>>(Ech, Gl2, C.Ks64, C.ldk, tiles);
             else fail(TG_ERR_ARGS, id, "level-2 Galerkin: %d children per coarse element", nCh);
             TG_LAUNCH_CHECK(id);
             if (nBnd)
-                k_galerkin_bnd<<<(unsigned)nBnd, 64 * GB_WAVES, 0, st>>>(bndList, bndPtr, (const BndChild *)bndChild.p, E64,
+                k_galerkin_bnd<false><<<(unsigned)nBnd, 64 * GB_WAVES, 0, st>>>(bndList, bndPtr, (const BndChild *)bndChild.p, E64,
                                                                         uFree, uFixed, C.P, C.Ks64, C.ldk);
-        } else if (i == 1) {
-            SrcDevSuper src;
-            static_cast<ChildGrid &>(src) = cg;
-            src.Kmat = F.Ks64; src.ldk = F.ldk; src.Esub = Esub; src.uf = uFree; src.ux = uFixed; src.uid = fullUid;
-            k_galerkin_dev<<<grid, GK_THREADS, 0, st>>>(src, C.eleMask, nCh, C.P, C.Ks64, C.ldk);
         } else {
-            if (nCh != 8) fail(TG_ERR_ARGS, id, "Galerkin level %d: %d children per coarse element", i + 1, nCh);
-            k_galerkin_half<<<dim3(grid_for(C.g.elems(), 16), 6), 256, 0, st>>>(Fi.Ks64, Fi.ldk, C.g.EY, C.g.EX, C.g.elems(),
-                                                                            Fi.g.EY, Fi.g.EX, C.P, C.Ks64, C.ldk);
+            // four wavefronts take per children each; super-element level 2 (64 children) in slices of them until
+            // there are two workgroups per CU
+            const int64_t nC = C.g.elems();
+            const unsigned groups = grid_for(nC, 16);
+            int slices = 1;
+            while (nCh == 64 && slices < 16 && (int64_t)groups * 6 * slices < 512) slices *= 2;
+            double *out = C.Ks64.p;
+            if (slices > 1) {
+                if (Gpart.n < (size_t)slices * 576 * C.ldk) Gpart.alloc((size_t)slices * 576 * C.ldk);
+                out = Gpart.p;
+            }
+            const int32_t *skip = i == 1 ? fullUid.p : nullptr;
+            const dim3 gg(groups, 6, slices);
+            if (nCh == 64)
+                k_galerkin_children<4><<<gg, 256, 0, st>>>(Fi.Ks64, Fi.ldk, skip, C.g.EY, C.g.EX, nC, Fi.g.EY, Fi.g.EX, C.P,
+                                                           16 / slices, out, C.ldk);
+            else if (nCh == 8)
+                k_galerkin_children<2><<<gg, 256, 0, st>>>(Fi.Ks64, Fi.ldk, skip, C.g.EY, C.g.EX, nC, Fi.g.EY, Fi.g.EX, C.P, 2,
+                                                           out, C.ldk);
+            else fail(TG_ERR_ARGS, id, "Galerkin level %d: %d children per coarse element", i + 1, nCh);
+            TG_LAUNCH_CHECK(id);
+            if (slices > 1)
+                k_sum_slices<<<grid_for(576 * C.ldk, 256), 256, 0, st>>>(Gpart, slices, C.ldk, nC, C.Ks64);
+            if (i == 1 && nBnd)
+                k_galerkin_bnd<true><<<(unsigned)nBnd, 64 * GB_WAVES, 0, st>>>(bndList, bndPtr, (const BndChild *)bndChild.p,
+                                                                              Esub, uFree, uFixed, C.P, C.Ks64, C.ldk);
         }
         TG_LAUNCH_CHECK(id);
     }
