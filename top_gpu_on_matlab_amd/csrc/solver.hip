@@ -61,7 +61,6 @@ __global__ __launch_bounds__(64 * GB_WAVES) void k_galerkin_bnd(const int64_t *_
             double v = 0.0;
             if (SUPER && on) {
                 const double *u = uf + (size_t)ch.uid * (576 * 64) + 64 * k + lane, *es = E + (size_t)ch.fine * 64;
-#pragma unroll 16
                 for (int q = 0; q < 64; ++q) v += u[(size_t)q * 576] * es[q];
                 v += ux[i];
             } else if (on) {
