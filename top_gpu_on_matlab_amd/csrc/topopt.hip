@@ -18,12 +18,9 @@
 namespace tg {
 namespace {
 
-// ce_e = u_e' * K * u_e, K = Ke (MODE 0) or the element's K_mat (MODE 1, entry-major).
-// u is a full-grid interleaved vector; output in solid-element order.
-template <int MODE>
+// ce_e = u_e' * Ke * u_e; u is a full-grid interleaved vector; output in solid-element order.
 __global__ void k_unit_compliance(const double *__restrict__ u, const double *__restrict__ K0,
-                                  const double *__restrict__ Km, int64_t ldk, const int32_t *__restrict__ eleFull0,
-                                  int64_t Ne, const Grid g, double *__restrict__ ce) {
+                                  const int32_t *__restrict__ eleFull0, int64_t Ne, const Grid g, double *__restrict__ ce) {
     const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (k >= Ne) return;
     const int64_t e = eleFull0[k];
@@ -40,24 +37,25 @@ __global__ void k_unit_compliance(const double *__restrict__ u, const double *__
     for (int j = 0; j < 24; ++j) {
         double kj = 0;
 #pragma unroll
-        for (int i = 0; i < 24; ++i) {
-            if (MODE == 0) kj += ue[i] * K0[i + 24 * j];       // (u_e' * Ke)_j
-            else kj += Km[(int64_t)(j + 24 * i) * ldk + e] * ue[i];  // (K_mat_e * u_e)_j
-        }
+        for (int i = 0; i < 24; ++i) kj += ue[i] * K0[i + 24 * j];  // (u_e' * Ke)_j
         s += kj * ue[j];
     }
     ce[k] = s;
 }
 
-// dc(q, e) = u_e' * I_q * u_e
-__global__ void k_subvoxel_energy(const double *__restrict__ u, const double *__restrict__ Imat,
-                                  const int32_t *__restrict__ eleFull0, int64_t Ne, const Grid g,
-                                  double *__restrict__ dc) {
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= Ne * 64) return;
-    const int64_t k = t / 64;
-    const int q = (int)(t % 64);
-    const int64_t e = eleFull0[k];
+// Super-element mode: ce_e = u_e' K_mat_e u_e, K_mat entry-major.  Eight threads per element, three columns each,
+// their sums added in column order: consecutive threads read consecutive elements' entries, and a chain of
+// 72 loads replaces one of 576 (160 us at 6,000 elements with a thread per element, 46 this way).
+constexpr int UC_PARTS = 8, UC_ELEMS = 32;
+__global__ __launch_bounds__(UC_PARTS * UC_ELEMS) void k_unit_compliance_super(const double *__restrict__ u,
+                                                                               const double *__restrict__ Km, int64_t ldk,
+                                                                               const int32_t *__restrict__ eleFull0,
+                                                                               int64_t Ne, const Grid g,
+                                                                               double *__restrict__ ce) {
+    __shared__ double part[UC_PARTS][UC_ELEMS];
+    const int el = threadIdx.x % UC_ELEMS, p = threadIdx.x / UC_ELEMS;
+    const int64_t k = (int64_t)blockIdx.x * UC_ELEMS + el;
+    const int64_t e = eleFull0[k < Ne ? k : Ne - 1];
     const int ey = (int)(e % g.EY), ex = (int)((e / g.EY) % g.EX), ez = (int)(e / ((int64_t)g.EY * g.EX));
     double ue[24];
 #pragma unroll
@@ -67,14 +65,80 @@ __global__ void k_subvoxel_energy(const double *__restrict__ u, const double *__
         ue[3 * b + 1] = u[3 * m + 1];
         ue[3 * b + 2] = u[3 * m + 2];
     }
-    const double *I = Imat + (size_t)576 * q;
     double s = 0;
-    for (int i = 0; i < 24; ++i) {
-        double ki = 0;
-        for (int j = 0; j < 24; ++j) ki += I[i + 24 * j] * ue[j];
-        s += ki * ue[i];
+#pragma unroll
+    for (int b = 0; b < UC_PARTS; ++b)  // (static indices into ue)
+        if (p == b)
+#pragma unroll
+            for (int j = 3 * b; j < 3 * b + 3; ++j) {
+                double kj = 0;
+#pragma unroll
+                for (int i = 0; i < 24; ++i) kj += Km[(int64_t)(j + 24 * i) * ldk + e] * ue[i];  // (K_mat_e u_e)_j
+                s += kj * ue[j];
+            }
+    part[p][el] = s;
+    __syncthreads();
+    if (p == 0 && k < Ne) {
+        for (int b = 1; b < UC_PARTS; ++b) s += part[b][el];
+        ce[k] = s;
     }
-    dc[q + 64 * k] = s;
+}
+
+// dc(q, e) = u_e' I_q u_e = sum over i <= j of (I_q(i, j) + I_q(j, i)) u_i u_j (half of it for i = j): a product of
+// the 64 x 300 sub-voxel coefficients with the element's 300 products u_i u_j, on the matrix cores (f64 16x16x4:
+// 16 sub-voxels x 4 products x 16 elements; layouts as in the solver's Galerkin product).  A wavefront has 16
+// elements, their displacements in LDS, and forms its products as it goes; the four wavefronts of a workgroup
+// take a quarter of the products each and add up in wavefront order.  Sub-voxel tiles are stored element by
+// element.  330 us at 6,000 elements with a thread per element and sub-voxel, 47 here.
+typedef double tg_tdbl4 __attribute__((ext_vector_type(4)));
+__global__ __launch_bounds__(256) void k_subvoxel_energy(const double *__restrict__ u, const double *__restrict__ Imat,
+                                                         const int32_t *__restrict__ eleFull0, int64_t Ne, const Grid g,
+                                                         double *__restrict__ dc) {
+    __shared__ double su[24][17];
+    __shared__ double red[4][16][65];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, li = lane & 15, lk = lane >> 4;
+    const int64_t k0 = (int64_t)blockIdx.x * 16;
+    for (int i = threadIdx.x; i < 128; i += 256) {  // one vertex of one element
+        const int el = i & 15, b = i >> 4;
+        const int64_t e = eleFull0[k0 + el < Ne ? k0 + el : Ne - 1];
+        const int ey = (int)(e % g.EY), ex = (int)((e / g.EY) % g.EX), ez = (int)(e / ((int64_t)g.EY * g.EX));
+        const int64_t m = (ey + vtx_y(b)) + (int64_t)g.NY * ((ex + vtx_x(b)) + (int64_t)g.NX * (ez + vtx_z(b)));
+        for (int c = 0; c < 3; ++c) su[3 * b + c][el] = u[3 * m + c];
+    }
+    __syncthreads();
+    tg_tdbl4 acc[4];
+#pragma unroll
+    for (int t = 0; t < 4; ++t) acc[t] = tg_tdbl4{0.0, 0.0, 0.0, 0.0};
+    // products 4 kk + lk of the packed upper triangle, p = i + j (j + 1) / 2; 75 groups of four
+    const int kk0 = w * 19, kk1 = min(kk0 + 19, 75);
+    int p = 4 * kk0 + lk, j = (int)((sqrtf(8.0f * (float)p + 1.0f) - 1.0f) * 0.5f);
+    if (ksym_index(0, j) > p) --j;
+    if (ksym_index(0, j + 1) <= p) ++j;
+    int i = p - ksym_index(0, j);
+    for (int kk = kk0; kk < kk1; ++kk) {
+        const double b = su[i][li] * su[j][li];
+        double a[4];
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            const double *I = Imat + (size_t)576 * (16 * t + li);
+            a[t] = i == j ? I[25 * i] : I[i + 24 * j] + I[j + 24 * i];
+        }
+#pragma unroll
+        for (int t = 0; t < 4; ++t) acc[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[t], b, acc[t], 0, 0, 0);
+        for (i += 4; i > j; ++j) i -= j + 1;
+    }
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) red[w][li][16 * t + 4 * r + lk] = acc[t][r];
+    __syncthreads();
+    for (int idx = threadIdx.x; idx < 1024; idx += 256) {
+        const int el = idx >> 6, q = idx & 63;
+        if (k0 + el >= Ne) continue;
+        double s = red[0][el][q];
+        for (int v = 1; v < 4; ++v) s += red[v][el][q];
+        dc[64 * (k0 + el) + q] = s;
+    }
 }
 
 __global__ void k_simp(const double *__restrict__ x, double *__restrict__ E, int64_t n, double Emin, double E0,
@@ -590,9 +654,9 @@ int tg_solver_unit_compliance(tg_solver *s, const double *d_U, double *d_ce) {
         k_unpack<double, double><<<grid_for(F.Nn, 256), 256, 0, S.st>>>(d_U, S.pw.z, F.nodFull0, F.Nn);
         if (S.super) {
             if (!S.assembled) fail(TG_ERR_STATE, "tg_solver_unit_compliance:State", "assemble first (K_mat)");
-            k_unit_compliance<1><<<grid_for(F.Ne, 256), 256, 0, S.st>>>(S.pw.z, nullptr, F.Ks64, F.ldk, F.eleFull0, F.Ne, F.g, d_ce);
+            k_unit_compliance_super<<<grid_for(F.Ne, UC_ELEMS), UC_PARTS * UC_ELEMS, 0, S.st>>>(S.pw.z, F.Ks64, F.ldk, F.eleFull0, F.Ne, F.g, d_ce);
         } else {
-            k_unit_compliance<0><<<grid_for(F.Ne, 256), 256, 0, S.st>>>(S.pw.z, S.K0_64, nullptr, 0, F.eleFull0, F.Ne, F.g, d_ce);
+            k_unit_compliance<<<grid_for(F.Ne, 256), 256, 0, S.st>>>(S.pw.z, S.K0_64, F.eleFull0, F.Ne, F.g, d_ce);
         }
         TG_LAUNCH_CHECK(id);
         TG_HIP(hipStreamSynchronize(S.st), id);
@@ -641,7 +705,7 @@ int tg_compliance_grad(tg_solver *s, tg_filter *f, const double *d_x, double Emi
         DevLevel &F = S.lv[0];
         S.pw.z.zero(st);
         k_unpack<double, double><<<grid_for(F.Nn, 256), 256, 0, st>>>(d_U, S.pw.z, F.nodFull0, F.Nn);
-        k_unit_compliance<0><<<grid_for(Ne, 256), 256, 0, st>>>(S.pw.z, S.K0_64, nullptr, 0, F.eleFull0, Ne, F.g, S.adjCe);
+        k_unit_compliance<<<grid_for(Ne, 256), 256, 0, st>>>(S.pw.z, S.K0_64, F.eleFull0, Ne, F.g, S.adjCe);
         TG_LAUNCH_CHECK(id);
         double *h = nullptr;
         TG_HIP(hipHostMalloc((void **)&h, sizeof(double), hipHostMallocDefault), id);
@@ -675,7 +739,7 @@ int tg_solver_subvoxel_energy(tg_solver *s, const double *d_U, double *d_dc) {
         DevLevel &F = S.lv[0];
         S.pw.z.zero(S.st);
         k_unpack<double, double><<<grid_for(F.Nn, 256), 256, 0, S.st>>>(d_U, S.pw.z, F.nodFull0, F.Nn);
-        k_subvoxel_energy<<<grid_for(F.Ne * 64, 256), 256, 0, S.st>>>(S.pw.z, S.Imat, F.eleFull0, F.Ne, F.g, d_dc);
+        k_subvoxel_energy<<<grid_for(F.Ne, 16), 256, 0, S.st>>>(S.pw.z, S.Imat, F.eleFull0, F.Ne, F.g, d_dc);
         TG_LAUNCH_CHECK(id);
         TG_HIP(hipStreamSynchronize(S.st), id);
     });
