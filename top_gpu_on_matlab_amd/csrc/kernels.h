@@ -324,6 +324,86 @@ __global__ __launch_bounds__(256) void k_kelem_gather(const T *__restrict__ f, i
     }
 }
 
+// The packed matrices' product, gather and epilogue in one launch, for small grids: a workgroup has 64 consecutive
+// nodes (plane by plane, y fastest), wavefront o the element of every node at octant o, whose three rows of
+// K_e it forms (24 products each, in k_kelem_sym's order: the same bits); the eight contributions meet in LDS and
+// are added in k_kelem_gather's order.  Every stored entry is read for both of its rows, twice the traffic of
+// the two launches, but the chain is one of 72 loads and one launch instead of 300 and two.  Product at level 2 in
+// FP64 (FP32), us: 432 elements 7.6 (6.6) against 16.3 (11.5), 8,192 8.3 (7.0) against 16.9 (12.0), 12,800 11.5 (7.3)
+// against 17.6 (12.2), 20,736 19.6 (12.3) against 18.3 (13.4), 65,536 53 (31) against 32 (20); super-element
+// finest level, 16,384: 9.2 against 18.0.  So up to 16,384 elements.
+// EPI_RESID_JAC0: the operand is x = omega r ./ diag, formed as it is loaded and written to xout (a launch fewer).
+constexpr int KN_NODES = 64;
+template <typename T, int EPI, bool MASKED>
+__global__ __launch_bounds__(8 * KN_NODES) void k_kelem_node(const T *__restrict__ u, T *__restrict__ out,
+                                                             const T *__restrict__ Kp, int64_t ldk,
+                                                             const uint8_t *__restrict__ eleMask,
+                                                             const uint8_t *__restrict__ mask, const Grid g,
+                                                             const T *__restrict__ r, const T *__restrict__ diag, T omega,
+                                                             T *__restrict__ xout) {
+    constexpr bool J0 = EPI == EPI_RESID_JAC0;
+    __shared__ T sf[8][3][KN_NODES];
+    __shared__ uint8_t sOn[8][KN_NODES];
+    const int lane = threadIdx.x & 63, o = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int64_t n = (int64_t)blockIdx.x * KN_NODES + lane;
+    const int oz = (o >> 2) - 1, ox = ((o >> 1) & 1) - 1, oy = (o & 1) - 1;  // the gather's order: z, x, y
+    const int iy = (int)(n % g.NY);
+    const int64_t t = n / g.NY;
+    const int ix = (int)(t % g.NX), iz = (int)(t / g.NX);
+    const int ey = iy + oy, ex = ix + ox, ez = iz + oz;
+    const bool in = n < g.nodes() && (unsigned)ey < (unsigned)g.EY && (unsigned)ex < (unsigned)g.EX &&
+                    (unsigned)ez < (unsigned)g.EZ;
+    const int64_t e = in ? ey + (int64_t)g.EY * (ex + (int64_t)g.EX * ez) : 0;
+    const bool on = in && eleMask[e];
+    if (on) {
+        T ue[24];
+#pragma unroll
+        for (int b = 0; b < 8; ++b) {
+            const int64_t m = (ey + vtx_y(b)) + (int64_t)g.NY * ((ex + vtx_x(b)) + (int64_t)g.NX * (ez + vtx_z(b)));
+            const uint8_t mm = MASKED ? mask[m] : (uint8_t)0;
+#pragma unroll
+            for (int d = 0; d < 3; ++d) {
+                const T v = J0 ? omega * (r[3 * m + d] / diag[3 * m + d]) : u[3 * m + d];
+                ue[3 * b + d] = (mm & (1 << d)) ? (T)0 : v;
+            }
+        }
+        const int a = vtx_of(-oy, -ox, -oz);
+        const T *K = Kp + e;
+        T f[3] = {0, 0, 0};
+#pragma unroll
+        for (int i = 0; i < 24; ++i)
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+                const int row = 3 * a + c;
+                f[c] += K[(int64_t)(i <= row ? ksym_index(i, row) : ksym_index(row, i)) * ldk] * ue[i];
+            }
+#pragma unroll
+        for (int c = 0; c < 3; ++c) sf[o][c][lane] = f[c];
+    }
+    sOn[o][lane] = on;
+    __syncthreads();
+    if (o >= 3 || n >= g.nodes()) return;
+    const int c = o;  // wavefronts 0..2: one component each
+    const uint8_t mk = mask[n];
+    const int64_t k = 3 * n + c;
+    if (!(mk & NODE_ACTIVE)) {
+        out[k] = 0;
+        if (J0) xout[k] = 0;
+        return;
+    }
+    T v = 0;
+#pragma unroll
+    for (int q = 0; q < 8; ++q)
+        if (sOn[q][lane]) v += sf[q][c][lane];
+    const T rk = EPI == EPI_KU ? (T)0 : r[k], dk = J0 || EPI == EPI_JACOBI ? diag[k] : (T)1;
+    const T uk = J0 ? omega * (rk / dk) : (MASKED || EPI == EPI_JACOBI ? u[k] : (T)0);
+    if (MASKED && (mk & (1 << c))) v = uk;
+    if (J0) xout[k] = uk;
+    if (EPI == EPI_RESID || J0) v = rk - v;
+    if (EPI == EPI_JACOBI) v = uk + (omega * (rk - v)) / dk;
+    out[k] = v;
+}
+
 // Trilinear weight of coarse vertex j at fine offset (a, b, c) of a span-S block; exact in binary.
 template <typename T, int S>
 __device__ inline T ri_w(int a, int b, int c, int j) {

@@ -84,6 +84,13 @@ struct Solver {
         return ktiles_for(lv[0].g, kfine_zchunk ? kfine_zchunk : kfine_auto[f64 || kfine_mfma ? 0 : 1]);
     }
     bool fine_tiled() const { return !super && kfine_kernel == 0 && walsh_ok; }
+    // Element-matrix products small enough for the one-launch form (k_kelem_node).
+    int64_t node_elems = 1 << 14;
+    bool elem_one_launch(const DevLevel &D) const { return D.ldk <= node_elems; }
+    template <typename T>
+    bool jac0_one_launch(const DevLevel &D) const {  // ... and with the packed matrices that it needs
+        return elem_one_launch(D) && (sizeof(T) == 4 || (kelem_parts == 1 && D.Ks64p.n));
+    }
     template <typename T>
     // pk (optional): also write the coarsest level's plane-order copy for its persistent solve
     void restrict_level(int c, const T *rf, T *rc, const PlanePack *pk = nullptr);

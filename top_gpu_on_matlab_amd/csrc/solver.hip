@@ -809,6 +809,20 @@ bool Solver::kbyu_level(int i, const T *u, T *out, int epi, const T *rr, const T
         // matrices is asked for; FP32: always packed
         const bool packed = !f64 || (kelem_parts == 1 && D.Ks64p.n);
         const T *Km = f64 ? (const T *)(packed ? D.Ks64p.p : D.Ks64.p) : (const T *)D.Ks32.p;
+        if (packed && elem_one_launch(D)) {
+            const unsigned gn = grid_for(D.g.nodes(), KN_NODES);
+#define TG_NODE_CASE(EPI)                                                                                        \
+    case EPI:                                                                                                    \
+        if (i == 0) k_kelem_node<T, EPI, true><<<gn, 8 * KN_NODES, 0, st>>>(u, out, Km, D.ldk, D.eleMask, D.nodeMask, D.g, rr, dg, w, xout); \
+        else k_kelem_node<T, EPI, false><<<gn, 8 * KN_NODES, 0, st>>>(u, out, Km, D.ldk, D.eleMask, D.nodeMask, D.g, rr, dg, w, xout); \
+        break;
+            switch (epi) {
+                TG_NODE_CASE(EPI_KU) TG_NODE_CASE(EPI_RESID) TG_NODE_CASE(EPI_JACOBI) TG_NODE_CASE(EPI_RESID_JAC0)
+            }
+#undef TG_NODE_CASE
+            TG_LAUNCH_CHECK("tg_solver:kbyu");
+            return false;
+        }
         T *fv = f64 ? (T *)D.fv64.p : (T *)D.fv32.p;
         const unsigned gs = grid_for(D.g.elems(), 256);
         const dim3 grp = gather_grid(D.g);
@@ -885,11 +899,11 @@ void Solver::vcycle_t(const T *r0, T *z0) {
         const PlanePack *pki = (packed && i + 1 == L - 1) ? &pk : nullptr;
         DevLevel &D = lv[i];
         const int64_t nv = 3 * D.g.nodes();
-        if (i == 0 && !adapted && fine_tiled()) {
+        if (!adapted && (i == 0 && !super ? fine_tiled() : jac0_one_launch<T>(D))) {
             // pre-smoothing x = omega r ./ diag fused into the residual product
             T *d = vec<T>(D, 2);
-            kbyu_level<T>(0, nullptr, d, EPI_RESID_JAC0, rr[0], diag_of<T>(D), -1, xx[0]);
-            restrict_level<T>(1, d, (T *)rr[1], pki);
+            kbyu_level<T>(i, nullptr, d, EPI_RESID_JAC0, rr[i], diag_of<T>(D), -1, xx[i]);
+            restrict_level<T>(i + 1, d, (T *)rr[i + 1], pki);
             continue;
         }
         k_jacobi0<T><<<grid_for(nv, 256), 256, 0, st>>>(rr[i], diag_of<T>(D), xx[i], w, nv);
