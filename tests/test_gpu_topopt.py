@@ -129,6 +129,42 @@ def test_oc_update_matches_bisection():
     assert abs(change - np.max(np.abs(xnew - x))) < 1e-15
 
 
+@pytest.mark.parametrize('n', [1, 255, 257, 40000, 200001])
+@pytest.mark.parametrize('passive, scale', [(False, 1e-2), (True, 1e-2), (True, 1e6), (False, 1e-12)])
+def test_oc_update_step_by_step(n, passive, scale):
+    """The bisection of several steps per launch against one step at a time: the same multiplier (so the update
+    to rounding), the same step count (rounded up to 16), with passive entries, multipliers from small to
+    large, and the result written over an input."""
+    import ctypes
+    from top_gpu_on_matlab_amd._lib import check, lib
+    rng = np.random.default_rng(n)
+    x = rng.random(n)
+    dc = -rng.random(n) * scale
+    dv = 0.5 + rng.random(n)
+    pas = (rng.random(n) < 0.1).astype(float) if passive else None
+    fval = -0.02
+    l1, l2, move, steps = 0.0, 1e9, 0.2, 0
+    while (l2 - l1) / (l1 + l2) > 1e-6:
+        lmid = 0.5 * (l2 + l1)
+        xnew = np.maximum(0, np.maximum(x - move, np.minimum(1, np.minimum(x + move, x * np.sqrt(-dc / dv / lmid)))))
+        if passive:
+            xnew[pas != 0] = 1.0
+        steps += 1
+        if fval + np.mean(xnew - x) > 0:
+            l1 = lmid
+        else:
+            l2 = lmid
+    d = {k: _t(v) for k, v in dict(x=x, dc=dc, dv=dv, pas=pas if passive else x, out=np.zeros(n)).items()}
+    ptr = lambda k: ctypes.c_void_p(d[k].data_ptr())
+    for out in ('out', 'dv'):
+        change, took = ctypes.c_double(), ctypes.c_int32()
+        check(lib().tg_oc_update(ptr('x'), ptr('dc'), ptr('dv'), ptr('pas') if passive else None, n, fval, move, ptr(out),
+                                 ctypes.byref(change), ctypes.byref(took), None))
+        assert _rel(d[out].cpu().numpy(), xnew) < 1e-14
+        assert abs(change.value - np.max(np.abs(xnew - x))) < 1e-15
+        assert took.value == 16 * -(-steps // 16)
+
+
 @pytest.mark.parametrize('cfg', [
     dict(shape=(8, 16, 8), case=1, ft=1, nLoop=6, se=False),
     dict(shape=(8, 16, 8), case=1, ft=2, nLoop=6, se=False),
