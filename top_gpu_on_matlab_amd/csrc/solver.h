@@ -107,7 +107,7 @@ struct Solver {
     const double *r64_dot = nullptr;  // mixed: the FP32 finest post-smoothing reduces z.r against this FP64 r
     DevBuf<double> dotp;   // per-workgroup partial sums of the fused dots
     // compliance-gradient work space (tg_compliance_grad)
-    DevBuf<double> adjF, adjXp, adjE, adjCe, adjG, adjPart, adjRes;
+    DevBuf<double> adjF, adjXp, adjE, adjCe, adjG;
     void pcg(const double *b_c, double *y_c, double tol, int maxIT, int warm, int *its, double *res);
 };
 

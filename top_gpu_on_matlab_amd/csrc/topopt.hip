@@ -9,6 +9,8 @@
 //   convolution filter  imfilter density filter of super-element mode, TOP_GPU.m:112-121, 220-227, 262-265
 #include <cmath>
 #include <cstring>
+#include <memory>
+#include <mutex>
 
 #include "kernels.h"
 #include "model.h"
@@ -206,9 +208,11 @@ __global__ __launch_bounds__(RED_THREADS) void k_red_partial(const double *__res
     if (threadIdx.x == 0) partial[blockIdx.x] = sh[0];
 }
 
+// host, seq: the result in pinned host memory, and the number published after it (Scratch::wait)
 template <int OP>
 __global__ __launch_bounds__(RED_THREADS) void k_red_final(const double *__restrict__ partial, int nb,
-                                                           double *__restrict__ out) {
+                                                           double *__restrict__ host, unsigned long long *seq_ptr,
+                                                           unsigned long long seq) {
     __shared__ double sh[RED_THREADS];
     double s = 0;
     for (int i = threadIdx.x; i < nb; i += blockDim.x) s = OP == R_MAXABSDIFF ? fmax(s, partial[i]) : s + partial[i];
@@ -219,7 +223,10 @@ __global__ __launch_bounds__(RED_THREADS) void k_red_final(const double *__restr
                                                                       : sh[threadIdx.x] + sh[threadIdx.x + w];
         __syncthreads();
     }
-    if (threadIdx.x == 0) *out = sh[0];
+    if (threadIdx.x == 0) {
+        *host = sh[0];
+        __hip_atomic_store(seq_ptr, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
 }
 
 // ---- optimality criteria ---------------------------------------------------------------------
@@ -334,7 +341,8 @@ __global__ __launch_bounds__(RED_THREADS) void k_oc_pass(const double *__restric
 // The state after the last pass, for the host's check (and the apply's midpoint).
 __global__ __launch_bounds__(RED_THREADS) void k_oc_close(int64_t n, double fval, const OcState *__restrict__ old,
                                                           OcState *__restrict__ now, const double *__restrict__ partial,
-                                                          int nb) {
+                                                          int nb, double *__restrict__ host, unsigned long long *seq_ptr,
+                                                          unsigned long long seq) {
     __shared__ double sums[OC_NODES];
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     for (int k = w; k < OC_NODES; k += RED_THREADS / 64) {
@@ -344,7 +352,12 @@ __global__ __launch_bounds__(RED_THREADS) void k_oc_close(int64_t n, double fval
         if (lane == 0) sums[k] = s;
     }
     __syncthreads();
-    if (threadIdx.x == 0) *now = oc_walk(*old, sums, fval, (double)n);
+    if (threadIdx.x == 0) {
+        const OcState s = oc_walk(*old, sums, fval, (double)n);
+        *now = s;
+        *(OcState *)host = s;
+        __hip_atomic_store(seq_ptr, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
 }
 
 // xnew, and each workgroup's max |xnew - x|
@@ -610,21 +623,107 @@ __global__ void k_conv_any(const double *__restrict__ in, const double *__restri
 }  // namespace
 
 // ---------------------------------------------------------------------------------------------
-double reduce_dev(int op, const double *a, const double *b, int64_t n, DevBuf<double> &partial, DevBuf<double> &res,
-                  double *h, hipStream_t st) {
-    const char *id = "tg_reduce:Input";
-    switch (op) {
-        case R_SUM: k_red_partial<R_SUM><<<RED_BLOCKS, RED_THREADS, 0, st>>>(a, b, n, partial); k_red_final<R_SUM><<<1, RED_THREADS, 0, st>>>(partial, RED_BLOCKS, res); break;
-        case R_DOT: k_red_partial<R_DOT><<<RED_BLOCKS, RED_THREADS, 0, st>>>(a, b, n, partial); k_red_final<R_DOT><<<1, RED_THREADS, 0, st>>>(partial, RED_BLOCKS, res); break;
-        case R_MAXABSDIFF: k_red_partial<R_MAXABSDIFF><<<RED_BLOCKS, RED_THREADS, 0, st>>>(a, b, n, partial); k_red_final<R_MAXABSDIFF><<<1, RED_THREADS, 0, st>>>(partial, RED_BLOCKS, res); break;
-        case R_SHARP: k_red_partial<R_SHARP><<<RED_BLOCKS, RED_THREADS, 0, st>>>(a, b, n, partial); k_red_final<R_SHARP><<<1, RED_THREADS, 0, st>>>(partial, RED_BLOCKS, res); break;
-        default: fail(TG_ERR_ARGS, id, "unknown reduction %d", op);
+namespace {
+
+// Working memory of the calls that have no object of their own (reductions, the OC update): device scratch and a
+// few pinned values that the last kernel writes and then publishes, so a call neither allocates (hipMalloc,
+// hipHostMalloc and their frees took 0.2 to 0.4 ms a call) nor copies.  Blocks are lent for one call, each to one
+// caller at a time, and come back once the host has seen the result, when nothing of theirs runs any more; at
+// most SCRATCH_KEPT idle ones per device are kept, the rest are freed.
+constexpr size_t SCRATCH_DOUBLES = (size_t)2 * OC_NODES * OC_BLOCKS + RED_BLOCKS + 16;
+constexpr size_t SCRATCH_KEPT = 4;
+struct ScratchBlock {
+    DevBuf<double> dev{SCRATCH_DOUBLES};
+    double *host = nullptr, *mapped = nullptr;  // 16 doubles, then the published number; their device address
+    unsigned long long seq = 0;
+    ScratchBlock() {
+        TG_HIP(hipHostMalloc((void **)&host, 17 * sizeof(double), hipHostMallocMapped | hipHostMallocCoherent), "topgpu:alloc");
+        *(unsigned long long *)(host + 16) = 0ull;
+        if (hipHostGetDevicePointer((void **)&mapped, host, 0) != hipSuccess) {
+            (void)hipHostFree(host);
+            fail(TG_ERR_HIP, "topgpu:alloc", "pinned memory is not mapped");
+        }
     }
-    TG_LAUNCH_CHECK(id);
-    TG_HIP(hipMemcpyAsync(h, res.p, sizeof(double), hipMemcpyDeviceToHost, st), id);
-    TG_HIP(hipStreamSynchronize(st), id);
-    return *h;
+    ~ScratchBlock() { (void)hipHostFree(host); }
+};
+struct ScratchPool {
+    std::mutex mu;
+    std::vector<std::unique_ptr<ScratchBlock>> idle[64];
+};
+ScratchPool &scratch_pool() {
+    static ScratchPool *p = new ScratchPool;  // not destroyed: the runtime may be gone before it at exit
+    return *p;
 }
+class Scratch {
+    hipStream_t st;
+    int dev = 0;
+    std::unique_ptr<ScratchBlock> b;
+    bool busy = false;  // work may be in flight that the host has not seen the end of
+
+  public:
+    explicit Scratch(hipStream_t s) : st(s) {
+        TG_HIP(hipGetDevice(&dev), "topgpu:alloc");
+        if (dev < 0 || dev >= 64) fail(TG_ERR_HIP, "topgpu:alloc", "device ordinal %d out of range", dev);
+        {
+            ScratchPool &p = scratch_pool();
+            std::lock_guard<std::mutex> lock(p.mu);
+            if (!p.idle[dev].empty()) {
+                b = std::move(p.idle[dev].back());
+                p.idle[dev].pop_back();
+            }
+        }
+        if (!b) b.reset(new ScratchBlock);
+        busy = true;
+    }
+    ~Scratch() {
+        if (busy) (void)hipStreamSynchronize(st);
+        ScratchPool &p = scratch_pool();
+        std::lock_guard<std::mutex> lock(p.mu);
+        if (p.idle[dev].size() < SCRATCH_KEPT) p.idle[dev].push_back(std::move(b));
+    }
+    double *dbl() const { return b->dev.p; }
+    double *host() const { return b->mapped; }                                              // device address
+    unsigned long long *seq_ptr() const { return (unsigned long long *)(b->mapped + 16); }  // device address
+    unsigned long long next() {
+        busy = true;
+        return ++b->seq;
+    }
+    // The values once the last kernel has published them.  The stream is queried now and then, so a device
+    // error, or a stream that finished without publishing, ends the wait.
+    const double *wait(const char *id) {
+        unsigned long long *hs = (unsigned long long *)(b->host + 16);
+        for (unsigned spins = 1; __atomic_load_n(hs, __ATOMIC_ACQUIRE) != b->seq; ++spins)
+            if ((spins & 4095) == 0) {
+                const hipError_t e = hipStreamQuery(st);
+                if (e != hipErrorNotReady) {
+                    TG_HIP(e, id);
+                    if (__atomic_load_n(hs, __ATOMIC_ACQUIRE) != b->seq) fail(TG_ERR_HIP, id, "result not published by a finished stream");
+                }
+            }
+        busy = false;
+        return b->host;
+    }
+};
+
+// Sum, dot, maximum or sharpness of device arrays on st, to the host.
+double reduce_dev(int op, const double *a, const double *b, int64_t n, hipStream_t st) {
+    const char *id = "tg_reduce:Input";
+    if (op != R_SUM && op != R_DOT && op != R_MAXABSDIFF && op != R_SHARP) fail(TG_ERR_ARGS, id, "unknown reduction %d", op);
+    Scratch sc(st);
+    double *part = sc.dbl();
+    const unsigned long long seq = sc.next();
+#define TG_RED_CASE(OP)                                                                                   \
+    case OP:                                                                                              \
+        k_red_partial<OP><<<RED_BLOCKS, RED_THREADS, 0, st>>>(a, b, n, part);                             \
+        k_red_final<OP><<<1, RED_THREADS, 0, st>>>(part, RED_BLOCKS, sc.host(), sc.seq_ptr(), seq);       \
+        break;
+    switch (op) { TG_RED_CASE(R_SUM) TG_RED_CASE(R_DOT) TG_RED_CASE(R_MAXABSDIFF) TG_RED_CASE(R_SHARP) }
+#undef TG_RED_CASE
+    TG_LAUNCH_CHECK(id);
+    return *sc.wait(id);
+}
+
+}  // namespace
 
 Filter::Filter(const tg_model &mm, double rMin, hipStream_t s) : m(mm), st(s) {
     const char *id = "tg_filter_create:Input";
@@ -776,8 +875,6 @@ int tg_compliance_grad(tg_solver *s, tg_filter *f, const double *d_x, double Emi
             S.adjE.alloc(Ne);
             S.adjCe.alloc(Ne);
             S.adjG.alloc(Ne);
-            S.adjPart.alloc(RED_BLOCKS);
-            S.adjRes.alloc(1);
         }
         int fits = 0;
         double fres = 0;
@@ -803,15 +900,7 @@ int tg_compliance_grad(tg_solver *s, tg_filter *f, const double *d_x, double Emi
         k_unpack<double, double><<<grid_for(F.Nn, 256), 256, 0, st>>>(d_U, S.pw.z, F.nodFull0, F.Nn);
         k_unit_compliance<<<grid_for(Ne, 256), 256, 0, st>>>(S.pw.z, S.K0_64, F.eleFull0, Ne, F.g, S.adjCe);
         TG_LAUNCH_CHECK(id);
-        double *h = nullptr;
-        TG_HIP(hipHostMalloc((void **)&h, sizeof(double), hipHostMallocDefault), id);
-        try {
-            *c_out = reduce_dev(R_DOT, S.adjE, S.adjCe, Ne, S.adjPart, S.adjRes, h, st);
-        } catch (...) {
-            (void)hipHostFree(h);
-            throw;
-        }
-        (void)hipHostFree(h);
+        *c_out = reduce_dev(R_DOT, S.adjE, S.adjCe, Ne, st);
         if (d_dcdx) {
             k_sens<<<grid_for(Ne, 256), 256, 0, st>>>(S.adjXp, S.adjCe, f ? S.adjG.p : d_dcdx, Ne, 1, Emin, E0, penal, 1.0);
             TG_LAUNCH_CHECK(id);
@@ -877,16 +966,7 @@ int tg_reduce(int32_t op, const double *d_a, const double *d_b, int64_t n, doubl
     return guard("tg_reduce:Input", [&] {
         if (!d_a || !out || n < 0 || ((op == TG_RED_DOT || op == TG_RED_MAXABSDIFF) && !d_b))
             fail(TG_ERR_ARGS, "tg_reduce:Input", "bad arguments");
-        DevBuf<double> partial(RED_BLOCKS), res(1);
-        double *h = nullptr;
-        TG_HIP(hipHostMalloc((void **)&h, sizeof(double), hipHostMallocDefault), "tg_reduce:HIP");
-        try {
-            *out = reduce_dev(op, d_a, d_b, n, partial, res, h, (hipStream_t)stream);
-        } catch (...) {
-            (void)hipHostFree(h);
-            throw;
-        }
-        (void)hipHostFree(h);
+        *out = reduce_dev(op, d_a, d_b, n, (hipStream_t)stream);
     });
 }
 
@@ -901,47 +981,38 @@ int tg_oc_update(const double *d_x, const double *d_dc, const double *d_dv, cons
         auto apart = [&](const double *a) { return !a || a + n <= d_xnew || d_xnew + n <= a; };
         DevBuf<double> own(apart(d_x) && apart(d_dc) && apart(d_dv) && apart(d_passive) ? 0 : n);
         double *b = own.n ? own.p : d_xnew;
-        DevBuf<double> partial((size_t)2 * OC_NODES * nb + RED_BLOCKS), res(1);
-        DevBuf<OcState> state(2);
-        double *h = nullptr;
-        TG_HIP(hipHostMalloc((void **)&h, sizeof(OcState), hipHostMallocDefault), id);
-        try {
-            double *part[2] = {partial.p, partial.p + (size_t)OC_NODES * nb};
-            int k = 0;  // launches; launch k's sums are in part[k & 1], and it left the state before them in state[k & 1]
-            OcState s{0.0, 1e9, 0.0, 0.0};
-            // (l2-l1)/(l1+l2) halves each step from 1: at most ~100 steps, more than 48 but for the largest
-            // multipliers; check after 48, then every 16
-            for (int upto = 48; ; upto += 16) {
-                for (; OC_DEPTH * k < upto; ++k) {
-                    if (k == 0)
-                        k_oc_pass<true><<<nb, RED_THREADS, 0, st>>>(d_x, d_dc, d_dv, b, d_passive, n, fval, move, nullptr,
-                                                                    state.p, nullptr, part[0]);
-                    else
-                        k_oc_pass<false><<<nb, RED_THREADS, 0, st>>>(d_x, d_dc, d_dv, b, d_passive, n, fval, move,
-                                                                     state.p + ((k - 1) & 1), state.p + (k & 1),
-                                                                     part[(k - 1) & 1], part[k & 1]);
-                }
-                k_oc_close<<<1, RED_THREADS, 0, st>>>(n, fval, state.p + ((k - 1) & 1), state.p + (k & 1), part[(k - 1) & 1], nb);
-                TG_LAUNCH_CHECK(id);
-                TG_HIP(hipMemcpyAsync(h, state.p + (k & 1), sizeof(OcState), hipMemcpyDeviceToHost, st), id);
-                TG_HIP(hipStreamSynchronize(st), id);
-                std::memcpy(&s, h, sizeof s);
-                if (!((s.l2 - s.l1) / (s.l1 + s.l2) > 1e-6)) break;
-                if (upto > 400) fail(TG_ERR_NUMERIC, "tg_oc_update:Numeric", "bisection did not converge");
+        Scratch sc(st);
+        OcState *state = (OcState *)sc.dbl();  // 16 doubles, then the sums of two launches, then the maxima
+        double *part[2] = {sc.dbl() + 16, sc.dbl() + 16 + (size_t)OC_NODES * nb}, *maxima = sc.dbl() + 16 + (size_t)2 * OC_NODES * nb;
+        int k = 0;  // launches; launch k's sums are in part[k & 1], and it left the state before them in state[k & 1]
+        OcState s{0.0, 1e9, 0.0, 0.0};
+        // (l2-l1)/(l1+l2) halves each step from 1: at most ~100 steps, more than 48 but for the largest
+        // multipliers; check after 48, then every 16
+        for (int upto = 48; ; upto += 16) {
+            for (; OC_DEPTH * k < upto; ++k) {
+                if (k == 0)
+                    k_oc_pass<true><<<nb, RED_THREADS, 0, st>>>(d_x, d_dc, d_dv, b, d_passive, n, fval, move, nullptr, state,
+                                                                nullptr, part[0]);
+                else
+                    k_oc_pass<false><<<nb, RED_THREADS, 0, st>>>(d_x, d_dc, d_dv, b, d_passive, n, fval, move,
+                                                                 state + ((k - 1) & 1), state + (k & 1), part[(k - 1) & 1],
+                                                                 part[k & 1]);
             }
-            k_oc_apply<<<RED_BLOCKS, RED_THREADS, 0, st>>>(d_x, d_dc, d_dv, d_passive, d_xnew, n, move, state.p + (k & 1),
-                                                           partial);
-            k_red_final<R_MAXABSDIFF><<<1, RED_THREADS, 0, st>>>(partial, RED_BLOCKS, res);
+            const unsigned long long seq = sc.next();
+            k_oc_close<<<1, RED_THREADS, 0, st>>>(n, fval, state + ((k - 1) & 1), state + (k & 1), part[(k - 1) & 1], nb,
+                                                  sc.host(), sc.seq_ptr(), seq);
             TG_LAUNCH_CHECK(id);
-            TG_HIP(hipMemcpyAsync(h, res.p, sizeof(double), hipMemcpyDeviceToHost, st), id);
-            TG_HIP(hipStreamSynchronize(st), id);
-            if (change) *change = h[0];
-            if (bisections) *bisections = 16 * (int)std::ceil(s.steps / 16);
-        } catch (...) {
-            (void)hipHostFree(h);
-            throw;
+            std::memcpy(&s, sc.wait(id), sizeof s);
+            if (!((s.l2 - s.l1) / (s.l1 + s.l2) > 1e-6)) break;
+            if (upto > 400) fail(TG_ERR_NUMERIC, "tg_oc_update:Numeric", "bisection did not converge");
         }
-        (void)hipHostFree(h);
+        const unsigned long long seq = sc.next();
+        k_oc_apply<<<RED_BLOCKS, RED_THREADS, 0, st>>>(d_x, d_dc, d_dv, d_passive, d_xnew, n, move, state + (k & 1), maxima);
+        k_red_final<R_MAXABSDIFF><<<1, RED_THREADS, 0, st>>>(maxima, RED_BLOCKS, sc.host(), sc.seq_ptr(), seq);
+        TG_LAUNCH_CHECK(id);
+        const double m = *sc.wait(id);
+        if (change) *change = m;
+        if (bisections) *bisections = 16 * (int)std::ceil(s.steps / 16);
     });
 }
 
