@@ -13,9 +13,11 @@ struct Filter {
     hipStream_t st;
     Grid g{};
     int64_t Ne = 0;
-    DevBuf<double> Kd, inv, b, y;
-    DevBuf<uint8_t> nodeMask, eleMask;
+    double kd[4] = {};           // the element matrix: entries between corners 0, 1, 2 and 3 edges apart
+    DevBuf<double> inv, y, parts;  // the preconditioner per set of solid elements around a node; the iterate; partial sums
+    DevBuf<uint8_t> code;        // the solid elements around each node
     DevBuf<int32_t> eleFwd, eleFull0;
+    int ty = 0, tx = 0, tyn = 0, tiles = 0, chunk = 0, chunks = 0, np = 0;  // k_filter_step's tiles; partials of a sum
     PcgWork pw;
     Filter(const tg_model &mm, double rMin, hipStream_t s);
     void apply(const double *src, double *tar, double tol, int maxIT, int *its, double *res);

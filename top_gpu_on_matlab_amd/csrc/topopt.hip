@@ -384,89 +384,234 @@ __global__ __launch_bounds__(RED_THREADS) void k_oc_apply(const double *__restri
 }
 
 // ---- PDE filter ------------------------------------------------------------------------------
-// element -> node: b_n = sum over solid elements around n of src_e * (1/8)  (TOP_GPU.m:975-996)
-__global__ void k_e2n(const double *__restrict__ src, const int32_t *__restrict__ eleFwd, const uint8_t *__restrict__ mask,
-                      const Grid g, double *__restrict__ b) {
+// The filter's Jacobi-PCG has two kernels an iteration.  k_filter_step makes the direction p = inv r +
+// beta p, adds the previous step to the iterate and applies the operator to the new direction;
+// k_filter_update takes the residual on.  Each finishes the other's partial sums in all its workgroups (one
+// order, one value), and workgroup 0 of the next k_filter_step tells the host the residual norm, so the
+// host's look at it runs beside that kernel: when the loop stops there, that launch has only made the last
+// update of the iterate, which is due anyway.
+constexpr int FS_THREADS = 512;
+
+// The solid elements around each node, one bit each: (oy+1) + 2(ox+1) + 4(oz+1) for offsets in {-1, 0}.
+__global__ void k_filter_codes(const uint8_t *__restrict__ eleMask, const Grid g, uint8_t *__restrict__ code) {
     const int64_t n = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (n >= g.nodes()) return;
-    double s = 0;
-    if (mask[n] & NODE_ACTIVE) {
-        const int iy = (int)(n % g.NY);
-        const int64_t t = n / g.NY;
-        const int ix = (int)(t % g.NX), iz = (int)(t / g.NX);
-        for (int oz = -1; oz <= 0; ++oz)
-            for (int ox = -1; ox <= 0; ++ox)
-                for (int oy = -1; oy <= 0; ++oy) {
-                    const int ey = iy + oy, ex = ix + ox, ez = iz + oz;
-                    if ((unsigned)ey >= (unsigned)g.EY || (unsigned)ex >= (unsigned)g.EX || (unsigned)ez >= (unsigned)g.EZ)
-                        continue;
-                    const int32_t k = eleFwd[ey + (int64_t)g.EY * (ex + (int64_t)g.EX * ez)];
-                    if (k > 0) s += src[k - 1] * (1.0 / 8);
-                }
+    const int iy = (int)(n % g.NY);
+    const int64_t t = n / g.NY;
+    const int ix = (int)(t % g.NX), iz = (int)(t / g.NX);
+    int c = 0;
+    for (int j = 0; j < 8; ++j) {
+        const int ey = iy - 1 + (j & 1), ex = ix - 1 + ((j >> 1) & 1), ez = iz - 1 + (j >> 2);
+        if ((unsigned)ey < (unsigned)g.EY && (unsigned)ex < (unsigned)g.EX && (unsigned)ez < (unsigned)g.EZ &&
+            eleMask[ey + (int64_t)g.EY * (ex + (int64_t)g.EX * ez)])
+            c |= 1 << j;
     }
-    b[n] = s;
+    code[n] = (uint8_t)c;
 }
 
-// y_n = sum over solid elements around n of (u_e' * iKEF)_a  (MatTimesVec_matrixFree_B, TOP_GPU.m:1008-1031)
-template <int MODE>
-__global__ void k_filter_apply(const double *__restrict__ u, double *__restrict__ y, const double *__restrict__ K,
-                               const uint8_t *__restrict__ eleMask, const uint8_t *__restrict__ mask, const Grid g,
-                               const double *__restrict__ inv) {
-    const int64_t n = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (n >= g.nodes()) return;
-    if (MODE == 1) {  // Jacobi preconditioner diagPrecond .* x
-        y[n] = inv[n] * u[n];
-        return;
+// The sums of a and of b over the workgroup (whole wavefronts, at most 16), in every thread.
+__device__ inline void block_sum2(double &a, double &b) {
+    __shared__ double sh[32];
+    for (int o = 32; o > 0; o >>= 1) {
+        a += __shfl_xor(a, o, 64);
+        b += __shfl_xor(b, o, 64);
     }
-    double s = 0;
-    if (mask[n] & NODE_ACTIVE) {
-        const int iy = (int)(n % g.NY);
-        const int64_t t = n / g.NY;
-        const int ix = (int)(t % g.NX), iz = (int)(t / g.NX);
-#pragma unroll
-        for (int oz = -1; oz <= 0; ++oz)
-#pragma unroll
-            for (int ox = -1; ox <= 0; ++ox)
-#pragma unroll
-                for (int oy = -1; oy <= 0; ++oy) {
-                    const int ey = iy + oy, ex = ix + ox, ez = iz + oz;
-                    if ((unsigned)ey >= (unsigned)g.EY || (unsigned)ex >= (unsigned)g.EX || (unsigned)ez >= (unsigned)g.EZ)
-                        continue;
-                    if (!eleMask[ey + (int64_t)g.EY * (ex + (int64_t)g.EX * ez)]) continue;
-                    const int a = vtx_of(-oy, -ox, -oz);
-                    double v = 0;
-#pragma unroll
-                    for (int b = 0; b < 8; ++b) {
-                        const int64_t m = (ey + vtx_y(b)) + (int64_t)g.NY * ((ex + vtx_x(b)) + (int64_t)g.NX * (ez + vtx_z(b)));
-                        v += u[m] * K[b + 8 * a];
-                    }
-                    s += v;
-                }
+    __syncthreads();  // the last use of the shared array is over
+    if ((threadIdx.x & 63) == 0) {
+        sh[threadIdx.x >> 6] = a;
+        sh[16 + (threadIdx.x >> 6)] = b;
     }
-    y[n] = s;
+    __syncthreads();
+    a = b = 0;
+    for (int w = 0; w < (int)blockDim.x >> 6; ++w) {
+        a += sh[w];
+        b += sh[16 + w];
+    }
 }
 
-__global__ void k_filter_diag(const double *__restrict__ K, const uint8_t *__restrict__ eleMask,
-                              const uint8_t *__restrict__ mask, const Grid g, double *__restrict__ inv) {
-    const int64_t n = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (n >= g.nodes()) return;
-    double s = 0;
-    if (mask[n] & NODE_ACTIVE) {
-        const int iy = (int)(n % g.NY);
-        const int64_t t = n / g.NY;
-        const int ix = (int)(t % g.NX), iz = (int)(t / g.NX);
-        for (int oz = -1; oz <= 0; ++oz)
-            for (int ox = -1; ox <= 0; ++ox)
-                for (int oy = -1; oy <= 0; ++oy) {
-                    const int ey = iy + oy, ex = ix + ox, ez = iz + oz;
-                    if ((unsigned)ey >= (unsigned)g.EY || (unsigned)ex >= (unsigned)g.EX || (unsigned)ez >= (unsigned)g.EZ)
-                        continue;
-                    if (!eleMask[ey + (int64_t)g.EY * (ex + (int64_t)g.EX * ez)]) continue;
-                    const int a = vtx_of(-oy, -ox, -oz);
-                    s += K[a + 8 * a];
-                }
+// element -> node: r_n = b_n = sum over solid elements around n of src_e * (1/8)  (TOP_GPU.m:975-996), with
+// partial sums of b.b and of the preconditioned b.(inv b).  A chain of three loads a node (its elements, their
+// numbers, their values): the workgroups are the widest there are, so that few nodes of a thread follow each
+// other (128x256x128: 45 us; of 256
+// threads, with a branch an element, 98)
+constexpr int E2N_THREADS = 1024;
+__global__ __launch_bounds__(E2N_THREADS) void k_e2n(const double *__restrict__ src, const int32_t *__restrict__ eleFwd,
+                                                     const uint8_t *__restrict__ code, const Grid g,
+                                                     const double *__restrict__ inv, double *__restrict__ r,
+                                                     double *__restrict__ pbb, double *__restrict__ pzr) {
+    double bb = 0, zr = 0;
+    const unsigned nn = (unsigned)g.nodes(), NY = g.NY, NX = g.NX;  // node numbers are 32 bits (the maps')
+    for (unsigned n = blockIdx.x * E2N_THREADS + threadIdx.x; n < nn; n += gridDim.x * E2N_THREADS) {
+        double s = 0;
+        const int c = code[n];
+        if (c) {
+            const unsigned t = n / NY, iy = n - t * NY, iz = t / NX, ix = t - iz * NX;
+            const int e0 = (int)(iy - 1 + g.EY * (ix - 1 + g.EX * (iz - 1)));
+            auto at = [&](int j) { return e0 + (j & 1) + g.EY * (((j >> 1) & 1) + g.EX * (j >> 2)); };
+            const int ok = at(__ffs(c) - 1);  // an element that is there, in place of those that are not: no branches
+            int32_t k[8];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) k[j] = eleFwd[c & (1 << j) ? at(j) : ok];
+            double v[8];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) v[j] = src[k[j] - 1];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) s += c & (1 << j) ? v[j] * (1.0 / 8) : 0.0;
+        }
+        r[n] = s;
+        bb += s * s;
+        zr += inv[c] * s * s;
     }
-    inv[n] = (mask[n] & NODE_ACTIVE) ? 1.0 / s : 0.0;
+    block_sum2(bb, zr);
+    if (threadIdx.x == 0) {
+        pbb[blockIdx.x] = bb;
+        pzr[blockIdx.x] = zr;
+    }
+}
+
+struct FilterStep {
+    Grid g;
+    int ty, tx, tyn, chunk;        // nodes of a tile along y and x, tiles along y, planes of a chunk
+    double k0, k1, k2, k3;         // the element matrix: entries between corners 0, 1, 2 and 3 edges apart
+    const uint8_t *code;
+    const double *inv, *r;
+    double *pold, *p, *y, *v;      // the last direction, the new one, the iterate, the product
+    const double *prr, *pzr;       // the partial sums r.r (b.b at first) and z.r that k_filter_update left
+    int np;
+    double *ppv;                   // the partial sums p.v for it
+    double *scal, *host;
+    unsigned long long seq;        // published with the residual norm
+    int xo, xn;                    // slots of z.r: the last direction's and this one's
+};
+
+// p = inv r + beta p;  y += lambda p of before;  v_n = sum over solid elements around n of (K p_e)_a
+// (MatTimesVec_matrixFree_B, TOP_GPU.m:1008-1031);  partial sums of p.v.   IT: 0 the first direction, 1 the
+// second (the iterate is still zero), 2 any later one.
+// A workgroup walks a tile of columns up z, a thread a column (the tile's rim only supplies its p to the
+// neighbours through LDS), with the next plane's loads in flight.  The element matrix has one entry per
+// distance of two corners, so a plane's part of an element's product is a sum over the quadrant of the 3x3
+// nodes around the column, and a layer of elements is two such parts: each plane is read and turned once.
+// Bound by memory: six streams of 8 bytes per node and the rims (128x256x128: 63 us, 3.5 TB/s without the
+// rims; with k_filter_update's 19 an iteration takes 82 us, where nine launches took 200; 24x48x24: 6.6 and
+// 4.7 us).  512 threads a tile: 256 take 72 us, more of them being rim, and 1024 take 61 but 9.5 at 24x48x24.
+template <int IT>
+__global__ __launch_bounds__(FS_THREADS) void k_filter_step(const FilterStep a) {
+    __shared__ double pl[2][FS_THREADS], tab[256];
+    const Grid &g = a.g;
+    const int t = threadIdx.x, h = a.ty + 2;
+    if (t < 256) tab[t] = a.inv[t];
+    double rr = 0, zr = 0;
+    for (int i = t; i < a.np; i += FS_THREADS) {
+        rr += a.prr[i];
+        zr += a.pzr[i];
+    }
+    block_sum2(rr, zr);  // its barriers cover tab too
+    double beta = 0, lam = 0;
+    if (IT) {
+        const double zr0 = a.scal[a.xo];
+        beta = zr / zr0;
+        lam = zr0 / a.scal[S_PV];
+    }
+    if (blockIdx.x == 0 && blockIdx.y == 0 && t == 0) {
+        a.scal[a.xn] = zr;  // the other slot: every workgroup reads the old one
+        if (IT == 0) {
+            a.scal[S_BB] = rr;
+        } else {
+            a.host[S_BB] = a.scal[S_BB];
+            a.host[S_RR] = rr;
+            __hip_atomic_store((unsigned long long *)(a.host + 16), a.seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+        }
+    }
+    const int ly = t % h, lx = t / h;
+    const int iy = (int)(blockIdx.x % a.tyn) * a.ty + ly - 1, ix = (int)(blockIdx.x / a.tyn) * a.tx + lx - 1;
+    const bool on = lx < a.tx + 2 && (unsigned)iy < (unsigned)g.NY && (unsigned)ix < (unsigned)g.NX;
+    const bool own = on && ly >= 1 && ly <= a.ty && lx >= 1 && lx <= a.tx;
+    const int64_t plane = (int64_t)g.NY * g.NX;
+    const int z0 = (int)blockIdx.y * a.chunk, z1 = min(z0 + a.chunk, g.NZ);
+    const int zb = max(z0 - 1, 0), ze = min(z1, g.NZ - 1);  // planes read
+    int64_t n = iy + (int64_t)g.NY * ix + plane * zb;
+    double r = 0, po = 0, y = 0;
+    int c = 0;
+    auto load = [&](int z, int64_t m) {
+        if (!on) return;
+        c = a.code[m];
+        r = a.r[m];
+        if (IT) po = a.pold[m];
+        if (IT == 2 && own && z >= z0 && z < z1) y = a.y[m];
+    };
+    load(zb, n);
+    double q1[4] = {}, q2[4] = {}, acc = 0, pc = 0, pv = 0;  // of the plane below
+    int cc = 0;
+    for (int z = zb; z <= ze; ++z, n += plane) {
+        const double p = IT ? tab[c] * r + beta * po : tab[c] * r, p0 = po, y0 = y;
+        const int cz = c;
+        if (z < ze) load(z + 1, n + plane);
+        double *b = pl[z & 1];
+        b[t] = p;
+        const bool in = own && z >= z0 && z < z1;
+        if (in) {
+            a.p[n] = p;
+            if (IT) a.y[n] = (IT == 2 ? y0 : 0.0) + lam * p0;
+        }
+        __syncthreads();
+        if (!own) continue;
+        const double up = b[t + 1], dn = b[t - 1], lf = b[t - h], rt = b[t + h];
+        const double f[4] = {dn + lf, up + lf, dn + rt, up + rt};
+        const double d[4] = {b[t - 1 - h], b[t + 1 - h], b[t - 1 + h], b[t + 1 + h]};
+        double below = 0;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const double e1 = a.k0 * p + a.k1 * f[k] + a.k2 * d[k], e2 = a.k1 * p + a.k2 * f[k] + a.k3 * d[k];
+            if (cc & (16 << k)) {  // the element between the two planes: above the last, below this one
+                acc += q1[k] + e2;
+                below += e1 + q2[k];
+            }
+            q1[k] = e1;
+            q2[k] = e2;
+        }
+        if (z > z0) {  // the plane below is complete (z0 - 1 is another chunk's)
+            a.v[n - plane] = acc;
+            pv += pc * acc;
+        }
+        acc = below;
+        pc = p;
+        cc = cz;
+    }
+    if (own && z1 == g.NZ) {  // the top plane has no layer above
+        a.v[n - plane] = acc;
+        pv += pc * acc;
+    }
+    double unused = 0;
+    block_sum2(pv, unused);
+    if (t == 0) a.ppv[blockIdx.x + gridDim.x * blockIdx.y] = pv;
+}
+
+// r -= lambda v, with partial sums of r.r and r.(inv r); p.v is finished here from k_filter_step's partials.
+__global__ __launch_bounds__(RED_THREADS) void k_filter_update(double *__restrict__ r, const double *__restrict__ v,
+                                                               int64_t n, const uint8_t *__restrict__ code,
+                                                               const double *__restrict__ inv,
+                                                               const double *__restrict__ ppv, int npv,
+                                                               double *__restrict__ scal, int ix,
+                                                               double *__restrict__ prr, double *__restrict__ pzr) {
+    __shared__ double tab[256];
+    tab[threadIdx.x] = inv[threadIdx.x];
+    double pv = 0, zr = 0, rr = 0;
+    for (int i = threadIdx.x; i < npv; i += RED_THREADS) pv += ppv[i];
+    block_sum2(pv, zr);
+    if (blockIdx.x == 0 && threadIdx.x == 0) scal[S_PV] = pv;
+    const double lam = scal[ix] / pv;
+    zr = 0;
+    for (int64_t i = (int64_t)blockIdx.x * RED_THREADS + threadIdx.x; i < n; i += (int64_t)gridDim.x * RED_THREADS) {
+        const double x = r[i] - lam * v[i];
+        r[i] = x;
+        rr += x * x;
+        zr += tab[code[i]] * x * x;
+    }
+    block_sum2(rr, zr);
+    if (threadIdx.x == 0) {
+        prr[blockIdx.x] = rr;
+        pzr[blockIdx.x] = zr;
+    }
 }
 
 // node -> element: tar_e = sum(tar(eNod(e,:))) * (1/8)  (TOP_GPU.m:1004-1005)
@@ -474,8 +619,8 @@ __global__ void k_n2e(const double *__restrict__ tar, const int32_t *__restrict_
                       double *__restrict__ out) {
     const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (k >= Ne) return;
-    const int64_t e = eleFull0[k];
-    const int ey = (int)(e % g.EY), ex = (int)((e / g.EY) % g.EX), ez = (int)(e / ((int64_t)g.EY * g.EX));
+    const unsigned e = eleFull0[k], EY = g.EY, EX = g.EX;
+    const unsigned c = e / EY, ey = e - c * EY, ez = c / EX, ex = c - ez * EX;
     double s = 0;
 #pragma unroll
     for (int b = 0; b < 8; ++b)
@@ -733,39 +878,90 @@ Filter::Filter(const tg_model &mm, double rMin, hipStream_t s) : m(mm), st(s) {
     Ne = L.Ne;
     double K[64];
     pde_filter_kernel(rMin, 1.0, K);  // eleSize(1) = 1 on the finest level (TOP_GPU.m:2066)
-    Kd.upload(K, 64, st);
-    std::vector<uint8_t> mask(g.nodes(), 0);
-    for (int64_t k = 0; k < L.Nn; ++k) mask[L.nodFull[k] - 1] = NODE_ACTIVE;
-    nodeMask.upload(mask, st);
-    eleMask.upload(L.solid, st);
+    // a cube of the Laplacian and the mass: one entry per number of edges between two corners
+    kd[0] = K[0];
+    kd[1] = K[1];
+    kd[2] = K[2];
+    kd[3] = K[6];
+    // the preconditioner 1 / (sum of the diagonal entries of the elements around a node), per set of elements
+    double tab[256];
+    for (int c = 0; c < 256; ++c) {
+        double s = 0;
+        for (int j = 0; j < 8; ++j)
+            if (c & (1 << j)) s += K[9 * vtx_of(!(j & 1), !(j & 2), !(j & 4))];
+        tab[c] = c ? 1.0 / s : 0.0;
+    }
+    inv.upload(tab, 256, st);
     eleFwd.upload(L.eleMapForward, st);
     std::vector<int32_t> ef(L.Ne);
     for (int64_t k = 0; k < L.Ne; ++k) ef[k] = L.eleMapBack[k] - 1;
     eleFull0.upload(ef, st);
-    inv.alloc(g.nodes());
-    b.alloc(g.nodes());
+    DevBuf<uint8_t> solid;
+    solid.upload(L.solid, st);
+    code.alloc(g.nodes());
+    k_filter_codes<<<grid_for(g.nodes(), 256), 256, 0, st>>>(solid, g, code);
+    TG_LAUNCH_CHECK(id);
     y.alloc(g.nodes());
     pw.init(g.nodes(), st);
-    k_filter_diag<<<grid_for(g.nodes(), 256), 256, 0, st>>>(Kd, eleMask, nodeMask, g, inv);
-    TG_LAUNCH_CHECK(id);
+    // the tile: the fewest workgroups a plane (rims included, a tile is at most FS_THREADS nodes)
+    int64_t best = INT64_MAX;
+    for (int n = (int)((g.NY + FS_THREADS / 3 - 3) / (FS_THREADS / 3 - 2)); n <= g.NY; ++n) {
+        const int cy = (g.NY + n - 1) / n, cx = FS_THREADS / (cy + 2) - 2;
+        const int64_t count = (int64_t)((g.NY + cy - 1) / cy) * ((g.NX + cx - 1) / cx);
+        if (count < best) {
+            best = count;
+            ty = cy;
+            tx = cx;
+        }
+        if (cy <= 16) break;  // shorter runs along y are not worth a few workgroups
+    }
+    tyn = (g.NY + ty - 1) / ty;
+    tiles = (int)best;
+    // The chunk: its planes are read once and the two beside it again; a plane takes a latency (as long as
+    // one workgroup's share of the traffic) and the shares of the workgroups on the compute unit.
+    int dev = 0, cus = 0;
+    TG_HIP(hipGetDevice(&dev), id);
+    TG_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev), id);
+    cus = std::max(cus, 1);
+    best = INT64_MAX;
+    for (int z = 1; z <= g.NZ; ++z) {
+        const int64_t n = (int64_t)tiles * ((g.NZ + z - 1) / z), cost = (z + 2) * (1 + (n + cus - 1) / cus);
+        if (cost < best) {
+            best = cost;
+            chunk = z;
+        }
+    }
+    chunks = (g.NZ + chunk - 1) / chunk;
+    np = (int)std::min<int64_t>(RED_BLOCKS, (g.nodes() + 2 * RED_THREADS - 1) / (2 * RED_THREADS));
+    parts.alloc((int64_t)tiles * chunks + 2 * np);
     TG_HIP(hipStreamSynchronize(st), id);
 }
 
 void Filter::apply(const double *src, double *tar, double tol, int maxIT, int *its, double *res) {
     const char *id = "tg_filter_apply:Numeric";
-    const unsigned gn = grid_for(g.nodes(), 256);
-    k_e2n<<<gn, 256, 0, st>>>(src, eleFwd, nodeMask, g, b);
-    y.zero(st);
-    TG_LAUNCH_CHECK(id);
-    pw.run([&](const double *u, double *out, int) {
-               k_filter_apply<0><<<gn, 256, 0, st>>>(u, out, Kd, eleMask, nodeMask, g, nullptr);
-               return false;
-           },
-           [&](const double *r, double *z, int) {
-               k_filter_apply<1><<<gn, 256, 0, st>>>(r, z, nullptr, nullptr, nullptr, g, inv);
-               return false;
-           },
-           b, y, tol, maxIT, false, its, res, id);
+    double *prr = parts, *pzr = prr + np, *ppv = pzr + np;
+    k_e2n<<<np, E2N_THREADS, 0, st>>>(src, eleFwd, code, g, inv, pw.r, prr, pzr);
+    const dim3 grid((unsigned)tiles, (unsigned)chunks);
+    FilterStep a{g, ty, tx, tyn, chunk, kd[0], kd[1], kd[2], kd[3], code, inv, pw.r, pw.z, pw.p, y, pw.v,
+                 prr, pzr, np, ppv, pw.scal, pw.d_hscal, 0, S_XB, S_XA};
+    k_filter_step<0><<<grid, FS_THREADS, 0, st>>>(a);
+    int it = 0;
+    double rn = 0;
+    for (it = 1; it <= maxIT; ++it) {
+        k_filter_update<<<np, RED_THREADS, 0, st>>>(pw.r, pw.v, g.nodes(), code, inv, ppv, tiles * chunks, pw.scal,
+                                                    a.xn, prr, pzr);
+        std::swap(a.xn, a.xo);
+        std::swap(a.p, a.pold);
+        a.seq = ++pw.seq;
+        if (it == 1) k_filter_step<1><<<grid, FS_THREADS, 0, st>>>(a);
+        else k_filter_step<2><<<grid, FS_THREADS, 0, st>>>(a);
+        TG_LAUNCH_CHECK(id);
+        rn = std::sqrt(pw.wait_rr()) / std::sqrt(pw.h_scal[S_BB]);
+        if (!std::isfinite(rn)) fail(TG_ERR_NUMERIC, id, "non-finite residual at iteration %d", it);
+        if (rn < tol) break;
+    }
+    if (its) *its = std::min(it, maxIT);
+    if (res) *res = rn;
     k_n2e<<<grid_for(Ne, 256), 256, 0, st>>>(y, eleFull0, Ne, g, tar);
     TG_LAUNCH_CHECK(id);
 }
