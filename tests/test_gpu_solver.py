@@ -131,6 +131,24 @@ def test_finest_kbyu_kernels_agree(nu):
     torch.cuda.synchronize()
 
 
+@pytest.mark.parametrize('shape', [(64, 64, 64), (72, 64, 64)])
+def test_restriction_on_both_sides_of_the_one_launch_limit(shape):
+    """The largest coarse grid (16 x 16 x 16) whose restriction is one launch and the first one past it, on a
+    perforated domain, against the oracle: sums of at most 8 x 125 terms in FP64, within 1e-13."""
+    from top_gpu_on_matlab_amd.model import Model
+    from top_gpu_on_matlab_amd.solver import Solver
+    vox = holey_mask(*shape, seed=3, frac=0.7)
+    om = M.build_cuboid_model(*shape, opt_case=1, voxels=vox)
+    gm = Model(vox)
+    gm.builtin_case(1)
+    gm.finalize()
+    gsv = Solver(gm)
+    gsv.set_modulus(np.ones(om.levels[0].numElements))
+    gsv.assemble()
+    rf = np.random.default_rng(4).standard_normal(3 * om.levels[0].numNodes)
+    assert _rel(gsv.restrict(rf, 2).cpu().numpy(), S.Solver(om).restrict(rf, 2)) < 1e-13
+
+
 def test_transfer_operators(pair):
     name, om, osv, gm, gsv, E = pair
     rng = np.random.default_rng(2)

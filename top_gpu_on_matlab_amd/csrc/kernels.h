@@ -516,6 +516,89 @@ __global__ __launch_bounds__(RT_THREADS) void k_restrict_tiled(const T *__restri
     }
 }
 
+// The restriction in one launch, for small coarse grids: k_restrict_tiled's planes and k_kelem_gather's sums by
+// (coarse node, element around it, plane, component), one thread each, in their order of operations (the same bits):
+// a thread forms its plane's 2D sum, the planes are folded and the eight elements added through LDS.  Its chain is one plane's loads where a workgroup of the tiled form
+// marches through nine; it reads every value for each of the elements and vertices it goes to.  Against the two
+// launches, us, FP64 (FP32), span 4: 432 coarse elements 6.3 (7.4) against 23 (19), 2,640 12.6 (13.4) against 24 (20),
+// 3,456 14.5 (17) against 24 (20), 8,192 27 (31) against 24 (19), 27,648 78 (85) against 27 (22); span 2: 54 elements 4.5
+// against 11, 3,456 7.2 against 14.  So up to 4,096 coarse elements.
+constexpr int RN_NODES = 4;
+template <typename T, int S>
+__global__ __launch_bounds__(RN_NODES * 24 * (S + 1)) void k_restrict_node(const T *__restrict__ rf,
+                                                                           const uint8_t *__restrict__ coeff,
+                                                                           const Grid gc, const Grid gf,
+                                                                           const uint8_t *__restrict__ eleMask,
+                                                                           const uint8_t *__restrict__ mask,
+                                                                           T *__restrict__ out, const PlanePack pk) {
+    constexpr int PL = S + 1;
+    __shared__ T sv[8][PL][RN_NODES][3], sf[8][RN_NODES][3];
+    __shared__ uint8_t sOn[8][RN_NODES];
+    const int t = threadIdx.x;
+    {
+        const int c = t % 3, k = (t / 3) % RN_NODES, pl = (t / (3 * RN_NODES)) % PL, o = t / (3 * RN_NODES * PL);
+        const int64_t n = (int64_t)blockIdx.x * RN_NODES + k, row = n / gc.NY;
+        const int jy = 1 - (o & 1), jx = 1 - ((o >> 1) & 1), jz = 1 - (o >> 2);  // the gather's order: z, x, y
+        const int ey = (int)(n - row * gc.NY) - jy, ex = (int)(row % gc.NX) - jx, ez = (int)(row / gc.NX) - jz;
+        const bool on = n < gc.nodes() && (unsigned)ey < (unsigned)gc.EY && (unsigned)ex < (unsigned)gc.EX &&
+                        (unsigned)ez < (unsigned)gc.EZ && eleMask[ey + (int64_t)gc.EY * (ex + (int64_t)gc.EX * ez)];
+        if (on) {
+            const int64_t m = S * ey + (int64_t)gf.NY * (S * ex + (int64_t)gf.NX * (S * ez + pl));
+            T x[PL][PL];
+            uint8_t w[PL][PL];
+#pragma unroll
+            for (int b = 0; b <= S; ++b)
+#pragma unroll
+                for (int a = 0; a <= S; ++a) {
+                    x[b][a] = rf[3 * (m + a + gf.NY * b) + c];
+                    w[b][a] = coeff[m + a + gf.NY * b];
+                }
+            T val = 0;
+#pragma unroll
+            for (int b = 0; b <= S; ++b) {
+                T sy = 0;
+#pragma unroll
+                for (int a = 0; a <= S; ++a) sy += (jy ? (T)a / S : (T)(S - a) / S) * (x[b][a] / (T)w[b][a]);
+                val += (jx ? (T)b / S : (T)(S - b) / S) * sy;
+            }
+            sv[o][pl][k][c] = val;
+        }
+        if (pl == 0 && c == 0) sOn[o][k] = on;
+    }
+    __syncthreads();
+    const int c = t % 3, k = (t / 3) % RN_NODES;
+    if (t < 24 * RN_NODES) {
+        const int o = t / (3 * RN_NODES);
+        if (sOn[o][k]) {
+            T acc = 0;
+#pragma unroll
+            for (int pl = 0; pl < S; ++pl) {
+                const T tz = (T)pl / S;
+                acc += (o >> 2 ? (T)1 - tz : tz) * sv[o][pl][k][c];
+            }
+            if (!(o >> 2)) acc += sv[o][S][k][c];  // the element's top plane has z weight 1 (0 for its lower vertices)
+            sf[o][k][c] = acc;
+        }
+    }
+    __syncthreads();
+    const int64_t n = (int64_t)blockIdx.x * RN_NODES + k;
+    if (t >= 3 * RN_NODES || n >= gc.nodes()) return;
+    const bool active = mask[n] & NODE_ACTIVE;
+    T acc = 0;
+    if (active)
+#pragma unroll
+        for (int o = 0; o < 8; ++o)
+            if (sOn[o][k]) acc += sf[o][k][c];
+    out[3 * n + c] = acc;
+    if (active && pk.b) {
+        const int64_t row = n / gc.NY;
+        const int p = (int)(pk.axis == 0 ? n - row * gc.NY : (pk.axis == 1 ? row % gc.NX : row / gc.NX));
+        const int64_t at = pk.off[p] + 3 * (int64_t)pk.lidx[n] + c;
+        pk.b[at] = (double)acc;
+        pk.e1[at] = pk.e2[at] = __longlong_as_double((long long)pk.empty);
+    }
+}
+
 // Prolongation x_f (+)= P x_c (Solving_InterpolationDeviation, TOP_GPU.m:848-878): the reference
 // sums the trilinear interpolants of every non-empty coarse element containing a fine node and
 // divides by their count (transferMatCoeffi).  The trilinear interpolant is continuous across

@@ -848,6 +848,14 @@ template <typename T>
 void Solver::restrict_level(int c, const T *rf, T *rc, const PlanePack *pk) {
     DevLevel &C = lv[c], &F = lv[c - 1];
     const uint8_t *cf = C.coeffCnt.p;
+    if (C.ldk <= restrict_elems) {
+        const unsigned gn = grid_for(C.g.nodes(), RN_NODES);
+        const PlanePack none{};
+        if (C.span == 4) k_restrict_node<T, 4><<<gn, RN_NODES * 24 * 5, 0, st>>>(rf, cf, C.g, F.g, C.eleMask, C.nodeMask, rc, pk ? *pk : none);
+        else k_restrict_node<T, 2><<<gn, RN_NODES * 24 * 3, 0, st>>>(rf, cf, C.g, F.g, C.eleMask, C.nodeMask, rc, pk ? *pk : none);
+        TG_LAUNCH_CHECK("tg_solver:restrict");
+        return;
+    }
     T *fv = sizeof(T) == 8 ? (T *)C.fv64.p : (T *)C.fv32.p;
     const unsigned gt = (unsigned)(((C.g.EY + RT_E - 1) / RT_E) * ((C.g.EX + RT_E - 1) / RT_E) *
                                    ((C.g.EZ + RT_Z - 1) / RT_Z));
