@@ -87,6 +87,51 @@ def test_assemble_entries_match_oracle():
     assert np.abs(_np(dKs3) - ref3).max() < 1e-14 * np.abs(ref3).max()
 
 
+@pytest.mark.parametrize('dtype', [np.float64, np.float32])
+@pytest.mark.parametrize('Ne, nCh', [(1, 1), (70, 3), (65, 8), (130, 64), (3, 70)])
+def test_assembly_entries_children_and_element_counts(Ne, nCh, dtype):
+    """Children counts that the wavefronts share unevenly and element counts at the edges of the tiles, with voids and
+    children with boundary matrices at random, general P: entry by entry within the rounding of a sum of nCh products of two 24-term sums,
+    (nCh + 50) unit roundoffs of the same sums over absolute values."""
+    from top_gpu_on_matlab_amd import mex
+    rng = np.random.default_rng(Ne + nCh)
+    nF, nU = 2 * Ne * nCh, 5
+    up = np.where(rng.random((Ne, nCh)) < 0.1, 0, rng.integers(1, nF + 1, size=(Ne, nCh))).astype(np.int32)
+    E = rng.random(nF).astype(dtype)
+    K0, P = rng.standard_normal((24, 24)).astype(dtype), rng.standard_normal((24, 24, nCh)).astype(dtype)
+    uid = np.where(rng.random(nF) < 0.3, rng.integers(1, nU + 1, size=nF), 0).astype(np.int32)
+    free, fixed = (rng.standard_normal((576, nU)).astype(dtype) for _ in range(2))
+    prev = rng.standard_normal((24, 24, nF)).astype(dtype)
+
+    def ref(child):  # the sums and the same of absolute values, in FP64
+        out, mag = np.zeros((24, 24, Ne)), np.zeros((24, 24, Ne))
+        for e in range(Ne):
+            for s in range(nCh):
+                if up[e, s] > 0:
+                    B = P[:, :, s].astype(np.float64)
+                    K, A = child(up[e, s] - 1)
+                    out[:, :, e] += B.T @ K @ B
+                    mag[:, :, e] += abs(B).T @ A @ abs(B)
+        return out, mag
+
+    def level2(f):
+        m = float(E[f])
+        if uid[f] == 0:
+            return K0.astype(np.float64) * m, abs(K0).astype(np.float64) * m
+        u, x = (a[:, uid[f] - 1].astype(np.float64).reshape(24, 24, order='F') for a in (free, fixed))
+        return u * m + x, abs(u) * m + abs(x)
+
+    eps = (nCh + 50) * np.finfo(dtype).eps
+    out, mag = ref(level2)
+    g = _ga(np.full((24, 24, Ne), np.nan), dtype)
+    mex.assembleKs_level2_inplace(g, _ga(up), _ga(E), _ga(K0.reshape(-1, order='F')), _ga(P), _ga(uid), _ga(free), _ga(fixed))
+    assert (abs(_np(g) - out) <= eps * mag).all()
+    out, mag = ref(lambda f: (prev[:, :, f].astype(np.float64), abs(prev[:, :, f]).astype(np.float64)))
+    g = _ga(np.full((24, 24, Ne), np.nan), dtype)
+    mex.assembleKs_higherLevel_inplace(g, _ga(up), _ga(prev), _ga(P))
+    assert (abs(_np(g) - out) <= eps * mag).all()
+
+
 def test_assemble_super_element_entry():
     from top_gpu_on_matlab_amd import mex
     m = M.build_cuboid_model(10, 20, 10, opt_case=2, super_element=True)

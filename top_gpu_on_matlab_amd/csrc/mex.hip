@@ -6,7 +6,7 @@
 //   * scatter / scatter_accum3: a stable radix sort of (target row, entry) pairs, kept per
 //     connectivity as a CSR incidence, then one lane per target row sums its entries in ascending
 //     entry order (no floating-point atomics);
-//   * Galerkin assembly: one wavefront per coarse element (galerkin.h); the FP64 level-2 entry uses the
+//   * Galerkin assembly: one workgroup per coarse element (galerkin.h); the FP64 level-2 entry uses the
 //     product's linearity in the children moduli (a GEMM on the matrix cores) and recomputes only the
 //     children that carry boundary matrices.
 #include <memory>
@@ -223,12 +223,18 @@ struct SrcLevel2 {
         const int32_t f = up[e + Ne * s];
         return (f > 0 && f <= nFine) ? f - 1 : -1;
     }
-    __device__ T kch(int f, int i) const {
+    __device__ void kch(int f, int t, T (&k)[9]) const {
         const T mod = E[f];
         int32_t uid = hasFixed ? mapU[f] - 1 : -1;
         if (uid >= nU) uid = -1;
-        if (uid >= 0) return uf[(size_t)uid * 576 + i] * mod + ux[(size_t)uid * 576 + i];
-        return K0[i] * mod;
+        if (uid >= 0) unique(uid, mod, t, k);
+        else
+#pragma unroll
+            for (int j = 0; j < 9; ++j) k[j] = K0[64 * j + t] * mod;
+    }
+    __device__ void unique(int32_t uid, T mod, int t, T (&k)[9]) const {
+#pragma unroll
+        for (int j = 0; j < 9; ++j) k[j] = uf[(size_t)uid * 576 + 64 * j + t] * mod + ux[(size_t)uid * 576 + 64 * j + t];
     }
 };
 
@@ -243,7 +249,10 @@ struct SrcHigher {
         const int32_t f = up[e + Ne * s];
         return (f > 0 && f <= nFine) ? f - 1 : -1;
     }
-    __device__ T kch(int f, int i) const { return prev[(size_t)f * 576 + i]; }
+    __device__ void kch(int f, int t, T (&k)[9]) const {
+#pragma unroll
+        for (int j = 0; j < 9; ++j) k[j] = prev[(size_t)f * 576 + 64 * j + t];
+    }
 };
 
 template <typename T>
@@ -259,16 +268,22 @@ struct SrcSuper {
         const int32_t f = up[e + Ne * s];
         return (f > 0 && f <= nFine) ? f - 1 : -1;
     }
-    __device__ T kch(int f, int i) const {
+    __device__ void kch(int f, int t, T (&k)[9]) const {
         int32_t uid1 = hasFixed ? mapU[f] : 0;
         if (uid1 > nU) uid1 = 0;
         if (uid1 > 0) {
-            const size_t fb = (size_t)(uid1 - 1) * 576 * 64, mb = (size_t)f * 64;
-            T acc = 0;
-            for (int q = 0; q < 64; ++q) acc += uf[fb + (size_t)q * 576 + i] * E[mb + q];
-            return acc + ux[(size_t)(uid1 - 1) * 576 + i];
+            const T *u = uf + (size_t)(uid1 - 1) * 576 * 64 + t, *mod = E + (size_t)f * 64;
+#pragma unroll
+            for (int j = 0; j < 9; ++j) k[j] = 0;
+            for (int q = 0; q < 64; ++q)
+#pragma unroll
+                for (int j = 0; j < 9; ++j) k[j] += u[(size_t)q * 576 + 64 * j] * mod[q];
+#pragma unroll
+            for (int j = 0; j < 9; ++j) k[j] += ux[(size_t)(uid1 - 1) * 576 + 64 * j + t];
+        } else {
+#pragma unroll
+            for (int j = 0; j < 9; ++j) k[j] = Ks0[(size_t)f * 576 + 64 * j + t];
         }
-        return Ks0[(size_t)f * 576 + i];
     }
 };
 
@@ -278,21 +293,19 @@ __global__ __launch_bounds__(GK_THREADS) void k_galerkin_mex(T *__restrict__ Ks,
                                                              const T *a0, const T *a1, const T *a2, const T *a3,
                                                              const int32_t *mapU, int hasFixed, int64_t nFine,
                                                              int64_t nU) {
-    __shared__ T sB[576], sK[576], sT[576];
+    __shared__ GalerkinLds<T> lds;
     const int e = blockIdx.x;
-    T acc[9];
+    T *out = Ks + (size_t)e * 576;
     if (MODE == 0) {
         SrcLevel2<T> src{up, Ne, e, a0, a1, a2, a3, mapU, hasFixed != 0, nFine, nU};
-        galerkin_block(acc, src, nCh, P, sB, sK, sT);
+        galerkin_block<false>(out, src, nCh, P, lds);
     } else if (MODE == 1) {
         SrcHigher<T> src{up, Ne, e, a0, nFine};
-        galerkin_block(acc, src, nCh, P, sB, sK, sT);
+        galerkin_block<false>(out, src, nCh, P, lds);
     } else {
         SrcSuper<T> src{up, Ne, e, a0, a1, a2, a3, mapU, hasFixed != 0, nFine, nU};
-        galerkin_block(acc, src, nCh, P, sB, sK, sT);
+        galerkin_block<false>(out, src, nCh, P, lds);
     }
-#pragma unroll
-    for (int i = 0; i < 9; ++i) Ks[(size_t)e * 576 + galerkin_entry(i)] = acc[i];
 }
 
 // ---- level-2 Galerkin through its linearity (FP64) ---------------------------------------------------
@@ -327,28 +340,48 @@ __global__ __launch_bounds__(256) void k_mex_gmat(const double *__restrict__ P, 
 }
 
 // Ech[e + Ne s] = modulus of child s of coarse element e, 0 for void children and children with boundary
-// matrices (those are added by k_mex_galerkin_bnd)
-__global__ void k_mex_ech(const int32_t *__restrict__ up, const double *__restrict__ E, const int32_t *__restrict__ mapU,
-                          int hasFixed, int64_t nFine, int64_t nU, int64_t Ne, int nCh, double *__restrict__ Ech) {
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= Ne * nCh) return;
-    const int32_t f1 = up[t];
-    double v = 0.0;
-    if (f1 > 0 && f1 <= nFine) {
-        const int32_t u1 = hasFixed ? mapU[f1 - 1] : 0;
-        if (!(u1 > 0 && u1 <= nU)) v = E[f1 - 1];
+// matrices (those are added by k_mex_galerkin_bnd); bnd[e]: whether e has any.  A workgroup has 64 elements, its
+// wavefronts every eighth child of theirs.
+__global__ __launch_bounds__(512) void k_mex_ech(const int32_t *__restrict__ up, const double *__restrict__ E,
+                                                 const int32_t *__restrict__ mapU, int hasFixed, int64_t nFine,
+                                                 int64_t nU, int64_t Ne, int nCh, double *__restrict__ Ech,
+                                                 int32_t *__restrict__ bnd) {
+    __shared__ int32_t any[8][64];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int64_t e = (int64_t)blockIdx.x * 64 + lane;
+    int32_t has = 0;
+    if (e < Ne)
+#pragma unroll 8
+        for (int s = w; s < nCh; s += 8) {
+            const int32_t f1 = up[e + Ne * s];
+            double v = 0.0;
+            if (f1 > 0 && f1 <= nFine) {
+                const int32_t u1 = hasFixed ? mapU[f1 - 1] : 0;
+                if (u1 > 0 && u1 <= nU) has = 1;
+                else v = E[f1 - 1];
+            }
+            Ech[e + Ne * s] = v;
+        }
+    any[w][lane] = has;
+    __syncthreads();
+    if (w == 0 && e < Ne) {
+#pragma unroll
+        for (int k = 1; k < 8; ++k) has |= any[k][lane];
+        bnd[e] = has;
     }
-    Ech[t] = v;
 }
 
 // Ks[e * 576 + i] = sum_k Ech[e + Ne k] G[k * 576 + i] on MFMA f64 16x16x4 (lane l holds A(l % 16, l / 16),
 // B(l / 16, l % 16), result register r at (4 r + l / 16, l % 16)): A = 16 elements x 4 children of Ech,
 // B = 4 children x 16 entries of G, so every store row is 16 consecutive entries of one element's page.
-// A wavefront owns 16 NG elements; elements past Ne read zero moduli and store nothing.
+// A wavefront owns 16 NG elements and `tiles` of the 36 tiles of entries (blockIdx.y: which), a serial chain of
+// 2.5 us a tile, so that few elements are shared out over more wavefronts; elements past Ne read zero moduli and store
+// nothing.  8,192 elements of 64 children: 26 us, all tiles in one wavefront 102.
 typedef double tg_mdbl4 __attribute__((ext_vector_type(4)));
 template <int KS, int NG>
 __global__ __launch_bounds__(256) void k_mex_galerkin_gemm(const double *__restrict__ Ech, const double *__restrict__ G,
-                                                           double *__restrict__ Ks, int64_t Ne) {
+                                                           double *__restrict__ Ks, int64_t Ne, int tiles) {
+    const int t0 = blockIdx.y * tiles, t1 = min(t0 + tiles, 36);
     const int lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4;
     const int64_t e0 = ((int64_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * (16 * NG);
     if (e0 >= Ne) return;
@@ -360,7 +393,7 @@ __global__ __launch_bounds__(256) void k_mex_galerkin_gemm(const double *__restr
         for (int kk = 0; kk < KS; ++kk) a[g][kk] = e < Ne ? Ech[e + Ne * (lk + 4 * kk)] : 0.0;
     }
     const double *gp = G + (int64_t)lk * 576 + li;
-    for (int t = 0; t < 36; ++t) {
+    for (int t = t0; t < t1; ++t) {
         tg_mdbl4 acc[NG];
 #pragma unroll
         for (int g = 0; g < NG; ++g) acc[g] = tg_mdbl4{0.0, 0.0, 0.0, 0.0};
@@ -380,7 +413,9 @@ __global__ __launch_bounds__(256) void k_mex_galerkin_gemm(const double *__restr
     }
 }
 
-// Children with boundary matrices only (child() skips the others), added to the GEMM's result.
+// Children with boundary matrices only (child() skips the others), added to the GEMM's result.  k_mex_ech has
+// marked the elements that have any, so that the other workgroups end at once: 8,192 elements, 256 of them with 16
+// such children, 40 us, where one wavefront an element that looked through its children singly took 190.
 struct SrcLevel2Bnd : SrcLevel2<double> {
     __device__ int child(int s) const {
         const int f = SrcLevel2<double>::child(s);
@@ -388,15 +423,17 @@ struct SrcLevel2Bnd : SrcLevel2<double> {
         const int32_t u1 = mapU[f];
         return (u1 > 0 && u1 <= nU) ? f : -1;
     }
+    __device__ void kch(int f, int t, double (&k)[9]) const { unique(mapU[f] - 1, E[f], t, k); }
 };
 
 __global__ __launch_bounds__(GK_THREADS) void k_mex_galerkin_bnd(double *__restrict__ Ks, const int32_t *__restrict__ up,
                                                                  int64_t Ne, int nCh, const double *__restrict__ P,
                                                                  const double *E, const double *K0, const double *uf,
                                                                  const double *ux, const int32_t *mapU, int64_t nFine,
-                                                                 int64_t nU) {
-    __shared__ double sB[576], sK[576], sT[576];
+                                                                 int64_t nU, const int32_t *__restrict__ bnd) {
+    __shared__ GalerkinLds<double> lds;
     const int e = blockIdx.x;
+    if (!bnd[e]) return;
     SrcLevel2Bnd src;
     src.up = up;
     src.Ne = Ne;
@@ -409,13 +446,7 @@ __global__ __launch_bounds__(GK_THREADS) void k_mex_galerkin_bnd(double *__restr
     src.hasFixed = true;
     src.nFine = nFine;
     src.nU = nU;
-    bool any = false;  // uniform over the wavefront
-    for (int s = 0; s < nCh && !any; ++s) any = src.child(s) >= 0;
-    if (!any) return;
-    double acc[9];
-    galerkin_block(acc, src, nCh, P, sB, sK, sT);
-#pragma unroll
-    for (int i = 0; i < 9; ++i) Ks[(size_t)e * 576 + galerkin_entry(i)] += acc[i];
+    galerkin_block<true>(Ks + (size_t)e * 576, src, nCh, P, lds);
 }
 
 }  // namespace
@@ -535,19 +566,26 @@ int assembleKs_level2_inplace(int nlhs, tg_array *plhs, int nrhs, const tg_array
         hipStream_t st = S(stream);
         if (Ne > 0) {
             if (cls == TG_DOUBLE && (nCh == 64 || nCh == 8)) {
-                DevBuf<double> G((size_t)nCh * 576), Ech((size_t)Ne * nCh);
+                // one allocation: G, the children's moduli, the flags of the elements with boundary matrices
+                const size_t nG = (size_t)nCh * 576, nE = (size_t)Ne * nCh;
+                DevBuf<double> buf(nG + nE + ((size_t)Ne + 1) / 2);
+                double *G = buf.p, *Ech = G + nG;
+                int32_t *bnd = (int32_t *)(Ech + nE);
                 k_mex_gmat<<<nCh, 256, 0, st>>>((const double *)pch.p, (const double *)k0.p, G);
-                k_mex_ech<<<grid_for(Ne * nCh, 256), 256, 0, st>>>((const int32_t *)up.p, (const double *)em.p,
-                                                                  (const int32_t *)mu.p, hasFixed, nFine, nU, Ne, nCh, Ech);
-                const unsigned gg = grid_for(Ne, 256);  // 64 elements per wavefront
-                if (nCh == 64) k_mex_galerkin_gemm<16, 4><<<gg, 256, 0, st>>>(Ech, G, (double *)Ks.p, Ne);
-                else k_mex_galerkin_gemm<2, 4><<<gg, 256, 0, st>>>(Ech, G, (double *)Ks.p, Ne);
+                k_mex_ech<<<grid_for(Ne, 64), 512, 0, st>>>((const int32_t *)up.p, (const double *)em.p, (const int32_t *)mu.p,
+                                                            hasFixed, nFine, nU, Ne, nCh, Ech, bnd);
+                // 64 elements per wavefront; the entry tiles shared out until there are 512 workgroups
+                const unsigned gg = grid_for(Ne, 256);
+                const int tiles = (int)std::max<int64_t>(1, std::min<int64_t>(36, 36 * (int64_t)gg / 512));
+                const dim3 gt(gg, (36 + tiles - 1) / tiles);
+                if (nCh == 64) k_mex_galerkin_gemm<16, 4><<<gt, 256, 0, st>>>(Ech, G, (double *)Ks.p, Ne, tiles);
+                else k_mex_galerkin_gemm<2, 4><<<gt, 256, 0, st>>>(Ech, G, (double *)Ks.p, Ne, tiles);
                 if (hasFixed)
                     k_mex_galerkin_bnd<<<(unsigned)Ne, GK_THREADS, 0, st>>>((double *)Ks.p, (const int32_t *)up.p, Ne, nCh,
                         (const double *)pch.p, (const double *)em.p, (const double *)k0.p, (const double *)uf.p,
-                        (const double *)ux.p, (const int32_t *)mu.p, nFine, nU);
+                        (const double *)ux.p, (const int32_t *)mu.p, nFine, nU, bnd);
                 TG_LAUNCH_CHECK(Cu);
-                TG_HIP(hipStreamSynchronize(st), Cu);  // G and Ech are released on leaving the scope
+                TG_HIP(hipStreamSynchronize(st), Cu);  // buf is released on leaving the scope
             } else if (cls == TG_DOUBLE)
                 k_galerkin_mex<double, 0><<<(unsigned)Ne, GK_THREADS, 0, st>>>((double *)Ks.p, (const int32_t *)up.p, Ne, nCh, (const double *)pch.p,
                     (const double *)em.p, (const double *)k0.p, (const double *)uf.p, (const double *)ux.p, (const int32_t *)mu.p, hasFixed, nFine, nU);
