@@ -228,3 +228,30 @@ def test_scatter_incidence_cache_follows_the_connectivity():
         assert np.abs(_np(gX) - ref).max() < 1e-13 * np.abs(ref).max()
         keys = rng.integers(1, 400, size=5000).astype(np.int32)
         gk.t.copy_(torch.from_numpy(keys).cuda())
+
+
+@pytest.mark.parametrize('shift', [0, 1])
+@pytest.mark.parametrize('n', [1, 3, 4, 4097, 8_400_003])
+def test_scatter_notices_one_changed_key(n, shift):
+    """A kept incidence is used again only for the same keys: one key changed in place, at the array's ends and inside,
+    of lengths with and without a rest of the hash's groups and of one and of several groups a thread, on an
+    array aligned to 16 bytes and one 4 bytes past that.  Whole numbers, so the sums are exact."""
+    import torch
+    from top_gpu_on_matlab_amd.mex import GpuArray, scatter_accum3_inplace
+    M = 50
+    rng = np.random.default_rng(n)
+    flat = torch.zeros(n + shift, dtype=torch.int32, device='cuda')
+    gk = GpuArray(flat[shift:], (n, 1))
+    keys = rng.integers(1, M + 1, size=n).astype(np.int32)
+    flat[shift:] = torch.from_numpy(keys).cuda()
+    vals = rng.integers(-4, 5, size=(n, 3)).astype(np.float64)
+    gT = _ga(vals)
+    for at in (None, 0, n - 1, n // 2):
+        if at is not None:
+            keys[at] = keys[at] % M + 1
+            gk.t[at] = int(keys[at])
+        ref = np.stack([np.bincount(keys - 1, weights=vals[:, c], minlength=M) for c in range(3)], axis=1)
+        for _ in range(2):
+            gX = _ga(np.zeros((M, 3)))
+            scatter_accum3_inplace(gk, gT, gX)
+            assert np.array_equal(_np(gX), ref), at
