@@ -256,16 +256,18 @@ __global__ void k_sum_slices(const double *__restrict__ part, int slices, int64_
 
 // Jacobi diagonal: sum over solid elements around the node of the element matrix diagonal.
 // MODE 0: E_e * K0(j,j) (finest, standard); 1: Km entry-major (super-element finest / coarse).
-// Fixed DOFs (finest level) get the identity row's 1; nodes outside the mesh get 1.
+// Fixed DOFs (finest level) get the identity row's 1; nodes outside the mesh get 1.  idiag (optional, finest level): the
+// reciprocal, one per node (of its free DOFs, whose entries are equal).
 template <int MODE>
 __global__ void k_diag(double *__restrict__ diag, const double *__restrict__ E, const double *__restrict__ K0,
                        const double *__restrict__ Km, int64_t ldk, const uint8_t *__restrict__ eleMask,
-                       const uint8_t *__restrict__ mask, const Grid g) {
+                       const uint8_t *__restrict__ mask, const Grid g, double *__restrict__ idiag) {
     const int64_t n = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (n >= g.nodes()) return;
     const uint8_t mk = mask[n];
     if (!(mk & NODE_ACTIVE)) {
         diag[3 * n] = diag[3 * n + 1] = diag[3 * n + 2] = 1.0;
+        if (MODE == 0 && idiag) idiag[n] = 1.0;
         return;
     }
     const int iy = (int)(n % g.NY);
@@ -291,6 +293,7 @@ __global__ void k_diag(double *__restrict__ diag, const double *__restrict__ E, 
                     a2 += Km[(int64_t)((3 * a + 2) * 25) * ldk + e];
                 }
             }
+    if (MODE == 0 && idiag) idiag[n] = 1.0 / a0;
     if (mk & 1) a0 = 1.0;
     if (mk & 2) a1 = 1.0;
     if (mk & 4) a2 = 1.0;
@@ -378,6 +381,7 @@ Solver::Solver(const tg_model &m, hipStream_t s) : model(m), st(s) {
         D.eleFull0.upload(ef, st);
         const int64_t nv = 3 * D.g.nodes();
         D.diag64.alloc(nv);
+        if (i == 0 && !super && prec != TG_PREC_MIXED) D.idiag64.alloc(D.g.nodes());
         D.r64.alloc(nv);
         D.x64.alloc(nv);
         D.t64.alloc(nv);
@@ -632,9 +636,9 @@ void Solver::assemble() {
         DevLevel &D = lv[i];
         const unsigned gr = grid_for(D.g.nodes(), 256);
         if (i == 0 && !super)
-            k_diag<0><<<gr, 256, 0, st>>>(D.diag64, E64, K0_64, nullptr, 0, D.eleMask, D.nodeMask, D.g);
+            k_diag<0><<<gr, 256, 0, st>>>(D.diag64, E64, K0_64, nullptr, 0, D.eleMask, D.nodeMask, D.g, D.idiag64);
         else
-            k_diag<1><<<gr, 256, 0, st>>>(D.diag64, nullptr, nullptr, D.Ks64, D.ldk, D.eleMask, D.nodeMask, D.g);
+            k_diag<1><<<gr, 256, 0, st>>>(D.diag64, nullptr, nullptr, D.Ks64, D.ldk, D.eleMask, D.nodeMask, D.g, nullptr);
         TG_LAUNCH_CHECK(id);
     }
     coarse.factor(lv[L - 1].Ks64, lv[L - 1].ldk, lv[L - 1].eleMask, lv[L - 1].nodeMask, st);
@@ -776,7 +780,7 @@ bool Solver::kbyu_level(int i, const T *u, T *out, int epi, const T *rr, const T
             if (ev) TG_HIP(hipEventRecord(ev[0], st), "tg_solver:kbyu");
             if (f64) {
                 const KWVals<double> &k = kw64;
-                const double *uu = (const double *)u, *r2 = (const double *)rr, *d2 = (const double *)dg;
+                const double *uu = (const double *)u, *r2 = (const double *)rr, *d2 = D.idiag64.p;
                 const double *E2 = (const double *)E;
                 double *o2 = (double *)out;
                 launch_walsh<double>(epi, const_k0, gt, st, uu, o2, E2, D.nodeMask, k, model.prm.cell_size, D.g, kt, r2, d2, omega, dp,
