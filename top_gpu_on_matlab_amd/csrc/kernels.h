@@ -333,14 +333,16 @@ __global__ __launch_bounds__(256) void k_kelem_gather(const T *__restrict__ f, i
 // against 17.6 (12.2), 20,736 19.6 (12.3) against 18.3 (13.4), 65,536 53 (31) against 32 (20); super-element
 // finest level, 16,384: 9.2 against 18.0.  So up to 16,384 elements.
 // EPI_RESID_JAC0: the operand is x = omega r ./ diag, formed as it is loaded and written to xout (a launch fewer).
+// DOT (finest level): also the workgroup's share of u.out (product) or r.out (Jacobi step), to partial: a dot of its
+// own is two launches an iteration more, p.v another (the update finishes it).
 constexpr int KN_NODES = 64;
-template <typename T, int EPI, bool MASKED>
+template <typename T, int EPI, bool MASKED, bool DOT = false>
 __global__ __launch_bounds__(8 * KN_NODES) void k_kelem_node(const T *__restrict__ u, T *__restrict__ out,
                                                              const T *__restrict__ Kp, int64_t ldk,
                                                              const uint8_t *__restrict__ eleMask,
                                                              const uint8_t *__restrict__ mask, const Grid g,
                                                              const T *__restrict__ r, const T *__restrict__ diag, T omega,
-                                                             T *__restrict__ xout) {
+                                                             T *__restrict__ xout, double *__restrict__ partial) {
     constexpr bool J0 = EPI == EPI_RESID_JAC0;
     __shared__ T sf[8][3][KN_NODES];
     __shared__ uint8_t sOn[8][KN_NODES];
@@ -382,26 +384,36 @@ __global__ __launch_bounds__(8 * KN_NODES) void k_kelem_node(const T *__restrict
     }
     sOn[o][lane] = on;
     __syncthreads();
-    if (o >= 3 || n >= g.nodes()) return;
-    const int c = o;  // wavefronts 0..2: one component each
-    const uint8_t mk = mask[n];
-    const int64_t k = 3 * n + c;
-    if (!(mk & NODE_ACTIVE)) {
-        out[k] = 0;
-        if (J0) xout[k] = 0;
-        return;
-    }
-    T v = 0;
+    double dot = 0;
+    if (o < 3 && n < g.nodes()) {
+        const int c = o;  // wavefronts 0..2: one component each
+        const uint8_t mk = mask[n];
+        const int64_t k = 3 * n + c;
+        if (mk & NODE_ACTIVE) {
+            T v = 0;
 #pragma unroll
-    for (int q = 0; q < 8; ++q)
-        if (sOn[q][lane]) v += sf[q][c][lane];
-    const T rk = EPI == EPI_KU ? (T)0 : r[k], dk = J0 || EPI == EPI_JACOBI ? diag[k] : (T)1;
-    const T uk = J0 ? omega * (rk / dk) : (MASKED || EPI == EPI_JACOBI ? u[k] : (T)0);
-    if (MASKED && (mk & (1 << c))) v = uk;
-    if (J0) xout[k] = uk;
-    if (EPI == EPI_RESID || J0) v = rk - v;
-    if (EPI == EPI_JACOBI) v = uk + (omega * (rk - v)) / dk;
-    out[k] = v;
+            for (int q = 0; q < 8; ++q)
+                if (sOn[q][lane]) v += sf[q][c][lane];
+            const T rk = EPI == EPI_KU ? (T)0 : r[k], dk = J0 || EPI == EPI_JACOBI ? diag[k] : (T)1;
+            const T uk = J0 ? omega * (rk / dk) : (MASKED || DOT || EPI == EPI_JACOBI ? u[k] : (T)0);
+            if (MASKED && (mk & (1 << c))) v = uk;
+            if (J0) xout[k] = uk;
+            if (EPI == EPI_RESID || J0) v = rk - v;
+            if (EPI == EPI_JACOBI) v = uk + (omega * (rk - v)) / dk;
+            out[k] = v;
+            if (DOT) dot = (double)v * (double)(EPI == EPI_KU ? uk : rk);
+        } else {
+            out[k] = 0;
+            if (J0) xout[k] = 0;
+        }
+    }
+    if (DOT) {
+        __shared__ double sd[3];
+        for (int w = 32; w > 0; w >>= 1) dot += __shfl_xor(dot, w, 64);
+        if (o < 3 && lane == 0) sd[o] = dot;
+        __syncthreads();
+        if (threadIdx.x == 0) partial[blockIdx.x] = sd[0] + sd[1] + sd[2];
+    }
 }
 
 // Trilinear weight of coarse vertex j at fine offset (a, b, c) of a span-S block; exact in binary.

@@ -755,8 +755,9 @@ static void launch_walsh(int epi, bool ck, unsigned gt, hipStream_t st, const T 
     }
 }
 
-// dot_slot >= 0 (finest level, tiled kernel, EPI_KU or EPI_JACOBI only): also leave u.out (K*u) or
-// r.out (Jacobi) in pw.scal[dot_slot] and return true; otherwise return false.
+// dot_slot >= 0 (finest level, EPI_KU or EPI_JACOBI only): where the kernel can (the tiled one, the one-launch
+// element matrices), also leave u.out (K*u) or r.out (Jacobi) in pw.scal[dot_slot] and return true; otherwise
+// return false.
 template <typename T>
 bool Solver::kbyu_level(int i, const T *u, T *out, int epi, const T *rr, const T *dg, int dot_slot, T *xout) {
     bool dotted = false;
@@ -815,10 +816,20 @@ bool Solver::kbyu_level(int i, const T *u, T *out, int epi, const T *rr, const T
         const T *Km = f64 ? (const T *)(packed ? D.Ks64p.p : D.Ks64.p) : (const T *)D.Ks32.p;
         if (packed && elem_one_launch(D)) {
             const unsigned gn = grid_for(D.g.nodes(), KN_NODES);
+            if (i == 0 && dot_slot >= 0 && (epi == EPI_KU || epi == EPI_JACOBI)) {
+                if ((int64_t)dotp.n < (int64_t)gn) dotp.alloc(gn);
+                if (epi == EPI_KU)
+                    k_kelem_node<T, EPI_KU, true, true><<<gn, 8 * KN_NODES, 0, st>>>(u, out, Km, D.ldk, D.eleMask, D.nodeMask, D.g, rr, dg, w, xout, dotp);
+                else
+                    k_kelem_node<T, EPI_JACOBI, true, true><<<gn, 8 * KN_NODES, 0, st>>>(u, out, Km, D.ldk, D.eleMask, D.nodeMask, D.g, rr, dg, w, xout, dotp);
+                TG_LAUNCH_CHECK("tg_solver:kbyu");
+                finish_dot(dotp, (int)gn, dot_slot);
+                return true;
+            }
 #define TG_NODE_CASE(EPI)                                                                                        \
     case EPI:                                                                                                    \
-        if (i == 0) k_kelem_node<T, EPI, true><<<gn, 8 * KN_NODES, 0, st>>>(u, out, Km, D.ldk, D.eleMask, D.nodeMask, D.g, rr, dg, w, xout); \
-        else k_kelem_node<T, EPI, false><<<gn, 8 * KN_NODES, 0, st>>>(u, out, Km, D.ldk, D.eleMask, D.nodeMask, D.g, rr, dg, w, xout); \
+        if (i == 0) k_kelem_node<T, EPI, true><<<gn, 8 * KN_NODES, 0, st>>>(u, out, Km, D.ldk, D.eleMask, D.nodeMask, D.g, rr, dg, w, xout, nullptr); \
+        else k_kelem_node<T, EPI, false><<<gn, 8 * KN_NODES, 0, st>>>(u, out, Km, D.ldk, D.eleMask, D.nodeMask, D.g, rr, dg, w, xout, nullptr); \
         break;
             switch (epi) {
                 TG_NODE_CASE(EPI_KU) TG_NODE_CASE(EPI_RESID) TG_NODE_CASE(EPI_JACOBI) TG_NODE_CASE(EPI_RESID_JAC0)
