@@ -69,7 +69,9 @@ struct CoarseSolver {
     bool pers_built = false, pers_ok = false;
     int pers_nk = 0, pers_groups = 0, pers_stages = 0, pers_L1 = 0, pers_L2 = 0;
     DevBuf<unsigned char> pers_table;        // the stage table (device copy)
-    DevBuf<int> pers_err;                    // set when a stage gave up waiting for its input
+    // set when a stage gave up waiting for its input: pinned host memory that the host looks at once the stream has
+    // finished (a copy from the device took 25 us of every call), and its device address
+    int *pers_err = nullptr, *d_pers_err = nullptr;
     bool pers_pending = false;               // launched since the last flag check
 
     ~CoarseSolver();

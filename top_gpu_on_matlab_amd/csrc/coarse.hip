@@ -766,9 +766,9 @@ __device__ __forceinline__ void coh_store(double *p, double v) {
 // the error flag is read too: once any wait of the launch has given up, every other one ends at once.
 __device__ __forceinline__ bool give_up(unsigned polls, int *err, unsigned max_polls) {
     if (polls <= max_polls &&
-        ((polls & 63) != 0 || __hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0))
+        ((polls & 63) != 0 || __hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM) == 0))
         return false;
-    __hip_atomic_store(err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     return true;
 }
 // The value at p (bits: as it was last read) once an earlier stage has written it.
@@ -959,6 +959,7 @@ __global__ void k_unpack_planes(const double *__restrict__ b, T *__restrict__ f,
 
 CoarseSolver::~CoarseSolver() {
     if (exec) (void)hipGraphExecDestroy(exec);
+    if (pers_err) (void)hipHostFree(pers_err);
 }
 
 void CoarseSolver::setup(const HostLevel &L, const Grid &grid, hipStream_t st) {
@@ -1317,9 +1318,12 @@ void CoarseSolver::build_persistent(hipStream_t st) {
     std::vector<unsigned char> bytes(tab.size() * sizeof(PStage));
     std::memcpy(bytes.data(), tab.data(), bytes.size());
     pers_table.upload(bytes, st);
-    pers_err.alloc(1);
-    pers_err.zero(st);
+    if (!pers_err) {
+        TG_HIP(hipHostMalloc((void **)&pers_err, sizeof(int), hipHostMallocMapped | hipHostMallocCoherent), id);
+        TG_HIP(hipHostGetDevicePointer((void **)&d_pers_err, pers_err, 0), id);
+    }
     TG_HIP(hipStreamSynchronize(st), id);
+    *pers_err = 0;
     pers_pending = false;
     pers_nk = nk;
     pers_groups = G;
@@ -1338,10 +1342,10 @@ void CoarseSolver::enqueue_persistent(hipStream_t st, double *x64, float *x32) {
 #define TG_PERS_CASE(K)                                                                                   \
     case K:                                                                                               \
         if (pers_streaming)                                                                                \
-            k_coarse_persistent<K, true><<<pers_groups, PERS_THREADS, lds, st>>>(tab, pers_stages, pers_L2, pers_err.p, \
+            k_coarse_persistent<K, true><<<pers_groups, PERS_THREADS, lds, st>>>(tab, pers_stages, pers_L2, d_pers_err, \
                                                                         pers_polls, o);                     \
         else                                                                                              \
-            k_coarse_persistent<K, false><<<pers_groups, PERS_THREADS, lds, st>>>(tab, pers_stages, pers_L2, pers_err.p, \
+            k_coarse_persistent<K, false><<<pers_groups, PERS_THREADS, lds, st>>>(tab, pers_stages, pers_L2, d_pers_err, \
                                                                          pers_polls, o);                    \
         break;
         TG_PERS_CASE(1) TG_PERS_CASE(2) TG_PERS_CASE(3) TG_PERS_CASE(4) TG_PERS_CASE(5) TG_PERS_CASE(6)
@@ -1357,13 +1361,10 @@ void CoarseSolver::enqueue_persistent(hipStream_t st, double *x64, float *x32) {
 void CoarseSolver::check_barrier(hipStream_t st) {
     if (!pers_pending) return;
     const char *id = "tg_solver:coarse";
-    int e = 0;
-    TG_HIP(hipMemcpyAsync(&e, pers_err.p, sizeof(int), hipMemcpyDeviceToHost, st), id);
     TG_HIP(hipStreamSynchronize(st), id);
     pers_pending = false;
-    if (e) {
-        pers_err.zero(st);
-        TG_HIP(hipStreamSynchronize(st), id);
+    if (__atomic_load_n(pers_err, __ATOMIC_ACQUIRE)) {
+        *pers_err = 0;
         fail(TG_ERR_HIP, id, "coarsest-level solve: a stage of the persistent launch timed out waiting for its input");
     }
 }

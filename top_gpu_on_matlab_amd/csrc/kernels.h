@@ -700,15 +700,16 @@ __global__ void k_convert(const A *__restrict__ a, B *__restrict__ b, int64_t n)
     if (i < n) b[i] = (B)a[i];
 }
 
-// compressed interleaved (reference order) -> full grid; nodFull0 = 0-based full index per solid node
+// compressed interleaved (reference order) -> full grid, zero at inactive nodes; nodFwd = 1-based compressed index per
+// full-grid node (0: inactive).  One launch, where clearing the vector takes two and the scatter a third (15 us of a
+// call at 24 x 48 x 24, 38 at 128 x 256 x 128).
 template <typename A, typename B>
-__global__ void k_unpack(const A *__restrict__ c, B *__restrict__ f, const int32_t *__restrict__ nodFull0, int64_t Nn) {
-    const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= Nn) return;
-    const int64_t n = nodFull0[k];
-    f[3 * n] = (B)c[3 * k];
-    f[3 * n + 1] = (B)c[3 * k + 1];
-    f[3 * n + 2] = (B)c[3 * k + 2];
+__global__ void k_unpack(const A *__restrict__ c, B *__restrict__ f, const int32_t *__restrict__ nodFwd, int64_t nodes) {
+    const int64_t n = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (n >= nodes) return;
+    const int64_t k = (int64_t)nodFwd[n] - 1;
+#pragma unroll
+    for (int d = 0; d < 3; ++d) f[3 * n + d] = k >= 0 ? (B)c[3 * k + d] : (B)0;
 }
 
 template <typename A, typename B>

@@ -149,12 +149,6 @@ struct PcgWork {
         k_reduce_final<<<1, RED_THREADS, 0, st>>>(partial, RED_BLOCKS, scal, slot, d_hscal);
         TG_LAUNCH_CHECK("tg_pcg:dot");
     }
-    // A scalar the stream's last final reduction into slot also left in pinned host memory (dot, or the
-    // residual norm of the update), once the stream has finished.
-    double read(int slot) {
-        TG_HIP(hipStreamSynchronize(st), "tg_pcg");
-        return h_scal[slot];
-    }
     // r.r of the update: reduced with a publish number, which the host polls in pinned memory (no
     // stream synchronisation in the loop).  The stream is queried now and then, so a device error, or
     // a stream that finished without publishing, ends the wait.
@@ -184,8 +178,8 @@ struct PcgWork {
     template <class AtX, class PtV>
     void run(AtX atx, PtV ptv, const double *b, double *y, double tol, int maxIT, bool warm, int *its_out,
              double *res_out, const char *id) {
-        dot(b, b, S_BB);
-        const double normB = std::sqrt(read(S_BB));
+        dot(b, b, S_BB);  // in host memory long before the first residual norm, which needs it
+        double normB = 0;
         if (warm) {
             atx(y, v.p, -1);
             k_sub<<<grid_for(n, 256), 256, 0, st>>>(b, v, r, n);
@@ -240,7 +234,9 @@ struct PcgWork {
             }
             reduce_rr();
             TG_LAUNCH_CHECK(id);
-            res = std::sqrt(wait_rr()) / normB;
+            const double rr = wait_rr();
+            if (its == 1) normB = std::sqrt(h_scal[S_BB]);
+            res = std::sqrt(rr) / normB;
             if (!std::isfinite(res)) fail(TG_ERR_NUMERIC, id, "non-finite residual at iteration %d", its);
             if (res < tol) {
                 k_pcg_axpy<<<grid_for(n, 256), 256, 0, st>>>(y, p, n, scal, sx1, S_PV);

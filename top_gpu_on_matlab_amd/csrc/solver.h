@@ -15,6 +15,7 @@ struct DevLevel {
     int64_t Nn = 0, Ne = 0, ldk = 0;       // ldk: entry stride of element matrices (padded element count)
     DevBuf<uint8_t> nodeMask, eleMask;
     DevBuf<int32_t> nodFull0, eleFull0;    // solid node / element -> 0-based full-grid index
+    DevBuf<int32_t> nodFwd;                // full-grid node -> 1-based solid node (0: none)
     DevBuf<double> idiag64;                // finest level, FP64: 1 / the diagonal entry of a node's free DOFs (tiled K*u)
     DevBuf<double> diag64, r64, x64, t64;  // Jacobi diagonal and V-cycle vectors (full grid, interleaved)
     DevBuf<float> diag32, r32, x32, t32;

@@ -378,6 +378,7 @@ Solver::Solver(const tg_model &m, hipStream_t s) : model(m), st(s) {
         D.nodeMask.upload(mask, st);
         D.eleMask.upload(H.solid, st);
         D.nodFull0.upload(nf, st);
+        D.nodFwd.upload(H.nodMapForward, st);
         D.eleFull0.upload(ef, st);
         const int64_t nv = 3 * D.g.nodes();
         D.diag64.alloc(nv);
@@ -1029,10 +1030,9 @@ void Solver::pcg(const double *b_c, double *y_c, double tol, int maxIT, int warm
     if (!assembled) fail(TG_ERR_STATE, id, "assemble before solving");
     DevLevel &F = lv[0];
     TG_HIP(hipEventRecord(ev0, st), id);
-    b.zero(st);
-    k_unpack<double, double><<<grid_for(F.Nn, 256), 256, 0, st>>>(b_c, b, F.nodFull0, F.Nn);
-    y.zero(st);
-    if (warm) k_unpack<double, double><<<grid_for(F.Nn, 256), 256, 0, st>>>(y_c, y, F.nodFull0, F.Nn);
+    k_unpack<double, double><<<grid_for(F.g.nodes(), 256), 256, 0, st>>>(b_c, b, F.nodFwd, F.g.nodes());
+    if (warm) k_unpack<double, double><<<grid_for(F.g.nodes(), 256), 256, 0, st>>>(y_c, y, F.nodFwd, F.g.nodes());
+    else y.zero(st);
     TG_LAUNCH_CHECK(id);
     int its = 0;
     double res = 0;
@@ -1118,8 +1118,7 @@ int tg_solver_kbyu(tg_solver *s, int32_t level, const double *d_u, double *d_y) 
         if (!S.assembled) fail(TG_ERR_STATE, "tg_solver_kbyu:State", "assemble first");
         if (!d_u || !d_y) fail(TG_ERR_ARGS, id, "null vector");
         DevLevel &D = S.lv[i];
-        D.x64.zero(S.st);
-        k_unpack<double, double><<<grid_for(D.Nn, 256), 256, 0, S.st>>>(d_u, D.x64, D.nodFull0, D.Nn);
+        k_unpack<double, double><<<grid_for(D.g.nodes(), 256), 256, 0, S.st>>>(d_u, D.x64, D.nodFwd, D.g.nodes());
         S.kbyu_level<double>(i, D.x64, D.t64, EPI_KU, nullptr, nullptr);
         k_pack<double, double><<<grid_for(D.Nn, 256), 256, 0, S.st>>>(D.t64, d_y, D.nodFull0, D.Nn);
         TG_LAUNCH_CHECK(id);
@@ -1133,8 +1132,7 @@ int tg_solver_vcycle(tg_solver *s, const double *d_r, double *d_z) {
         Solver &S = S_of(s, id);
         if (!S.assembled) fail(TG_ERR_STATE, "tg_solver_vcycle:State", "assemble first");
         DevLevel &F = S.lv[0];
-        S.pw.r.zero(S.st);
-        k_unpack<double, double><<<grid_for(F.Nn, 256), 256, 0, S.st>>>(d_r, S.pw.r, F.nodFull0, F.Nn);
+        k_unpack<double, double><<<grid_for(F.g.nodes(), 256), 256, 0, S.st>>>(d_r, S.pw.r, F.nodFwd, F.g.nodes());
         S.vcycle(S.pw.r, S.pw.z);
         k_pack<double, double><<<grid_for(F.Nn, 256), 256, 0, S.st>>>(S.pw.z, d_z, F.nodFull0, F.Nn);
         TG_LAUNCH_CHECK(id);
@@ -1150,8 +1148,7 @@ int tg_solver_restrict(tg_solver *s, int32_t coarse_level, const double *d_rf, d
         const int c = level_index(S, coarse_level, id);
         if (c < 1) fail(TG_ERR_ARGS, id, "coarse_level must be >= 2");
         DevLevel &C = S.lv[c], &F = S.lv[c - 1];
-        F.t64.zero(S.st);
-        k_unpack<double, double><<<grid_for(F.Nn, 256), 256, 0, S.st>>>(d_rf, F.t64, F.nodFull0, F.Nn);
+        k_unpack<double, double><<<grid_for(F.g.nodes(), 256), 256, 0, S.st>>>(d_rf, F.t64, F.nodFwd, F.g.nodes());
         S.restrict_level<double>(c, F.t64, C.r64);
         k_pack<double, double><<<grid_for(C.Nn, 256), 256, 0, S.st>>>(C.r64, d_rc, C.nodFull0, C.Nn);
         TG_LAUNCH_CHECK(id);
@@ -1166,8 +1163,7 @@ int tg_solver_interpolate(tg_solver *s, int32_t coarse_level, const double *d_xc
         const int c = level_index(S, coarse_level, id);
         if (c < 1) fail(TG_ERR_ARGS, id, "coarse_level must be >= 2");
         DevLevel &C = S.lv[c], &F = S.lv[c - 1];
-        C.x64.zero(S.st);
-        k_unpack<double, double><<<grid_for(C.Nn, 256), 256, 0, S.st>>>(d_xc, C.x64, C.nodFull0, C.Nn);
+        k_unpack<double, double><<<grid_for(C.g.nodes(), 256), 256, 0, S.st>>>(d_xc, C.x64, C.nodFwd, C.g.nodes());
         S.prolong_level<double>(c, C.x64, F.t64, false);
         k_pack<double, double><<<grid_for(F.Nn, 256), 256, 0, S.st>>>(F.t64, d_xf, F.nodFull0, F.Nn);
         TG_LAUNCH_CHECK(id);
@@ -1181,8 +1177,7 @@ int tg_solver_coarse_solve(tg_solver *s, const double *d_r, double *d_x) {
         Solver &S = S_of(s, id);
         if (!S.assembled) fail(TG_ERR_STATE, "tg_solver_coarse_solve:State", "assemble first");
         DevLevel &C = S.lv[S.L - 1];
-        C.r64.zero(S.st);
-        k_unpack<double, double><<<grid_for(C.Nn, 256), 256, 0, S.st>>>(d_r, C.r64, C.nodFull0, C.Nn);
+        k_unpack<double, double><<<grid_for(C.g.nodes(), 256), 256, 0, S.st>>>(d_r, C.r64, C.nodFwd, C.g.nodes());
         S.coarse.solve<double>(C.r64, C.x64, C.nodeMask, S.st);
         k_pack<double, double><<<grid_for(C.Nn, 256), 256, 0, S.st>>>(C.x64, d_x, C.nodFull0, C.Nn);
         TG_LAUNCH_CHECK(id);

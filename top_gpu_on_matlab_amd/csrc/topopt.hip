@@ -964,8 +964,7 @@ int tg_solver_unit_compliance(tg_solver *s, const double *d_U, double *d_ce) {
         if (!s || !s->s || !d_U || !d_ce) fail(TG_ERR_ARGS, id, "null argument");
         Solver &S = *s->s;
         DevLevel &F = S.lv[0];
-        S.pw.z.zero(S.st);
-        k_unpack<double, double><<<grid_for(F.Nn, 256), 256, 0, S.st>>>(d_U, S.pw.z, F.nodFull0, F.Nn);
+        k_unpack<double, double><<<grid_for(F.g.nodes(), 256), 256, 0, S.st>>>(d_U, S.pw.z, F.nodFwd, F.g.nodes());
         if (S.super) {
             if (!S.assembled) fail(TG_ERR_STATE, "tg_solver_unit_compliance:State", "assemble first (K_mat)");
             k_unit_compliance_super<<<grid_for(F.Ne, UC_ELEMS), UC_PARTS * UC_ELEMS, 0, S.st>>>(S.pw.z, F.Ks64, F.ldk, F.eleFull0, F.Ne, F.g, d_ce);
@@ -1015,8 +1014,7 @@ int tg_compliance_grad(tg_solver *s, tg_filter *f, const double *d_x, double Emi
         S.pcg(S.adjF, d_U, tol, max_it, warm, &its, &res);
         // ce_e = u_e' K0 u_e, c = sum E_e ce_e, g = -p (E0 - Emin) xPhys^(p-1) ce
         DevLevel &F = S.lv[0];
-        S.pw.z.zero(st);
-        k_unpack<double, double><<<grid_for(F.Nn, 256), 256, 0, st>>>(d_U, S.pw.z, F.nodFull0, F.Nn);
+        k_unpack<double, double><<<grid_for(F.g.nodes(), 256), 256, 0, st>>>(d_U, S.pw.z, F.nodFwd, F.g.nodes());
         k_unit_compliance<<<grid_for(Ne, 256), 256, 0, st>>>(S.pw.z, S.K0_64, F.eleFull0, Ne, F.g, S.adjCe);
         TG_LAUNCH_CHECK(id);
         *c_out = reduce_dev(R_DOT, S.adjE, S.adjCe, Ne, st);
@@ -1041,8 +1039,7 @@ int tg_solver_subvoxel_energy(tg_solver *s, const double *d_U, double *d_dc) {
         Solver &S = *s->s;
         if (!S.super) fail(TG_ERR_STATE, id, "super-element mode only");
         DevLevel &F = S.lv[0];
-        S.pw.z.zero(S.st);
-        k_unpack<double, double><<<grid_for(F.Nn, 256), 256, 0, S.st>>>(d_U, S.pw.z, F.nodFull0, F.Nn);
+        k_unpack<double, double><<<grid_for(F.g.nodes(), 256), 256, 0, S.st>>>(d_U, S.pw.z, F.nodFwd, F.g.nodes());
         k_subvoxel_energy<<<grid_for(F.Ne, 16), 256, 0, S.st>>>(S.pw.z, S.Imat, F.eleFull0, F.Ne, F.g, d_dc);
         TG_LAUNCH_CHECK(id);
         TG_HIP(hipStreamSynchronize(S.st), id);
