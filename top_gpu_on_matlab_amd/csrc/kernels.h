@@ -440,19 +440,19 @@ __device__ __forceinline__ int xcd_contiguous(int b, int n) {
 // (S+1)^3 fine nodes; coeff is transferMatCoeffi per fine grid node, a count of at most 8 non-empty
 // coarse elements (1 where unused), stored as one byte and converted exactly to T.
 // Element-centric and LDS-tiled, the trilinear weights applied in separable order.  A
-// workgroup owns RT_E x RT_E coarse elements (y, x) over RT_Z coarse layers and marches through the
+// workgroup owns RT_E x RT_E coarse elements (y, x) over a few coarse layers and marches through the
 // fine node planes of that box: each plane of v = r_f ./ coeff is staged in LDS (the next one is
 // prefetched into registers), every lane forms, for its (element, vertex column (jy, jx), component),
 // the 2D trilinear sum over the element's (S+1)^2 fine nodes of the plane, and folds it into the
 // vertex's two z weights.  When a coarse layer is complete the lane writes its part of the element's
 // 8-vertex contributions C_e (entry-major f[(3 j + c) * ldk + e]); k_kelem_gather then sums them per
 // coarse node over the non-empty elements, which is r_c = P^T r_f.
-constexpr int RT_E = 8, RT_Z = 2;
+constexpr int RT_E = 8;
 constexpr int RT_THREADS = RT_E * RT_E * 12;  // one lane per (element, vertex column, component)
 template <typename T, int S>
 __global__ __launch_bounds__(RT_THREADS) void k_restrict_tiled(const T *__restrict__ rf, const uint8_t *__restrict__ coeff,
                                                                const Grid gc, const Grid gf, T *__restrict__ f,
-                                                               int64_t ldk) {
+                                                               int64_t ldk, int layers) {
     constexpr int FN = RT_E * S + 1;                      // fine nodes per tile side
     constexpr int NV = 3 * FN * FN;                       // staged values per plane
     constexpr int NI = (NV + RT_THREADS - 1) / RT_THREADS;  // staged values per lane
@@ -462,8 +462,8 @@ __global__ __launch_bounds__(RT_THREADS) void k_restrict_tiled(const T *__restri
     int bid = xcd_contiguous((int)blockIdx.x, (int)gridDim.x);
     const int tz = bid / (tilesY * tilesX);
     bid -= tz * tilesY * tilesX;
-    const int e0y = (bid % tilesY) * RT_E, e0x = (bid / tilesY) * RT_E, e0z = tz * RT_Z;
-    const int ez1 = min(e0z + RT_Z, gc.EZ);
+    const int e0y = (bid % tilesY) * RT_E, e0x = (bid / tilesY) * RT_E, e0z = tz * layers;
+    const int ez1 = min(e0z + layers, gc.EZ);
     const int64_t NYX = (int64_t)gf.NY * gf.NX;
     // this lane's output: component, vertex column (jy, jx), element (ly, lx) of the tile
     const int oc = t % 3, q = t / 3, jy = q & 1, jx = (q >> 1) & 1, el = q >> 2;

@@ -88,6 +88,7 @@ struct Solver {
     bool fine_tiled() const { return !super && kfine_kernel == 0 && walsh_ok; }
     // Element-matrix products small enough for the one-launch form (k_kelem_node).
     int64_t node_elems = 1 << 14;
+    int cus = 0;  // compute units of the device
     // restriction in one launch (k_restrict_node) on coarse grids up to this many elements
     int64_t restrict_elems = 1 << 12;
     bool elem_one_launch(const DevLevel &D) const { return D.ldk <= node_elems; }

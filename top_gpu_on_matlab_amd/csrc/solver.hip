@@ -420,7 +420,7 @@ Solver::Solver(const tg_model &m, hipStream_t s) : model(m), st(s) {
         }
     }
     DevLevel &F = lv[0];
-    int dev = 0, cus = 0;
+    int dev = 0;
     TG_HIP(hipGetDevice(&dev), id);
     TG_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev), id);
     for (int v = 0; v < 2; ++v) kfine_auto[v] = kfine_chunk_for(F.g, 3 + v, std::max(cus, 1));
@@ -873,10 +873,18 @@ void Solver::restrict_level(int c, const T *rf, T *rc, const PlanePack *pk) {
         return;
     }
     T *fv = sizeof(T) == 8 ? (T *)C.fv64.p : (T *)C.fv32.p;
-    const unsigned gt = (unsigned)(((C.g.EY + RT_E - 1) / RT_E) * ((C.g.EX + RT_E - 1) / RT_E) *
-                                   ((C.g.EZ + RT_Z - 1) / RT_Z));
-    if (C.span == 4) k_restrict_tiled<T, 4><<<gt, RT_THREADS, 0, st>>>(rf, cf, C.g, F.g, fv, C.ldk);
-    else k_restrict_tiled<T, 2><<<gt, RT_THREADS, 0, st>>>(rf, cf, C.g, F.g, fv, C.ldk);
+    const int64_t tiles = (int64_t)((C.g.EY + RT_E - 1) / RT_E) * ((C.g.EX + RT_E - 1) / RT_E);
+    // Coarse layers per workgroup: one if that leaves at most one workgroup per CU, else two, or four in FP64 (FP32: from
+    // two workgroups per CU on) where two are still more.  Fewer share the fine planes out over more CUs, more read the
+    // planes between layers once.  With 1, 2, 4 layers, us, FP64: 64 x 128 x 64 11.6, 17.7, 30.1 (128 workgroups with
+    // one layer); 96 x 192 x 96 23.2, 20.7, 32.4 (432); 128 x 256 x 128 46.1, 41.6, 38.4 (1,024); FP32: 8.8, 13.2, 21.4;
+    // 14.2, 14.4, 22.9; 25.8, 22.4, 24.6.
+    int layers = 1;
+    while (layers < 4 && tiles * ((C.g.EZ + layers - 1) / layers) > (sizeof(T) == 8 || layers == 1 ? 1 : 2) * (int64_t)cus)
+        layers *= 2;
+    const unsigned gt = (unsigned)(tiles * ((C.g.EZ + layers - 1) / layers));
+    if (C.span == 4) k_restrict_tiled<T, 4><<<gt, RT_THREADS, 0, st>>>(rf, cf, C.g, F.g, fv, C.ldk, layers);
+    else k_restrict_tiled<T, 2><<<gt, RT_THREADS, 0, st>>>(rf, cf, C.g, F.g, fv, C.ldk, layers);
     k_kelem_gather<T, EPI_KU, false><<<gather_grid(C.g), 256, 0, st>>>(
         fv, C.ldk, rc, nullptr, C.eleMask, C.nodeMask, C.g, nullptr, nullptr, (T)0, pk ? *pk : PlanePack{});
     TG_LAUNCH_CHECK("tg_solver:restrict");
