@@ -331,7 +331,9 @@ int tg_compliance_grad(tg_solver *s, tg_filter *f, const double *d_x, double Emi
                        double *d_dcdx, int32_t *its_out);
 
 /* Super-element density filter: imfilter with the cone max(0, r - |d|) on the num-times refined box,
- * zero boundary (TOP_GPU.m:112-121, 220-227, 262-265); arrays are [num^3 x Ne] element-major. */
+ * zero boundary (TOP_GPU.m:112-121, 220-227, 262-265); arrays are [num^3 x Ne] element-major.  forward and adjoint
+ * enqueue one launch on the handle's stream and change nothing in the handle, so they may be called from several
+ * threads and captured; the output must not overlap the input. */
 typedef struct tg_convfilter tg_convfilter;
 int tg_convfilter_create(int32_t nelx, int32_t nely, int32_t nelz, double rMin_subvoxels, int32_t num, void *stream,
                          tg_convfilter **out);

@@ -138,6 +138,63 @@ def test_convolution_filter_reach_and_edges(r, dims, num):
     assert np.array_equal(np.isnan(grid(gf.forward(_t(x)).cpu().numpy())), hit)
 
 
+@pytest.mark.parametrize('r', [3.5, 13.2])
+def test_convolution_filter_calls_overlap_on_one_handle(r):
+    """A call leaves nothing in the handle that another one could pick up: four threads calling one handle, each with
+    inputs of its own, and a captured call replayed on a second stream beside them, get bit for bit what they
+    get alone."""
+    import ctypes
+    import threading
+    import torch
+    from top_gpu_on_matlab_amd import top_gpu as G
+    from top_gpu_on_matlab_amd._lib import check, lib
+    nelx, nely, nelz, num = 7, 9, 5, 4
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        gf = G.ConvolutionFilter(nelx, nely, nelz, r, num)
+    n = num ** 3 * nelx * nely * nelz
+    gen = torch.Generator().manual_seed(9)
+    x = [torch.rand(n, dtype=torch.float64, generator=gen).cuda() for _ in range(5)]
+    call = [lib().tg_convfilter_forward, lib().tg_convfilter_adjoint]
+    out = [[torch.zeros_like(a) for _ in range(20)] for a in x]
+    torch.cuda.synchronize()
+
+    def run(t, k):
+        check(call[t % 2](gf.h, ctypes.c_void_p(x[t].data_ptr()), ctypes.c_void_p(out[t][k].data_ptr())))
+    alone = []
+    for t in range(5):
+        run(t, 0)
+        torch.cuda.synchronize()
+        alone.append(out[t][0].clone())
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        run(4, 0)
+    for t in range(5):
+        out[t][0].zero_()
+    other = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    gate = threading.Barrier(5)
+
+    def worker(t):
+        gate.wait()
+        for k in range(20):
+            run(t, k)
+    threads = [threading.Thread(target=worker, args=(t,)) for t in range(4)]
+    for th in threads:
+        th.start()
+    gate.wait()
+    with torch.cuda.stream(other):
+        for k in range(20):
+            graph.replay()
+            out[4][k].copy_(out[4][0])
+    for th in threads:
+        th.join()
+    torch.cuda.synchronize()
+    for t in range(5):
+        for k in range(20):
+            assert torch.equal(out[t][k], alone[t]), (t, k)
+
+
 def test_oc_update_matches_bisection():
     from top_gpu_on_matlab_amd import top_gpu as G
     rng = np.random.default_rng(3)

@@ -27,7 +27,7 @@ struct Filter {
 struct ConvFilter {
     int num, X = 0, Y = 0, Z = 0, GY = 0, GX = 0, GZ = 0, hr = 0;
     hipStream_t st;
-    DevBuf<double> hd, Hs, tmp;  // weights (one octant), their sums on the grid, the input in grid order
+    DevBuf<double> hd, Hs;       // weights (one octant), their sums on the grid
     DevBuf<int32_t> lim;         // last dy with a weight, per (dx, dz)
     int LY = 0, LX = 0, pitch = 0;  // lanes along y and x of k_conv's workgroups, LDS column stride (LY = 0: k_conv_any)
     ConvFilter(int nelx, int nely, int nelz, double r, int n, hipStream_t s);

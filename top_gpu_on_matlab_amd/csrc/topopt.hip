@@ -637,8 +637,9 @@ __device__ inline int64_t cv_new_index(int iy, int ix, int iz, int num, int Y, i
     return loc + (int64_t)num * num * num * big;
 }
 
-// out[p] = sum_q h(q) * in(p + q - c) on a zero-padded grid (imfilter, 'same', bcF = 0), the input on the grid
-// (k_conv_in).
+// out[p] = sum_q h(q) * in(p + q - c) on a zero-padded grid (imfilter, 'same', bcF = 0), in = src, for the adjoint
+// src ./ Hs, or ones for Hs itself, read where the caller has it: a call leaves nothing in the handle, so calls on one
+// handle may overlap (threads, replays of a captured call).
 // MODE 0: out = result ./ Hs  (forward: xPhys = imfilter(x)./Hs)   MODE 1: out = result  (adjoint: imfilter(dc./Hs))
 // MODE 2: out = result on the grid  (Hs = imfilter(1))
 template <int MODE>
@@ -650,20 +651,19 @@ __device__ __forceinline__ void conv_store(double *__restrict__ out, const doubl
     else out[p] = s;
 }
 
-// The convolution's input in grid order: src (element-major), for the adjoint ./ Hs, or ones for Hs itself.
-template <int MODE>
-__global__ void k_conv_in(const double *__restrict__ src, const double *__restrict__ Hs, int GY, int GX, int GZ, int num,
-                          int Y, int X, double *__restrict__ in) {
-    const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= (int64_t)GY * GX * GZ) return;
-    if (MODE == 2) {
-        in[p] = 1.0;
-        return;
+// cv_new_index is a sum of one term per axis; this is that term of one axis, voxel by voxel (loc: between voxels of an
+// element, big: between elements).
+struct CvAxis {
+    int64_t off, loc, skip;
+    int rem, num;
+    __device__ CvAxis(int i, int n, int64_t l, int64_t big)
+        : off(i / n * big + i % n * l), loc(l), skip(big - (n - 1) * l), rem(i % n), num(n) {}
+    __device__ void next() {
+        const bool last = ++rem == num;
+        off += last ? skip : loc;
+        rem = last ? 0 : rem;
     }
-    const int iy = (int)(p % GY), ix = (int)((p / GY) % GX), iz = (int)(p / ((int64_t)GY * GX));
-    const double v = src[cv_new_index(iy, ix, iz, num, Y, X)];
-    in[p] = MODE == 1 ? v / Hs[p] : v;
-}
+};
 
 // Cones of up to CONV_HR voxels' reach.  The cone is even in each direction: the planes z - dz and z + dz are added
 // as they are staged, which halves the products.  A workgroup has LY x LX blocks of CONV_Y voxels along y in
@@ -671,12 +671,12 @@ __global__ void k_conv_in(const double *__restrict__ src, const double *__restri
 // wide and the narrow discs of the ball fall together), each with a plane of its own in LDS and no barrier but
 // for the sum at the end.  Per row (dx, dz) of the cone a lane reads CONV_Y + 2 HR values of a column into registers
 // for up to CONV_Y (2 HR + 1) products, over the taps with a weight only (lim: the last such dy, uniform).
-// Bound by LDS reads and FP64 products together: 62 us for the 40 x 240 x 40 sub-voxels of a 10 x 60 x 10 beam at
-// a reach of 6 (and 3 for the input), against 670 (forward) and 930 (adjoint) with a thread per voxel that
-// walked the whole cube and found each tap's address by division.
+// Bound by LDS reads and FP64 products together: 56 us (forward) and 67 (adjoint, which divides every value as it stages
+// it) for the 40 x 240 x 40 sub-voxels of a 10 x 60 x 10 beam at a reach of 6, against 670 and 930 with a thread per
+// voxel that walked the whole cube and found each tap's address by division.
 constexpr int CONV_Y = 8, CONV_HR = 12;
 template <int HR, int MODE>
-__global__ __launch_bounds__(256) void k_conv(const double *__restrict__ in, const double *__restrict__ Hs,
+__global__ __launch_bounds__(256) void k_conv(const double *__restrict__ src, const double *__restrict__ Hs,
                                               const double *__restrict__ h, const int32_t *__restrict__ lim, int GY, int GX,
                                               int GZ, int num, int Y, int X, int LY, int LX, int pitch,
                                               double *__restrict__ out) {
@@ -695,17 +695,26 @@ __global__ __launch_bounds__(256) void k_conv(const double *__restrict__ in, con
         if (4 * k > HR) break;
         if (dz > HR) continue;
         const int zl = iz - dz, zh = iz + dz;
-        const bool okl = zl >= 0 && zl < GZ, okh = dz > 0 && zh < GZ;
-        for (int xx = 0; xx < cols; ++xx) {
-            const int x = x0 - HR + xx;
-            const bool okx = (unsigned)x < (unsigned)GX;
-            for (int yy = lane; yy < rows; yy += 64) {
-                const int y = y0 - HR + yy;
+        const bool okl = zl >= 0, okh = dz > 0 && zh < GZ;
+        const int64_t n3 = (int64_t)num * num * num, layer = n3 * Y * X;
+        const double *sl = src + (okl ? CvAxis(zl, num, num * num, layer).off : 0);
+        const double *sh = src + (okh ? CvAxis(zh, num, num * num, layer).off : 0);
+        const double *Hl = Hs + (int64_t)GY * GX * (okl ? zl : 0), *Hh = Hs + (int64_t)GY * GX * (okh ? zh : 0);
+        for (int yy = lane; yy < rows; yy += 64) {
+            const int y = y0 - HR + yy;
+            const bool oky = (unsigned)y < (unsigned)GY;
+            const CvAxis ay(oky ? y : 0, num, 1, n3);
+            CvAxis ax(max(x0 - HR, 0), num, num, n3 * Y);
+            for (int xx = 0; xx < cols; ++xx) {
+                const int x = x0 - HR + xx;
                 double v = 0.0;
-                if (okx && (unsigned)y < (unsigned)GY) {
-                    const int64_t p = y + (int64_t)GY * x;
-                    if (okl) v = in[p + (int64_t)GY * GX * zl];
-                    if (okh) v += in[p + (int64_t)GY * GX * zh];
+                if ((unsigned)x < (unsigned)GX) {
+                    if (oky) {
+                        const int64_t at = ax.off + ay.off, p = y + (int64_t)GY * x;
+                        if (okl) v = MODE == 2 ? 1.0 : MODE == 1 ? sl[at] / Hl[p] : sl[at];
+                        if (okh) v += MODE == 2 ? 1.0 : MODE == 1 ? sh[at] / Hh[p] : sh[at];
+                    }
+                    ax.next();
                 }
                 plane[xx * pitch + yy] = v;
             }
@@ -751,18 +760,27 @@ __global__ __launch_bounds__(256) void k_conv(const double *__restrict__ in, con
 
 // Any reach: one thread per voxel.  h: the (hr + 1)^3 weights of the cone's even octant.
 template <int MODE>
-__global__ void k_conv_any(const double *__restrict__ in, const double *__restrict__ Hs, const double *__restrict__ h, int hr,
+__global__ void k_conv_any(const double *__restrict__ src, const double *__restrict__ Hs, const double *__restrict__ h, int hr,
                            int GY, int GX, int GZ, int num, int Y, int X, double *__restrict__ out) {
     const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (p >= (int64_t)GY * GX * GZ) return;
     const int iy = (int)(p % GY), ix = (int)((p / GY) % GX), iz = (int)(p / ((int64_t)GY * GX));
+    const int64_t n3 = (int64_t)num * num * num;
+    const CvAxis ay0(max(iy - hr, 0), num, 1, n3), ax0(max(ix - hr, 0), num, num, n3 * Y);
+    CvAxis az(max(iz - hr, 0), num, num * num, n3 * Y * X);
     double s = 0;
-    for (int z = max(iz - hr, 0); z <= min(iz + hr, GZ - 1); ++z)
-        for (int x = max(ix - hr, 0); x <= min(ix + hr, GX - 1); ++x)
-            for (int y = max(iy - hr, 0); y <= min(iy + hr, GY - 1); ++y) {
+    for (int z = max(iz - hr, 0); z <= min(iz + hr, GZ - 1); ++z, az.next()) {
+        CvAxis ax = ax0;
+        for (int x = max(ix - hr, 0); x <= min(ix + hr, GX - 1); ++x, ax.next()) {
+            CvAxis ay = ay0;
+            for (int y = max(iy - hr, 0); y <= min(iy + hr, GY - 1); ++y, ay.next()) {
                 const double hv = h[abs(y - iy) + (int64_t)(hr + 1) * (abs(x - ix) + (int64_t)(hr + 1) * abs(z - iz))];
-                if (hv != 0.0) s += hv * in[y + (int64_t)GY * (x + (int64_t)GX * z)];
+                if (hv == 0.0) continue;
+                const double v = MODE == 2 ? 1.0 : src[az.off + ax.off + ay.off];
+                s += hv * (MODE == 1 ? v / Hs[y + (int64_t)GY * (x + (int64_t)GX * z)] : v);
             }
+        }
+    }
     conv_store<MODE>(out, Hs, iy, ix, iz, GY, GX, num, Y, X, s);
 }
 
@@ -910,7 +928,6 @@ ConvFilter::ConvFilter(int nelx, int nely, int nelz, double r, int n, hipStream_
     lim.upload(last, st);
     const int64_t ng = (int64_t)GY * GX * GZ;
     Hs.alloc(ng);
-    tmp.alloc(ng);
     // lanes along y and x of a workgroup's plane: the least (products + staging) over the grid that fits the LDS
     LY = 0;
     double least = 1e300;
@@ -935,16 +952,15 @@ ConvFilter::ConvFilter(int nelx, int nely, int nelz, double r, int n, hipStream_
 template <int MODE>
 void ConvFilter::convolve(const double *src, double *out) {
     const int64_t ng = (int64_t)GY * GX * GZ;
-    k_conv_in<MODE><<<grid_for(ng, 256), 256, 0, st>>>(src, Hs, GY, GX, GZ, num, Y, X, tmp);
     const size_t lds = std::max(4 * (size_t)(LX + 2 * hr) * pitch, (size_t)4 * CONV_Y * 64) * sizeof(double);
     const dim3 grid(grid_for(GY, CONV_Y * std::max(LY, 1)) * grid_for(GX, std::max(LX, 1)), (unsigned)GZ);
     switch (LY ? hr : -1) {
 #define TG_CONV_CASE(H) \
-    case H: k_conv<H, MODE><<<grid, 256, lds, st>>>(tmp, Hs, hd, lim, GY, GX, GZ, num, Y, X, LY, LX, pitch, out); break;
+    case H: k_conv<H, MODE><<<grid, 256, lds, st>>>(src, Hs, hd, lim, GY, GX, GZ, num, Y, X, LY, LX, pitch, out); break;
         TG_CONV_CASE(0) TG_CONV_CASE(1) TG_CONV_CASE(2) TG_CONV_CASE(3) TG_CONV_CASE(4) TG_CONV_CASE(5) TG_CONV_CASE(6)
         TG_CONV_CASE(7) TG_CONV_CASE(8) TG_CONV_CASE(9) TG_CONV_CASE(10) TG_CONV_CASE(11) TG_CONV_CASE(12)
 #undef TG_CONV_CASE
-        default: k_conv_any<MODE><<<grid_for(ng, 256), 256, 0, st>>>(tmp, Hs, hd, hr, GY, GX, GZ, num, Y, X, out);
+        default: k_conv_any<MODE><<<grid_for(ng, 256), 256, 0, st>>>(src, Hs, hd, hr, GY, GX, GZ, num, Y, X, out);
     }
     TG_LAUNCH_CHECK("tg_convfilter:convolve");
 }
