@@ -306,7 +306,8 @@ int tg_reduce(int32_t op, const double *d_a, const double *d_b, int64_t n, doubl
  * nonzero entry where xnew is held at 1 in every bisection step (TOP_GPU.m:239, 247; in super-element
  * mode the caller marks sub-voxel row 4 of each passive element, as xnew(Num_, passiveElements) does).
  * Writes d_xnew, *change = max|xnew - x|, *bisections = steps run (a multiple of 16; trailing steps are
- * no-ops).  Synchronises. */
+ * no-ops).  TG_ERR_NUMERIC where the bisection does not end (a volume that the move limits cannot reach): d_xnew
+ * then holds what it held.  Synchronises. */
 int tg_oc_update(const double *d_x, const double *d_dc, const double *d_dv, const double *d_passive, int64_t n,
                  double fval, double move, double *d_xnew, double *change, int32_t *bisections, void *stream);
 

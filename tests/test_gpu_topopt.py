@@ -252,6 +252,41 @@ def test_oc_update_step_by_step(n, passive, scale):
         assert took.value == 16 * -(-steps // 16)
 
 
+@pytest.mark.parametrize('n', [1, 257, 40000])
+@pytest.mark.parametrize('fval, scale', [(-0.9, 1e-2), (float('nan'), 1e-2), (-0.02, 1e-240), (-0.02, 1e-100)])
+def test_oc_update_that_cannot_end_leaves_the_output(n, fval, scale):
+    """A volume that the move limits cannot reach, one that is not a number and multipliers below any that the steps get to:
+    refused, and the output holds what it held, beside the inputs and in place of one.  Multipliers of
+    1e-100 are reached, after some 360 steps; the update is then the one of the same steps one by one."""
+    import ctypes
+    from top_gpu_on_matlab_amd._lib import lib
+    rng = np.random.default_rng(n)
+    x, dc, dv = 0.3 + 0.1 * rng.random(n), -(0.5 + rng.random(n)) * scale, 0.5 + rng.random(n)
+    l1, l2, move, steps = 0.0, 1e9, 0.2, 0
+    while (l2 - l1) / (l1 + l2) > 1e-6 and steps < 416:
+        lmid = 0.5 * (l2 + l1)
+        xnew = np.maximum(0, np.maximum(x - move, np.minimum(1, np.minimum(x + move, x * np.sqrt(-dc / dv / lmid)))))
+        steps += 1
+        if fval + np.mean(xnew - x) > 0:
+            l1 = lmid
+        else:
+            l2 = lmid
+    ends = steps < 416
+    assert ends == (scale == 1e-100)
+    for out in ('out', 'dv'):
+        d = {k: _t(v) for k, v in dict(x=x, dc=dc, dv=dv, out=np.arange(n) + 0.5).items()}
+        held = d[out].clone()
+        ptr = lambda k: ctypes.c_void_p(d[k].data_ptr())
+        took = ctypes.c_int32(-1)
+        rc = lib().tg_oc_update(ptr('x'), ptr('dc'), ptr('dv'), None, n, fval, move, ptr(out), None, ctypes.byref(took), None)
+        if ends:
+            assert rc == 0 and took.value == 16 * -(-steps // 16)
+            assert _rel(d[out].cpu().numpy(), xnew) < 1e-14
+        else:
+            assert rc == 6 and took.value == -1
+            assert bool((d[out] == held).all())
+
+
 @pytest.mark.parametrize('cfg', [
     dict(shape=(8, 16, 8), case=1, ft=1, nLoop=6, se=False),
     dict(shape=(8, 16, 8), case=1, ft=2, nLoop=6, se=False),

@@ -240,16 +240,24 @@ __device__ inline double oc_xnew(double x, double dc, double dv, double lmid, do
 // The bisection on the multiplier, OC_DEPTH steps a launch.  From a bracket (l1, l2) those steps can meet
 // 2^OC_DEPTH - 1 midpoints, a binary tree (node 1 the middle; from node m to 2 m + 1 where gt > 0, l1 = mid, else to
 // 2 m): every launch sums xnew - x for all of them over one pass of the data, and the next launch's workgroups each
-// walk the tree with the finished sums, to the bracket that the same steps one by one would reach.  The pass
-// reads x and b = x sqrt(-dc / dv) (formed by the first one, kept in xnew until that is written), so a midpoint costs
-// a product with 1 / sqrt(mid) and the clamps; k_oc_apply evaluates the update itself at the last midpoint.
+// walk the tree with the finished sums, to the bracket that the same steps one by one would reach.  A pass needs x and
+// b = x sqrt(-dc / dv), so a midpoint costs a product with 1 / sqrt(mid) and the clamps; k_oc_apply evaluates the update
+// itself at the last midpoint.
+// b is kept in xnew until that is written, but only where the bisection is known to end: a call that fails leaves
+// the caller's array as it was.  The bracket closes within 19 steps of the first gt > 0, and gt does not increase with
+// the multiplier (nor do its rounded sums, in one fixed order), so gt > 0 at OC_FLOOR, the midpoint that is reached after 397
+// steps of l1 = 0, says that it closes within the 416 steps there are.  The first pass sums for OC_FLOOR too, the
+// second one decides and writes b (at 4.2 million entries 35 and 40 us, the later ones 30); where it may not (or the
+// caller's arrays overlap), every pass forms b itself.
 // passive (may be null): entries with a nonzero indicator take xnew = 1 inside every step, so
 // they enter gt (xnew(passiveElements) = 1.0, TOP_GPU.m:239, 247).
 // Bound by the passes' two streams on large designs and by launches on small ones: 16 passes for 64 steps, 30 us each
 // at 4.2 million entries and 11 at 27,648, against 64 pairs of launches of 21 and 6 us.
 constexpr int OC_DEPTH = 4, OC_NODES = (1 << OC_DEPTH) - 1, OC_BLOCKS = 512;
+constexpr double OC_FLOOR = 1e9 * 0x1p-397;
 struct OcState {
     double l1, l2, lmid, steps;  // bracket, the last executed step's midpoint, steps executed
+    double keep;                 // whether xnew holds b
 };
 
 // The state after the steps that the sums decide; sums[m - 1]: node m's sum of xnew - x.
@@ -267,37 +275,41 @@ __device__ inline OcState oc_walk(OcState s, const double *sums, double fval, do
 }
 
 // old: the state that the previous launch's sums (partial_in, nb rows) refine; now: where the result goes.
-template <bool FIRST>
+// PASS: 0 the first, 1 the second, 2 any later one.  b (may be null): where b may be kept.
+template <int PASS>
 __global__ __launch_bounds__(RED_THREADS) void k_oc_pass(const double *__restrict__ x, const double *__restrict__ dc,
                                                          const double *__restrict__ dv, double *__restrict__ b,
                                                          const double *__restrict__ passive, int64_t n, double fval,
                                                          double move, const OcState *__restrict__ old,
                                                          OcState *__restrict__ now, const double *__restrict__ partial_in,
                                                          double *__restrict__ partial_out) {
-    __shared__ double sh[4][OC_NODES], sums[OC_NODES], scale[OC_NODES];
+    constexpr int NIN = OC_NODES + (PASS == 1), NOUT = OC_NODES + (PASS == 0);  // the last of them: OC_FLOOR's
+    __shared__ double sh[4][OC_NODES + 1], sums[OC_NODES + 1], scale[OC_NODES + 1];
     __shared__ OcState st;
     const int t = threadIdx.x, lane = t & 63, w = t >> 6, nb = gridDim.x;
-    auto reduce = [&](double (&v)[OC_NODES]) {  // over the workgroup, in a fixed order; in sums
+    auto reduce = [&](double *v, int count) {  // over the workgroup, in a fixed order; in sums
 #pragma unroll
-        for (int k = 0; k < OC_NODES; ++k) {
-            for (int o = 32; o > 0; o >>= 1) v[k] += __shfl_down(v[k], o, 64);
-            if (lane == 0) sh[w][k] = v[k];
-        }
+        for (int k = 0; k < OC_NODES + 1; ++k)
+            if (k < count) {
+                for (int o = 32; o > 0; o >>= 1) v[k] += __shfl_down(v[k], o, 64);
+                if (lane == 0) sh[w][k] = v[k];
+            }
         __syncthreads();
-        if (t < OC_NODES) sums[t] = (sh[0][t] + sh[1][t]) + (sh[2][t] + sh[3][t]);
+        if (t < count) sums[t] = (sh[0][t] + sh[1][t]) + (sh[2][t] + sh[3][t]);
         __syncthreads();
     };
-    double acc[OC_NODES];
+    double acc[OC_NODES + 1];
 #pragma unroll
-    for (int k = 0; k < OC_NODES; ++k) acc[k] = 0.0;
-    if (!FIRST) {
+    for (int k = 0; k < OC_NODES + 1; ++k) acc[k] = 0.0;
+    if (PASS > 0) {
         for (int r = t; r < nb; r += RED_THREADS)
 #pragma unroll
-            for (int k = 0; k < OC_NODES; ++k) acc[k] += partial_in[(int64_t)k * nb + r];
-        reduce(acc);
+            for (int k = 0; k < NIN; ++k) acc[k] += partial_in[(int64_t)k * nb + r];
+        reduce(acc, NIN);
     }
     if (t == 0) {
-        st = FIRST ? OcState{0.0, 1e9, 0.0, 0.0} : oc_walk(*old, sums, fval, (double)n);
+        st = PASS == 0 ? OcState{0.0, 1e9, 0.0, 0.0, 0.0} : oc_walk(*old, sums, fval, (double)n);
+        if (PASS == 1) st.keep = b && fval + sums[OC_NODES] / (double)n > 0 ? 1.0 : 0.0;
         if (blockIdx.x == 0) *now = st;
     }
     __syncthreads();
@@ -311,32 +323,33 @@ __global__ __launch_bounds__(RED_THREADS) void k_oc_pass(const double *__restric
             else l2 = mid;
         }
         scale[t] = 1.0 / sqrt(0.5 * (l2 + l1));
+    } else if (t == OC_NODES) {
+        scale[t] = 1.0 / sqrt(OC_FLOOR);
     }
     __syncthreads();
-    double sc[OC_NODES];
+    double sc[NOUT];
 #pragma unroll
-    for (int k = 0; k < OC_NODES; ++k) {
+    for (int k = 0; k < NOUT; ++k) {
         sc[k] = scale[k];
         acc[k] = 0.0;
     }
     const int64_t stride = (int64_t)nb * RED_THREADS;
+    auto sweep = [&](auto root) {  // root(i, x): b of entry i
 #pragma unroll 2
-    for (int64_t i = (int64_t)blockIdx.x * RED_THREADS + t; i < n; i += stride) {
-        const double xi = x[i];
-        double bi;
-        if (FIRST) {
-            bi = xi * sqrt(-dc[i] / dv[i]);
-            b[i] = bi;
-        } else {
-            bi = b[i];
-        }
-        double lo = fmax(0.0, xi - move), hi = fmin(1.0, xi + move);
-        if (passive && passive[i] != 0.0) lo = hi = 1.0;
+        for (int64_t i = (int64_t)blockIdx.x * RED_THREADS + t; i < n; i += stride) {
+            const double xi = x[i], bi = root(i, xi);
+            double lo = fmax(0.0, xi - move), hi = fmin(1.0, xi + move);
+            if (passive && passive[i] != 0.0) lo = hi = 1.0;
 #pragma unroll
-        for (int k = 0; k < OC_NODES; ++k) acc[k] += fmax(lo, fmin(hi, bi * sc[k])) - xi;
-    }
-    reduce(acc);
-    if (t < OC_NODES) partial_out[(int64_t)t * nb + blockIdx.x] = sums[t];
+            for (int k = 0; k < NOUT; ++k) acc[k] += fmax(lo, fmin(hi, bi * sc[k])) - xi;
+        }
+    };
+    auto form = [&](int64_t i, double xi) { return xi * sqrt(-dc[i] / dv[i]); };
+    if (PASS == 0 || st.keep == 0.0) sweep(form);
+    else if (PASS == 1) sweep([&](int64_t i, double xi) { return b[i] = form(i, xi); });
+    else sweep([&](int64_t i, double) { return b[i]; });
+    reduce(acc, NOUT);
+    if (t < NOUT) partial_out[(int64_t)t * nb + blockIdx.x] = sums[t];
 }
 
 // The state after the last pass, for the host's check (and the apply's midpoint).
@@ -789,7 +802,9 @@ __global__ void k_conv_any(const double *__restrict__ src, const double *__restr
 // ---------------------------------------------------------------------------------------------
 namespace {
 
-static_assert((size_t)2 * OC_NODES * OC_BLOCKS + RED_BLOCKS + 16 <= SCRATCH_DOUBLES, "the OC update's working memory");
+static_assert(2 * sizeof(OcState) <= 16 * sizeof(double) && RED_BLOCKS <= 2 * (OC_NODES + 1) * OC_BLOCKS &&
+                  (size_t)2 * (OC_NODES + 1) * OC_BLOCKS + 16 <= SCRATCH_DOUBLES,
+              "the OC update's working memory");
 
 // Sum, dot, maximum or sharpness of device arrays on st, to the host.
 double reduce_dev(int op, const double *a, const double *b, int64_t n, hipStream_t st) {
@@ -1109,26 +1124,29 @@ int tg_oc_update(const double *d_x, const double *d_dc, const double *d_dv, cons
         if (!d_x || !d_dc || !d_dv || !d_xnew || n < 1) fail(TG_ERR_ARGS, id, "bad arguments");
         hipStream_t st = (hipStream_t)stream;
         const int nb = (int)std::min<int64_t>(OC_BLOCKS, (n + RED_THREADS - 1) / RED_THREADS);
-        // b goes to xnew until that is written, unless the caller's arrays overlap
         auto apart = [&](const double *a) { return !a || a + n <= d_xnew || d_xnew + n <= a; };
-        DevBuf<double> own(apart(d_x) && apart(d_dc) && apart(d_dv) && apart(d_passive) ? 0 : n);
-        double *b = own.n ? own.p : d_xnew;
+        double *b = apart(d_x) && apart(d_dc) && apart(d_dv) && apart(d_passive) ? d_xnew : nullptr;
         Scratch sc(st);
-        OcState *state = (OcState *)sc.dbl();  // 16 doubles, then the sums of two launches, then the maxima
-        double *part[2] = {sc.dbl() + 16, sc.dbl() + 16 + (size_t)OC_NODES * nb}, *maxima = sc.dbl() + 16 + (size_t)2 * OC_NODES * nb;
+        // 16 doubles of states, then the sums of two launches, whose place the maxima take after the last one
+        OcState *state = (OcState *)sc.dbl();
+        double *part[2] = {sc.dbl() + 16, sc.dbl() + 16 + (size_t)(OC_NODES + 1) * nb}, *maxima = part[0];
         int k = 0;  // launches; launch k's sums are in part[k & 1], and it left the state before them in state[k & 1]
-        OcState s{0.0, 1e9, 0.0, 0.0};
+        OcState s{0.0, 1e9, 0.0, 0.0, 0.0};
         // (l2-l1)/(l1+l2) halves each step from 1: at most ~100 steps, more than 48 but for the largest
         // multipliers; check after 48, then every 16
         for (int upto = 48; ; upto += 16) {
             for (; OC_DEPTH * k < upto; ++k) {
+                const OcState *old = state + ((k + 1) & 1);
+                const double *in = part[(k + 1) & 1];
                 if (k == 0)
-                    k_oc_pass<true><<<nb, RED_THREADS, 0, st>>>(d_x, d_dc, d_dv, b, d_passive, n, fval, move, nullptr, state,
-                                                                nullptr, part[0]);
+                    k_oc_pass<0><<<nb, RED_THREADS, 0, st>>>(d_x, d_dc, d_dv, b, d_passive, n, fval, move, nullptr, state,
+                                                             nullptr, part[0]);
+                else if (k == 1)
+                    k_oc_pass<1><<<nb, RED_THREADS, 0, st>>>(d_x, d_dc, d_dv, b, d_passive, n, fval, move, old, state + 1, in,
+                                                             part[1]);
                 else
-                    k_oc_pass<false><<<nb, RED_THREADS, 0, st>>>(d_x, d_dc, d_dv, b, d_passive, n, fval, move,
-                                                                 state + ((k - 1) & 1), state + (k & 1), part[(k - 1) & 1],
-                                                                 part[k & 1]);
+                    k_oc_pass<2><<<nb, RED_THREADS, 0, st>>>(d_x, d_dc, d_dv, b, d_passive, n, fval, move, old,
+                                                             state + (k & 1), in, part[k & 1]);
             }
             const unsigned long long seq = sc.next();
             k_oc_close<<<1, RED_THREADS, 0, st>>>(n, fval, state + ((k - 1) & 1), state + (k & 1), part[(k - 1) & 1], nb,
