@@ -372,6 +372,8 @@ __device__ __forceinline__ void tri_block(int b, int &I, int &J) {
     while ((I + 1) * (I + 2) / 2 <= b) ++I;
     J = b - I * (I + 1) / 2;
 }
+// Doubles of a plane's blocks, nb block rows of the lower triangle.
+__host__ __device__ __forceinline__ int64_t tri_size(int64_t nb) { return nb * (nb + 1) / 2 * (CB * CB); }
 __device__ __forceinline__ double *tri_tiles(double *W, int I, int J) {
     return W + ((int64_t)I * (I + 1) / 2 + J) * (CB * CB);
 }
@@ -1050,7 +1052,7 @@ void CoarseSolver::setup(const HostLevel &L, const Grid &grid, hipStream_t st) {
     Bop.alloc(std::max<int64_t>(bOff[P], 1));
     Fop.zero(st);  // row padding stays zero
     Bop.zero(st);
-    W.alloc(maxpad > CB ? 4 * maxpad * maxpad : 1);
+    W.alloc(maxpad > CB ? 4 * tri_size(maxpad / CB) : 1);
     Dk.alloc(4 * CB * CB);
     bb.alloc(std::max<int64_t>(ntot, 1));
     yy.alloc(std::max<int64_t>(ntot, 1));
@@ -1102,7 +1104,7 @@ void CoarseSolver::factor(const double *Ks, int64_t ldk, const uint8_t *eleMask,
         const int pl[2] = {p, q};
         for (int y = 0; y < 2; ++y) {
             if (!has(pl[y])) continue;
-            pr[y] = SweepProb{S_of(pl[y]), W.p + 2 * y * maxpad * maxpad, W.p + (2 * y + 1) * maxpad * maxpad,
+            pr[y] = SweepProb{S_of(pl[y]), W.p + 2 * y * tri_size(maxpad / CB), W.p + (2 * y + 1) * tri_size(maxpad / CB),
                               npad[pl[y]], (int)(npad[pl[y]] / CB), Dk.p + 2 * y * CB * CB, info.p + pl[y]};
             nbmax = std::max(nbmax, pr[y].nb);
         }
