@@ -138,6 +138,29 @@ def test_convolution_filter_reach_and_edges(r, dims, num):
     assert np.array_equal(np.isnan(grid(gf.forward(_t(x)).cpu().numpy())), hit)
 
 
+@pytest.mark.parametrize('dims, num', [((2, 330, 1), 1), ((1, 90, 2), 3), ((70, 1, 2), 2), ((3, 33, 20), 1)])
+def test_convolution_filter_long_reach(dims, num):
+    """A reach of 110 voxels, where a column comes in several segments of 256, on grids that are a few voxels thin in
+    one direction or two, against scipy's zero-padded correlation with the part of the cone that falls on them."""
+    import scipy.ndimage
+    from top_gpu_on_matlab_amd import top_gpu as G
+    nelx, nely, nelz = dims
+    r = 110.5
+    gf = G.ConvolutionFilter(nelx, nely, nelz, r, num)
+    shape = (num * nely, num * nelx, num * nelz)
+    v = [np.arange(-min(110, k - 1), min(110, k - 1) + 1) for k in shape]
+    dy, dx, dz = np.meshgrid(*v, indexing='ij')
+    h = np.maximum(0.0, r - np.sqrt(dx ** 2 + dy ** 2 + dz ** 2))
+    conv = lambda a: scipy.ndimage.correlate(a, h, mode='constant', cval=0.0)
+    def grid(vec):  # element-major -> [y, x, z]
+        a = vec.reshape(nelz, nelx, nely, num, num, num).transpose(2, 5, 1, 4, 0, 3)
+        return np.ascontiguousarray(a.reshape(shape))
+    x = np.random.default_rng(6).random(num ** 3 * nelx * nely * nelz)
+    Hs = conv(np.ones(shape))
+    assert _rel(grid(gf.forward(_t(x)).cpu().numpy()), conv(grid(x)) / Hs) < 1e-12
+    assert _rel(grid(gf.adjoint(_t(x)).cpu().numpy()), conv(grid(x) / Hs)) < 1e-12
+
+
 @pytest.mark.parametrize('r', [3.5, 13.2])
 def test_convolution_filter_calls_overlap_on_one_handle(r):
     """A call leaves nothing in the handle that another one could pick up: four threads calling one handle, each with

@@ -771,30 +771,60 @@ __global__ __launch_bounds__(256) void k_conv(const double *__restrict__ src, co
     }
 }
 
-// Any reach: one thread per voxel.  h: the (hr + 1)^3 weights of the cone's even octant.
+// Any reach.  A thread per voxel, TY x 64 / TY of them along y and x a workgroup of one wavefront (TY: fitted to the grid's
+// y side), which brings the columns along y that they reach into LDS (CONV_COLS at once, CONV_SEG voxels at a time), so
+// a column is read and, for the adjoint, divided once for all of them.  Sums run over z, x, y ascending.  h: the
+// (hr + 1)^3 weights of the cone's even octant.  Bound by a product's two loads, value and weight: 40 x 240 x 40 voxels at
+// a reach of 14, 12,893 weights, forward 2.2 ms, adjoint 2.5, against 5.0 and 6.4 with every value read (and divided)
+// from memory for each product; 32 x 4 x 32 voxels 0.41 and 0.46 ms against 1.9 and 2.1.
+constexpr int CONV_SEG = 256, CONV_COLS = 4;
 template <int MODE>
-__global__ void k_conv_any(const double *__restrict__ src, const double *__restrict__ Hs, const double *__restrict__ h, int hr,
-                           int GY, int GX, int GZ, int num, int Y, int X, double *__restrict__ out) {
-    const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= (int64_t)GY * GX * GZ) return;
-    const int iy = (int)(p % GY), ix = (int)((p / GY) % GX), iz = (int)(p / ((int64_t)GY * GX));
+__global__ __launch_bounds__(64) void k_conv_any(const double *__restrict__ src, const double *__restrict__ Hs,
+                                                 const double *__restrict__ h, const int32_t *__restrict__ lim, int hr, int GY,
+                                                 int GX, int GZ, int num, int Y, int X, int TY, double *__restrict__ out) {
+    __shared__ double col[CONV_COLS][CONV_SEG];
+    const int t = threadIdx.x, TX = 64 / TY, W = hr + 1;
+    const int tilesY = (GY + TY - 1) / TY, tilesX = (GX + TX - 1) / TX;
+    const unsigned tile = blockIdx.x / tilesY;
+    const int y0 = (int)(blockIdx.x % tilesY) * TY, x0 = (int)(tile % tilesX) * TX, iz = (int)(tile / tilesX);
+    const int iy = y0 + t % TY, ix = x0 + t / TY;
+    const int ya = max(y0 - hr, 0), yb = min(y0 + TY + hr, GY), xa = max(x0 - hr, 0), xb = min(x0 + TX + hr, GX);
     const int64_t n3 = (int64_t)num * num * num;
-    const CvAxis ay0(max(iy - hr, 0), num, 1, n3), ax0(max(ix - hr, 0), num, num, n3 * Y);
     CvAxis az(max(iz - hr, 0), num, num * num, n3 * Y * X);
     double s = 0;
     for (int z = max(iz - hr, 0); z <= min(iz + hr, GZ - 1); ++z, az.next()) {
-        CvAxis ax = ax0;
-        for (int x = max(ix - hr, 0); x <= min(ix + hr, GX - 1); ++x, ax.next()) {
-            CvAxis ay = ay0;
-            for (int y = max(iy - hr, 0); y <= min(iy + hr, GY - 1); ++y, ay.next()) {
-                const double hv = h[abs(y - iy) + (int64_t)(hr + 1) * (abs(x - ix) + (int64_t)(hr + 1) * abs(z - iz))];
-                if (hv == 0.0) continue;
-                const double v = MODE == 2 ? 1.0 : src[az.off + ax.off + ay.off];
-                s += hv * (MODE == 1 ? v / Hs[y + (int64_t)GY * (x + (int64_t)GX * z)] : v);
+        const int dz = abs(z - iz);
+        CvAxis ax(xa, num, num, n3 * Y);
+        for (int xc = xa; xc < xb; xc += CONV_COLS) {
+            int64_t off[CONV_COLS];
+#pragma unroll
+            for (int c = 0; c < CONV_COLS; ++c, ax.next()) off[c] = az.off + (xc + c < xb ? ax.off : 0);
+            for (int ys = ya; ys < yb; ys += CONV_SEG) {
+                const int len = min(CONV_SEG, yb - ys);
+                for (int k = t; k < len; k += 64) {
+                    const int64_t oy = CvAxis(ys + k, num, 1, n3).off;
+                    double v[CONV_COLS];
+#pragma unroll
+                    for (int c = 0; c < CONV_COLS; ++c) v[c] = MODE == 2 ? 1.0 : src[off[c] + oy];
+#pragma unroll
+                    for (int c = 0; c < CONV_COLS; ++c) {
+                        if (MODE == 1) v[c] /= Hs[ys + k + (int64_t)GY * ((xc + c < xb ? xc + c : 0) + (int64_t)GX * z)];
+                        col[c][k] = v[c];
+                    }
+                }
+                __syncthreads();
+                for (int x = xc; x < min(xc + CONV_COLS, xb); ++x) {
+                    const int dx = abs(x - ix), last = dx <= hr ? lim[dx + (int64_t)W * dz] : -1;
+                    const double *hx = h + (int64_t)W * (min(dx, hr) + (int64_t)W * dz), *cx = col[x - xc];
+                    const int d1 = min(last, ys + len - 1 - iy);
+#pragma unroll 4
+                    for (int d = max(-last, ys - iy); d <= d1; ++d) s += hx[abs(d)] * cx[iy + d - ys];
+                }
+                __syncthreads();
             }
         }
     }
-    conv_store<MODE>(out, Hs, iy, ix, iz, GY, GX, num, Y, X, s);
+    if (iy < GY && ix < GX) conv_store<MODE>(out, Hs, iy, ix, iz, GY, GX, num, Y, X, s);
 }
 
 }  // namespace
@@ -966,7 +996,6 @@ ConvFilter::ConvFilter(int nelx, int nely, int nelz, double r, int n, hipStream_
 
 template <int MODE>
 void ConvFilter::convolve(const double *src, double *out) {
-    const int64_t ng = (int64_t)GY * GX * GZ;
     const size_t lds = std::max(4 * (size_t)(LX + 2 * hr) * pitch, (size_t)4 * CONV_Y * 64) * sizeof(double);
     const dim3 grid(grid_for(GY, CONV_Y * std::max(LY, 1)) * grid_for(GX, std::max(LX, 1)), (unsigned)GZ);
     switch (LY ? hr : -1) {
@@ -975,7 +1004,12 @@ void ConvFilter::convolve(const double *src, double *out) {
         TG_CONV_CASE(0) TG_CONV_CASE(1) TG_CONV_CASE(2) TG_CONV_CASE(3) TG_CONV_CASE(4) TG_CONV_CASE(5) TG_CONV_CASE(6)
         TG_CONV_CASE(7) TG_CONV_CASE(8) TG_CONV_CASE(9) TG_CONV_CASE(10) TG_CONV_CASE(11) TG_CONV_CASE(12)
 #undef TG_CONV_CASE
-        default: k_conv_any<MODE><<<grid_for(ng, 256), 256, 0, st>>>(src, Hs, hd, hr, GY, GX, GZ, num, Y, X, out);
+        default: {
+            int ty = 64;
+            while (ty > 1 && ty >= 2 * GY) ty /= 2;
+            const unsigned tiles = grid_for(GY, ty) * grid_for(GX, 64 / ty) * (unsigned)GZ;
+            k_conv_any<MODE><<<tiles, 64, 0, st>>>(src, Hs, hd, lim, hr, GY, GX, GZ, num, Y, X, ty, out);
+        }
     }
     TG_LAUNCH_CHECK("tg_convfilter:convolve");
 }
