@@ -132,6 +132,67 @@ def test_assembly_entries_children_and_element_counts(Ne, nCh, dtype):
     assert (abs(_np(g) - out) <= eps * mag).all()
 
 
+@pytest.mark.parametrize('dtype', [np.float64, np.float32])
+@pytest.mark.parametrize('Ne, nCh', [(2048, 3), (2049, 3), (2049, 8), (7200, 8), (7200, 64), (2100, 1)])
+def test_assembly_entries_many_elements(Ne, nCh, dtype):
+    """All three entries with element counts on both sides of the wavefronts' rule and where a wavefront has several
+    tiles of the FP64 level-2 product (past 7,168), with voids and children with boundary matrices, general P: the first and
+    last elements and a sample of the others, entry by entry within the rounding of sums of nCh products of two 24-term
+    sums, of moduli over 64 sub-voxels for super-elements: (nCh + 115) unit roundoffs of the sums over absolute values."""
+    from top_gpu_on_matlab_amd import mex
+    rng = np.random.default_rng(Ne + nCh)
+    nU = 5
+    nF = min(2 * Ne * nCh, 100000)
+    up = np.where(rng.random((Ne, nCh)) < 0.1, 0, rng.integers(1, nF + 1, size=(Ne, nCh))).astype(np.int32)
+    E = rng.random(nF).astype(dtype)
+    K0, P = rng.standard_normal((24, 24)).astype(dtype), rng.standard_normal((24, 24, nCh)).astype(dtype)
+    uid = np.where(rng.random(nF) < 0.2, rng.integers(1, nU + 1, size=nF), 0).astype(np.int32)
+    free, fixed = (rng.standard_normal((576, nU)).astype(dtype) for _ in range(2))
+    prev = rng.standard_normal((24, 24, nF)).astype(dtype)
+    sub = rng.random((64, nF)).astype(dtype)
+    free64 = rng.standard_normal((576, 64, nU)).astype(dtype)
+    some = np.unique(np.concatenate([np.arange(3), np.arange(Ne - 70, Ne), rng.integers(0, Ne, 40)]))
+    f64 = lambda a: a.astype(np.float64)
+    mat = lambda v: v.reshape(24, 24, order='F')
+
+    def higher(f):
+        return f64(prev[:, :, f]), abs(f64(prev[:, :, f]))
+
+    def level2(f):
+        m = float(E[f])
+        if uid[f] == 0:
+            return f64(K0) * m, abs(f64(K0)) * m
+        u, x = mat(f64(free[:, uid[f] - 1])), mat(f64(fixed[:, uid[f] - 1]))
+        return u * m + x, abs(u) * m + abs(x)
+
+    def super_(f):
+        if uid[f] == 0:
+            return higher(f)
+        u, x, m = f64(free64[:, :, uid[f] - 1]), f64(fixed[:, uid[f] - 1]), f64(sub[:, f])
+        return mat(u @ m + x), mat(abs(u) @ m + abs(x))
+
+    dup, dP, duid, dfixed, dprev = _ga(up), _ga(P), _ga(uid), _ga(fixed), _ga(prev)
+    entries = [
+        (level2, lambda g: mex.assembleKs_level2_inplace(g, dup, _ga(E), _ga(K0.reshape(-1, order='F')), dP, duid, _ga(free), dfixed)),
+        (higher, lambda g: mex.assembleKs_higherLevel_inplace(g, dup, dprev, dP)),
+        (super_, lambda g: mex.assembleKs_level2_superEle_inplace(g, dup, dprev, dP, duid, _ga(sub), _ga(free64), dfixed)),
+    ]
+    for child, entry in entries:
+        g = _ga(np.full((24, 24, Ne), np.nan), dtype)
+        entry(g)
+        got = _np(g)
+        assert np.isfinite(got).all()
+        for e in some:
+            out, mag = np.zeros((24, 24)), np.zeros((24, 24))
+            for s in range(nCh):
+                if up[e, s] > 0:
+                    B = f64(P[:, :, s])
+                    K, A = child(up[e, s] - 1)
+                    out += B.T @ K @ B
+                    mag += abs(B).T @ A @ abs(B)
+            assert (abs(got[:, :, e] - out) <= (nCh + 115) * np.finfo(dtype).eps * mag).all(), (child.__name__, e)
+
+
 def test_assemble_super_element_entry():
     from top_gpu_on_matlab_amd import mex
     m = M.build_cuboid_model(10, 20, 10, opt_case=2, super_element=True)

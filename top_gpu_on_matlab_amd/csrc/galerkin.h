@@ -1,17 +1,16 @@
 // Galerkin coarse-stiffness core of the MEX entry points:
 //   Kout = sum_s  B_s^T * Kch_s * B_s      (24 x 24, FP32/FP64)
-// One workgroup per coarse element, its children dealt to the GK_WAVES wavefronts in turn and their sums added in
+// One workgroup per coarse element, its children dealt to its WAVES wavefronts in turn and their sums added in
 // wavefront order; lane t of a wavefront owns the 3x3 block (rows 3*(t%8).., cols 3*(t/8)..) of a product.  B
 // (row-major) and Kch (column-major), then T = Kch*B (row-major), are the wavefront's own LDS, so it never
 // waits for the others.  Every product runs over k = 0..23 in order.  Bound by a child's chain of loads and two
-// products out of LDS: 1,024 elements of 8 children 31 us, from 51 with one wavefront for all of them.
+// products out of LDS where there are few elements (1,024 of 8 children: 31 us, from 51 with one wavefront for all of
+// them), by LDS reads where there are many.
 #pragma once
 
 #include <hip/hip_runtime.h>
 
 namespace tg {
-
-constexpr int GK_WAVES = 4, GK_THREADS = 64 * GK_WAVES;
 
 // LDS written by this wavefront is read by it: the hardware keeps one wavefront's LDS accesses in order, this
 // keeps the compiler's.
@@ -21,25 +20,25 @@ __device__ inline void wave_sync() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-template <typename T>
+template <typename T, int WAVES>
 struct GalerkinLds {
-    T B[GK_WAVES][576], K[GK_WAVES][576];
+    T B[WAVES][576], K[WAVES][576];
 };
 
 // Src must provide:
 //   __device__ int child(int s) const;              // < 0: skip child s
 //   __device__ void kch(int f, int t, T (&k)[9]) const;  // entries 64 j + t (= r + 24c) of the child's matrix
 // ADD: to what Kout holds.
-template <bool ADD, typename T, class Src>
+template <bool ADD, int WAVES, typename T, class Src>
 __device__ inline void galerkin_block(T *__restrict__ Kout, const Src &src, int nCh, const T *__restrict__ P,
-                                      GalerkinLds<T> &lds) {
+                                      GalerkinLds<T, WAVES> &lds) {
     const int t = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int rb = 3 * (t & 7), cb = 3 * (t >> 3);
     T *sB = lds.B[w], *sK = lds.K[w];
     T acc[9];
 #pragma unroll
     for (int i = 0; i < 9; ++i) acc[i] = (T)0;
-    // this wavefront's children: every GK_WAVES-th of those there are, looked up 64 at a time
+    // this wavefront's children: every WAVES-th of those there are, looked up 64 at a time
     int turn = 0, s0 = -64, mine = -1;
     unsigned long long left = 0;
     auto next = [&](int &s, int &f) {
@@ -52,7 +51,7 @@ __device__ inline void galerkin_block(T *__restrict__ Kout, const Src &src, int 
             }
             const int l = __ffsll(left) - 1;
             left &= left - 1;
-            if (turn++ % GK_WAVES != w) continue;
+            if (turn++ % WAVES != w) continue;
             s = s0 + l;
             f = __builtin_amdgcn_readlane(mine, l);
             return true;
@@ -113,10 +112,10 @@ __device__ inline void galerkin_block(T *__restrict__ Kout, const Src &src, int 
 #pragma unroll
     for (int i = 0; i < 9; ++i) sK[64 * i + t] = acc[i];
     __syncthreads();
-    for (int o = threadIdx.x; o < 576; o += GK_THREADS) {  // entry r + 24 c
+    for (int o = threadIdx.x; o < 576; o += 64 * WAVES) {  // entry r + 24 c
         const int r = o % 24, c = o / 24, at = 64 * (3 * (r % 3) + c % 3) + r / 3 + 8 * (c / 3);
         T v = lds.K[0][at];
-        for (int k = 1; k < GK_WAVES; ++k) v += lds.K[k][at];
+        for (int k = 1; k < WAVES; ++k) v += lds.K[k][at];
         Kout[o] = ADD ? Kout[o] + v : v;
     }
 }

@@ -401,24 +401,51 @@ struct SrcSuper {
     }
 };
 
-template <typename T, int MODE>
-__global__ __launch_bounds__(GK_THREADS) void k_galerkin_mex(T *__restrict__ Ks, const int32_t *__restrict__ up,
-                                                             int64_t Ne, int nCh, const T *__restrict__ P,
+template <typename T, int MODE, int WAVES>
+__global__ __launch_bounds__(64 * WAVES) void k_galerkin_mex(T *__restrict__ Ks, const int32_t *__restrict__ up, int64_t Ne,
+                                                             int nCh, const T *__restrict__ P,
                                                              const T *a0, const T *a1, const T *a2, const T *a3,
                                                              const int32_t *mapU, int hasFixed, int64_t nFine,
                                                              int64_t nU) {
-    __shared__ GalerkinLds<T> lds;
+    __shared__ GalerkinLds<T, WAVES> lds;
     const int e = blockIdx.x;
     T *out = Ks + (size_t)e * 576;
     if (MODE == 0) {
         SrcLevel2<T> src{up, Ne, e, a0, a1, a2, a3, mapU, hasFixed != 0, nFine, nU};
-        galerkin_block<false>(out, src, nCh, P, lds);
+        galerkin_block<false, WAVES>(out, src, nCh, P, lds);
     } else if (MODE == 1) {
         SrcHigher<T> src{up, Ne, e, a0, nFine};
-        galerkin_block<false>(out, src, nCh, P, lds);
+        galerkin_block<false, WAVES>(out, src, nCh, P, lds);
     } else {
         SrcSuper<T> src{up, Ne, e, a0, a1, a2, a3, mapU, hasFixed != 0, nFine, nU};
-        galerkin_block<false>(out, src, nCh, P, lds);
+        galerkin_block<false, WAVES>(out, src, nCh, P, lds);
+    }
+}
+
+// Wavefronts per element.  With few elements the chain of one element's children is what bounds a call, and four
+// wavefronts share it; with many the chip is full of elements, and wavefronts whose share of the children is uneven or
+// empty only take LDS from others.  Measured, us, with 1, 2, 4 wavefronts: single, level 2 of 8 children: 200 elements
+// 40, 32, 28; 2,500 58, 54, 60; 20,000 260, 239, 310; of 64: 157, 101, 63; 284, 248, 272; 1704, 1676, 2065; double, the
+// levels above, 8 children: 40, 31, 28; 87, 90, 85; 504, 475, 489; 3 children, 20,000: 201, 220, 243.  Super-elements in
+// double, whose children's sums over 64 sub-voxels fill the registers: 207, 142, 41; 334, 302, 90; 655, 658, 486.
+template <typename T, int MODE>
+int galerkin_waves(int64_t Ne, int nCh) {
+    if (nCh == 1) return 1;
+    if (Ne <= 2048 || (MODE == 2 && sizeof(T) == 8)) return 4;
+    return nCh < 4 ? 1 : 2;
+}
+template <typename T, int MODE>
+void launch_galerkin(hipStream_t st, void *Ks, const void *up, int64_t Ne, int nCh, const void *P, const void *a0,
+                     const void *a1 = nullptr, const void *a2 = nullptr, const void *a3 = nullptr,
+                     const void *mapU = nullptr, int hasFixed = 0, int64_t nFine = 0, int64_t nU = 0) {
+    auto go = [&](auto kernel, int waves) {
+        kernel<<<(unsigned)Ne, 64 * waves, 0, st>>>((T *)Ks, (const int32_t *)up, Ne, nCh, (const T *)P, (const T *)a0, (const T *)a1,
+                                                    (const T *)a2, (const T *)a3, (const int32_t *)mapU, hasFixed, nFine, nU);
+    };
+    switch (galerkin_waves<T, MODE>(Ne, nCh)) {
+        case 1: go(k_galerkin_mex<T, MODE, 1>, 1); break;
+        case 2: go(k_galerkin_mex<T, MODE, 2>, 2); break;
+        default: go(k_galerkin_mex<T, MODE, 4>, 4);
     }
 }
 
@@ -540,12 +567,13 @@ struct SrcLevel2Bnd : SrcLevel2<double> {
     __device__ void kch(int f, int t, double (&k)[9]) const { unique(mapU[f] - 1, E[f], t, k); }
 };
 
-__global__ __launch_bounds__(GK_THREADS) void k_mex_galerkin_bnd(double *__restrict__ Ks, const int32_t *__restrict__ up,
+constexpr int GB_WAVES = 4;
+__global__ __launch_bounds__(64 * GB_WAVES) void k_mex_galerkin_bnd(double *__restrict__ Ks, const int32_t *__restrict__ up,
                                                                  int64_t Ne, int nCh, const double *__restrict__ P,
                                                                  const double *E, const double *K0, const double *uf,
                                                                  const double *ux, const int32_t *mapU, int64_t nFine,
                                                                  int64_t nU, const int32_t *__restrict__ bnd) {
-    __shared__ GalerkinLds<double> lds;
+    __shared__ GalerkinLds<double, GB_WAVES> lds;
     const int e = blockIdx.x;
     if (!bnd[e]) return;
     SrcLevel2Bnd src;
@@ -560,7 +588,7 @@ __global__ __launch_bounds__(GK_THREADS) void k_mex_galerkin_bnd(double *__restr
     src.hasFixed = true;
     src.nFine = nFine;
     src.nU = nU;
-    galerkin_block<true>(Ks + (size_t)e * 576, src, nCh, P, lds);
+    galerkin_block<true, GB_WAVES>(Ks + (size_t)e * 576, src, nCh, P, lds);
 }
 
 }  // namespace
@@ -695,17 +723,15 @@ int assembleKs_level2_inplace(int nlhs, tg_array *plhs, int nrhs, const tg_array
                 if (nCh == 64) k_mex_galerkin_gemm<16, 4><<<gt, 256, 0, st>>>(Ech, G, (double *)Ks.p, Ne, tiles);
                 else k_mex_galerkin_gemm<2, 4><<<gt, 256, 0, st>>>(Ech, G, (double *)Ks.p, Ne, tiles);
                 if (hasFixed)
-                    k_mex_galerkin_bnd<<<(unsigned)Ne, GK_THREADS, 0, st>>>((double *)Ks.p, (const int32_t *)up.p, Ne, nCh,
+                    k_mex_galerkin_bnd<<<(unsigned)Ne, 64 * GB_WAVES, 0, st>>>((double *)Ks.p, (const int32_t *)up.p, Ne, nCh,
                         (const double *)pch.p, (const double *)em.p, (const double *)k0.p, (const double *)uf.p,
                         (const double *)ux.p, (const int32_t *)mu.p, nFine, nU, bnd);
                 TG_LAUNCH_CHECK(Cu);
                 TG_HIP(hipStreamSynchronize(st), Cu);  // buf is released on leaving the scope
             } else if (cls == TG_DOUBLE)
-                k_galerkin_mex<double, 0><<<(unsigned)Ne, GK_THREADS, 0, st>>>((double *)Ks.p, (const int32_t *)up.p, Ne, nCh, (const double *)pch.p,
-                    (const double *)em.p, (const double *)k0.p, (const double *)uf.p, (const double *)ux.p, (const int32_t *)mu.p, hasFixed, nFine, nU);
+                launch_galerkin<double, 0>(st, Ks.p, up.p, Ne, nCh, pch.p, em.p, k0.p, uf.p, ux.p, mu.p, hasFixed, nFine, nU);
             else
-                k_galerkin_mex<float, 0><<<(unsigned)Ne, GK_THREADS, 0, st>>>((float *)Ks.p, (const int32_t *)up.p, Ne, nCh, (const float *)pch.p,
-                    (const float *)em.p, (const float *)k0.p, (const float *)uf.p, (const float *)ux.p, (const int32_t *)mu.p, hasFixed, nFine, nU);
+                launch_galerkin<float, 0>(st, Ks.p, up.p, Ne, nCh, pch.p, em.p, k0.p, uf.p, ux.p, mu.p, hasFixed, nFine, nU);
             TG_LAUNCH_CHECK(Cu);
         }
         TG_HIP(hipStreamSynchronize(st), Cu);
@@ -733,11 +759,9 @@ int assembleKs_higherLevel_inplace(int nlhs, tg_array *plhs, int nrhs, const tg_
         hipStream_t st = S(stream);
         if (Ne > 0) {
             if (cls == TG_DOUBLE)
-                k_galerkin_mex<double, 1><<<(unsigned)Ne, GK_THREADS, 0, st>>>((double *)Ks.p, (const int32_t *)up.p, Ne, nSub, (const double *)ps.p,
-                    (const double *)prev.p, nullptr, nullptr, nullptr, nullptr, 0, nFine, 0);
+                launch_galerkin<double, 1>(st, Ks.p, up.p, Ne, nSub, ps.p, prev.p, nullptr, nullptr, nullptr, nullptr, 0, nFine, 0);
             else
-                k_galerkin_mex<float, 1><<<(unsigned)Ne, GK_THREADS, 0, st>>>((float *)Ks.p, (const int32_t *)up.p, Ne, nSub, (const float *)ps.p,
-                    (const float *)prev.p, nullptr, nullptr, nullptr, nullptr, 0, nFine, 0);
+                launch_galerkin<float, 1>(st, Ks.p, up.p, Ne, nSub, ps.p, prev.p, nullptr, nullptr, nullptr, nullptr, 0, nFine, 0);
             TG_LAUNCH_CHECK(Cu);
         }
         TG_HIP(hipStreamSynchronize(st), Cu);
@@ -786,11 +810,9 @@ int assembleKs_level2_superEle_inplace(int nlhs, tg_array *plhs, int nrhs, const
         hipStream_t st = S(stream);
         if (Ne > 0) {
             if (cls == TG_DOUBLE)
-                k_galerkin_mex<double, 2><<<(unsigned)Ne, GK_THREADS, 0, st>>>((double *)Ks.p, (const int32_t *)up.p, Ne, nSub, (const double *)ps.p,
-                    (const double *)ks0.p, (const double *)em.p, (const double *)uf.p, (const double *)ux.p, (const int32_t *)mu.p, hasFixed, nFine, nU);
+                launch_galerkin<double, 2>(st, Ks.p, up.p, Ne, nSub, ps.p, ks0.p, em.p, uf.p, ux.p, mu.p, hasFixed, nFine, nU);
             else
-                k_galerkin_mex<float, 2><<<(unsigned)Ne, GK_THREADS, 0, st>>>((float *)Ks.p, (const int32_t *)up.p, Ne, nSub, (const float *)ps.p,
-                    (const float *)ks0.p, (const float *)em.p, (const float *)uf.p, (const float *)ux.p, (const int32_t *)mu.p, hasFixed, nFine, nU);
+                launch_galerkin<float, 2>(st, Ks.p, up.p, Ne, nSub, ps.p, ks0.p, em.p, uf.p, ux.p, mu.p, hasFixed, nFine, nU);
             TG_LAUNCH_CHECK(Cu);
         }
         TG_HIP(hipStreamSynchronize(st), Cu);
