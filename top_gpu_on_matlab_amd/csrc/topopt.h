@@ -29,7 +29,7 @@ struct ConvFilter {
     hipStream_t st;
     DevBuf<double> hd, Hs;       // weights (one octant), their sums on the grid
     DevBuf<int32_t> lim;         // last dy with a weight, per (dx, dz)
-    int LY = 0, LX = 0, pitch = 0;  // lanes along y and x of k_conv's workgroups, LDS column stride (LY = 0: k_conv_any)
+    int LY = 0, LX = 0, pitch = 0;  // lanes along y and x of k_conv's workgroups, LDS column stride (LY = 0: another form)
     ConvFilter(int nelx, int nely, int nelz, double r, int n, hipStream_t s);
     void forward(const double *x, double *out);
     void adjoint(const double *dc, double *out);
