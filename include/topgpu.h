@@ -231,14 +231,15 @@ int tg_solver_time_kbyu(tg_solver *s, int32_t level, int32_t precision, int32_t 
 /* Launch tuning of the finest-level standard-voxel K*u (no reference counterpart: the reference's
  * K*u is a MATLAB pagemtimes, TOP_GPU.m:1729-1741).  Keys:
  *   TG_TUNE_KFINE_KERNEL  0 = element-centric LDS-tiled z-march (default), 1 = node-centric gather
- *   TG_TUNE_KFINE_ZCHUNK  node planes per workgroup of the tiled kernel (1..4096; until set,
- *                         chosen by the grid so that the chip is filled)
+ *   TG_TUNE_KFINE_ZCHUNK  node planes per workgroup of the tiled kernel: 1..4096, or 0 (default) =
+ *                         chosen by the grid so that the chip is filled
  *   TG_TUNE_TIME_KFINE    1 = bracket every tiled finest K*u launch with HIP events, 2 = only the
  *                         plain products (the PCG operator), 0 = stop; 1 and 2 clear the record
  *   TG_TUNE_KELEM_PARTS   threads per element of the FP64 per-element-matrix K*u (coarse levels and
  *                         the super-element finest level): 1 (default) = the packed upper triangles of
- *                         the symmetric element matrices, 300 of 576 entries; 4, 6, 8, 12 or 24 = the
- *                         full matrices, split over that many threads; the FP32 V-cycle's product is
+ *                         the symmetric element matrices, 300 of 576 entries, one thread per element or,
+ *                         up to 16,384 elements, one per node and element around it; 4, 6, 8, 12 or 24 =
+ *                         the full matrices, split over that many threads; the FP32 V-cycle's product is
  *                         always the packed one
  *   TG_TUNE_COARSE_GRAPH  1 = replay the coarsest solve's step-by-step launch sequence as a captured
  *                         HIP graph, 0 = launch it kernel by kernel (measured 1% faster per PCG iteration)

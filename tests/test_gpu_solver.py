@@ -459,6 +459,30 @@ def test_finest_product_chunk_chosen_by_grid(shape):
     assert torch.equal(out[0][1], out[1][1])
 
 
+def test_finest_product_chunk_can_be_given_back():
+    """A chunk of the finest product that was set can be given back to the grid's choice: 48 x 96 x 48 elements have more
+    planes than any grid's chunk here, so a chunk of all 49 planes is several times slower (few workgroups)
+    and the time tells which one runs; the values are the same either way."""
+    import torch
+    from top_gpu_on_matlab_amd._lib import TopGpuError
+    from top_gpu_on_matlab_amd.model import cuboid_model
+    from top_gpu_on_matlab_amd.solver import Solver
+    s = Solver(cuboid_model(48, 96, 48, 1, precision='fp64'))
+    s.set_modulus(np.ones(s.model.num_elements))
+    s.assemble()
+    u = torch.rand(s.ndof(), generator=torch.Generator().manual_seed(1), dtype=torch.float64).cuda()
+    ref = s.kbyu(u)
+    ms = []
+    for zchunk in (49, 0):
+        s.set_tuning(kfine_zchunk=zchunk)
+        assert torch.equal(s.kbyu(u), ref)
+        ms.append(min(s.time_kbyu(1, reps=20) for _ in range(5)))
+    assert ms[1] < 0.6 * ms[0]
+    for bad in (-1, 4097):
+        with pytest.raises(TopGpuError):
+            s.set_tuning(kfine_zchunk=bad)
+
+
 @pytest.mark.parametrize('shape, blocks', [((24, 48, 24), 1), ((32, 48, 32), 2), ((56, 64, 56), 3), ((56, 64, 64), 4),
                                            ((128, 136, 128), 14)])
 def test_coarse_factorisation_at_block_edges(shape, blocks):

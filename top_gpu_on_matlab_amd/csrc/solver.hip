@@ -1268,7 +1268,7 @@ int tg_solver_set_tuning(tg_solver *s, int32_t key, int32_t value) {
         const char *id = "tg_solver_set_tuning:Input";
         Solver &S = S_of(s, id);
         if (key == TG_TUNE_KFINE_KERNEL && (value == 0 || value == 1)) S.kfine_kernel = value;
-        else if (key == TG_TUNE_KFINE_ZCHUNK && value >= 1 && value <= 4096) S.kfine_zchunk = value;
+        else if (key == TG_TUNE_KFINE_ZCHUNK && value >= 0 && value <= 4096) S.kfine_zchunk = value;
         else if (key == TG_TUNE_KELEM_PARTS && (value == 1 || value == 4 || value == 6 || value == 8 || value == 12 || value == 24))
             S.kelem_parts = value;
         else if (key == TG_TUNE_COARSE_GRAPH && (value == 0 || value == 1)) S.coarse.use_graph = value != 0;
