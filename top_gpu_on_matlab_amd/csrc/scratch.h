@@ -51,6 +51,7 @@ class Scratch {
         {
             ScratchPool &p = scratch_pool();
             std::lock_guard<std::mutex> lock(p.mu);
+            p.idle[dev].reserve(SCRATCH_KEPT);  // so that giving a block back, in a destructor, allocates nothing
             if (!p.idle[dev].empty()) {
                 b = std::move(p.idle[dev].back());
                 p.idle[dev].pop_back();
