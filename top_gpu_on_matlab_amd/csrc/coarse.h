@@ -67,7 +67,7 @@ struct CoarseSolver {
     bool pers_streaming = true;  // non-temporal loads of the factor rows
     unsigned pers_polls = 1u << 17;  // polls of an input (~1 us apart) before a stage gives up (~0.1 s)
     bool pers_built = false, pers_ok = false;
-    int pers_nk = 0, pers_groups = 0, pers_stages = 0, pers_L1 = 0, pers_L2 = 0;
+    int pers_nk = 0, pers_groups = 0, pers_stages = 0, pers_L2 = 0;
     DevBuf<unsigned char> pers_table;        // the stage table (device copy)
     // set when a stage gave up waiting for its input: pinned host memory that the host looks at once the stream has
     // finished (a copy from the device took 25 us of every call), and its device address

@@ -1330,7 +1330,6 @@ void CoarseSolver::build_persistent(hipStream_t st) {
     pers_nk = nk;
     pers_groups = G;
     pers_stages = (int)tab.size();
-    pers_L1 = (int)L1;
     pers_L2 = (int)L2;
     pers_ok = true;
 }
