@@ -1,5 +1,5 @@
 """The forms that the solver's operators take on grids past the one-launch limits (16,384 elements for the packed
-element-matrix products, 4,096 coarse elements for the restriction) and in their several shares of the work: two
+element-matrix products, 4,096 coarse elements for the restriction, 3,072 of span 4 in FP32) and in their several shares of the work: two
 and four coarse layers to a workgroup of the tiled restriction, 16 to 1 slices of the children in the super-element
 assembly, several entry tiles to a wavefront in the level-2 product.  The boxes are whole, so every operator has a
 closed form: the restriction is the transpose of a product of 1-D hat-function interpolations, and level 2 is
@@ -47,6 +47,7 @@ def _hats(coarse, fine):
 
 BOXES = [((104, 104, 104), False),    # level 2: 17,576 elements, two layers, two entry tiles
          ((16, 16, 4128), False),     # level 2: 4 x 4 x 1032 elements, four layers in both precisions
+         ((64, 56, 56), False),       # level 2: 3,136 elements, past FP32's limit of the restriction's one launch, not FP64's
          ((8, 8, 8), True), ((24, 24, 24), True), ((32, 32, 32), True), ((40, 40, 40), True),
          ((48, 48, 48), True)]        # 16, 8, 4, 2 slices and one; from 32^3 the finest level takes two launches
 

@@ -331,11 +331,13 @@ __global__ __launch_bounds__(256) void k_kelem_gather(const T *__restrict__ f, i
 // the two launches, but the chain is one of 72 loads and one launch instead of 300 and two.  Product at level 2 in
 // FP64 (FP32), us: 432 elements 7.6 (6.6) against 16.3 (11.5), 8,192 8.3 (7.0) against 16.9 (12.0), 12,800 11.5 (7.3)
 // against 17.6 (12.2), 20,736 19.6 (12.3) against 18.3 (13.4), 65,536 53 (31) against 32 (20); super-element
-// finest level, 16,384: 9.2 against 18.0.  So up to 16,384 elements.
+// finest level, 16,384: 9.2 against 18.0.  So up to 16,384 elements, where FP64 is even in a V-cycle (16,128 elements: 19.6
+// against 12.3 and 6.2 in two launches; FP32 is still ahead there, 12.5 against 8.4 and 6.2).
 // EPI_RESID_JAC0: the operand is x = omega r ./ diag, formed as it is loaded and written to xout (a launch fewer).
 // DOT (finest level): also the workgroup's share of u.out (product) or r.out (Jacobi step), to partial: a dot of its
 // own is two launches an iteration more, p.v another (the update finishes it).
 constexpr int KN_NODES = 64;
+constexpr int64_t KN_ELEMS = 1 << 14;
 template <typename T, int EPI, bool MASKED, bool DOT = false>
 __global__ __launch_bounds__(8 * KN_NODES) void k_kelem_node(const T *__restrict__ u, T *__restrict__ out,
                                                              const T *__restrict__ Kp, int64_t ldk,
@@ -530,11 +532,14 @@ __global__ __launch_bounds__(RT_THREADS) void k_restrict_tiled(const T *__restri
 
 // The restriction in one launch, for small coarse grids: k_restrict_tiled's planes and k_kelem_gather's sums by
 // (coarse node, element around it, plane, component), one thread each, in their order of operations (the same bits):
-// a thread forms its plane's 2D sum, the planes are folded and the eight elements added through LDS.  Its chain is one plane's loads where a workgroup of the tiled form
-// marches through nine; it reads every value for each of the elements and vertices it goes to.  Against the two
-// launches, us, FP64 (FP32), span 4: 432 coarse elements 6.3 (7.4) against 23 (19), 2,640 12.6 (13.4) against 24 (20),
-// 3,456 14.5 (17) against 24 (20), 8,192 27 (31) against 24 (19), 27,648 78 (85) against 27 (22); span 2: 54 elements 4.5
-// against 11, 3,456 7.2 against 14.  So up to 4,096 coarse elements.
+// a thread forms its plane's 2D sum, the planes are folded and the eight elements added through LDS.  Its chain is one
+// plane's loads where a workgroup of the tiled form marches through five (one coarse layer at these sizes); it reads
+// every value for each of the elements and vertices it goes to.  Span 4, us, FP64 (FP32), against the tiled kernel alone, to which a launch and a gather of 6 to 7 us come:
+// 1,024 coarse elements 8.7 (10.1) against 11.7 (9.0), 2,304 11.0 (13.3) against 11.4 (9.1), 3,136 13.8 (15.9) against
+// 11.6 (9.1), 4,096 18.5 (20.2) against 11.4 (9.0), 8,000 26.5 (29.9) against 11.7 (8.9); span 2: 1,728 elements 5.2
+// (5.2) against 5.3 (4.9), 3,328 7.1 (6.9) against 5.2 (4.9).  So up to 4,096 coarse elements, 3,072 of span 4 in FP32.
+template <typename T>
+constexpr int64_t rn_elems(int span) { return sizeof(T) == 8 || span == 2 ? 4096 : 3072; }
 constexpr int RN_NODES = 4;
 template <typename T, int S>
 __global__ __launch_bounds__(RN_NODES * 24 * (S + 1)) void k_restrict_node(const T *__restrict__ rf,

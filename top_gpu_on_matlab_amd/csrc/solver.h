@@ -86,12 +86,9 @@ struct Solver {
         return ktiles_for(lv[0].g, kfine_zchunk ? kfine_zchunk : kfine_auto[f64 || kfine_mfma ? 0 : 1]);
     }
     bool fine_tiled() const { return !super && kfine_kernel == 0 && walsh_ok; }
-    // Element-matrix products small enough for the one-launch form (k_kelem_node).
-    int64_t node_elems = 1 << 14;
     int cus = 0;  // compute units of the device
-    // restriction in one launch (k_restrict_node) on coarse grids up to this many elements
-    int64_t restrict_elems = 1 << 12;
-    bool elem_one_launch(const DevLevel &D) const { return D.ldk <= node_elems; }
+    // Element-matrix products small enough for the one-launch form (k_kelem_node).
+    static bool elem_one_launch(const DevLevel &D) { return D.ldk <= KN_ELEMS; }
     template <typename T>
     bool jac0_one_launch(const DevLevel &D) const {  // ... and with the packed matrices that it needs
         return elem_one_launch(D) && (sizeof(T) == 4 || (kelem_parts == 1 && D.Ks64p.n));

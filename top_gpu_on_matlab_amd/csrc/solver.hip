@@ -864,7 +864,7 @@ template <typename T>
 void Solver::restrict_level(int c, const T *rf, T *rc, const PlanePack *pk) {
     DevLevel &C = lv[c], &F = lv[c - 1];
     const uint8_t *cf = C.coeffCnt.p;
-    if (C.ldk <= restrict_elems) {
+    if (C.ldk <= rn_elems<T>(C.span)) {
         const unsigned gn = grid_for(C.g.nodes(), RN_NODES);
         const PlanePack none{};
         if (C.span == 4) k_restrict_node<T, 4><<<gn, RN_NODES * 24 * 5, 0, st>>>(rf, cf, C.g, F.g, C.eleMask, C.nodeMask, rc, pk ? *pk : none);
