@@ -177,7 +177,7 @@ __global__ __launch_bounds__(256) void k_galerkin_l2_mfma(const double *__restri
 // (at a stride of SPAN: the other children read those between), and products whose weights are all zero are
 // left out.  Children outside the mesh have zero matrices; children with boundary matrices (uid > 0, super-element
 // level 2) are left to k_galerkin_bnd.  Bound by reading the finer level's matrices: levels 3 and up at 128 x 256 x 128
-// (201 MB of them) 188 us, against 714 for one wavefront per element that gathered each child's 576 entries
+// (201 MB of them) 193 us, against 714 for one wavefront per element that gathered each child's 576 entries
 // singly; super-element level 2 of a 64 x 16 x 16 grid 63 with the slices' sum, against 477.
 template <int SPAN>
 __global__ __launch_bounds__(256) void k_galerkin_children(const double *__restrict__ prev, int64_t ldp,

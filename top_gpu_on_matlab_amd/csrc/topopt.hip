@@ -252,7 +252,7 @@ __device__ inline double oc_xnew(double x, double dc, double dv, double lmid, do
 // passive (may be null): entries with a nonzero indicator take xnew = 1 inside every step, so
 // they enter gt (xnew(passiveElements) = 1.0, TOP_GPU.m:239, 247).
 // Bound by the passes' two streams on large designs and by launches on small ones: 16 passes for 64 steps, 30 us each
-// at 4.2 million entries and 11 at 27,648, against 64 pairs of launches of 21 and 6 us.
+// at 4.2 million entries and 11 at 27,648, against 64 steps of two launches each, 21.6 us (17 and 4.6) and 6.2 a step.
 constexpr int OC_DEPTH = 4, OC_NODES = (1 << OC_DEPTH) - 1, OC_BLOCKS = 512;
 constexpr double OC_FLOOR = 1e9 * 0x1p-397;
 struct OcState {
@@ -505,7 +505,7 @@ struct FilterStep {
 // neighbours through LDS), with the next plane's loads in flight.  The element matrix has one entry per
 // distance of two corners, so a plane's part of an element's product is a sum over the quadrant of the 3x3
 // nodes around the column, and a layer of elements is two such parts: each plane is read and turned once.
-// Bound by memory: six streams of 8 bytes per node and the rims (128x256x128: 63 us, 3.5 TB/s without the
+// Bound by memory: six streams of 8 bytes per node and the rims (128x256x128: 63 us, 3.3 TB/s without the
 // rims; with k_filter_update's 19 an iteration takes 82 us, where nine launches took 200; 24x48x24: 6.6 and
 // 4.7 us).  512 threads a tile: 256 take 72 us, more of them being rim, and 1024 take 61 but 9.5 at 24x48x24.
 template <int IT>
