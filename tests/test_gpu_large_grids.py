@@ -96,3 +96,23 @@ def test_operators_past_the_small_grid_limits(shape, super_):
     del s
     mixed = _solver(shape, super_, 'mixed')
     assert _rel(mixed.vcycle(v), z) < 1e-4
+
+
+@pytest.mark.parametrize('shape', [(24, 24, 40), (72, 64, 64), (104, 104, 104)])
+def test_restriction_keeps_what_is_not_finite_where_it_has_a_weight(shape):
+    """A NaN or infinity of the fine residual on a plane of coarse nodes reaches coarse nodes of that plane alone, and between
+    two such planes those two alone: in one launch, and tiled with one and with two layers (levels 2 and 3)."""
+    import torch
+    s = _solver(shape, False, 'fp64')
+    dims = [(l['resY'], l['resX'], l['resZ']) for l in s.levels]
+    for level in range(2, s.num_levels + 1):
+        (fy, fx, fz), (cy, cx, cz) = dims[level - 2], dims[level - 1]
+        span = fz // cz
+        for z in (0, span, 2 * span, 2 * span + 1, 3 * span, fz):
+            for bad in (float('nan'), float('inf')):
+                r = _rand(s.ndof(level - 1), level).reshape(fz + 1, fx + 1, fy + 1, 3)
+                r[z, fx // 2, fy // 2] = bad
+                got = s.restrict(r.reshape(-1), level).reshape(cz + 1, -1)
+                hit = (~torch.isfinite(got)).any(dim=1).cpu().numpy()
+                near = np.abs(np.arange(cz + 1) * span - z) < span
+                assert np.array_equal(hit, near), (level, z, bad)

@@ -512,10 +512,11 @@ __global__ __launch_bounds__(RT_THREADS) void k_restrict_tiled(const T *__restri
             val += (jx ? (T)b / S : (T)(S - b) / S) * sy;
         }
         const int cz = (iz - iz0) % S;  // offset inside the current coarse layer
-        if (cz == 0 && iz > iz0) {
-            // this plane closes the layer below (top face, z weight 1) and opens the next one
+        if (cz == 0) {
+            // this plane closes the layer below (top face, z weight 1) and opens the next one, whose upper vertices have
+            // nothing of it (no product with their weight 0: what is not finite stays where it has a weight)
             acc1 += val;
-            if (own) {
+            if (own && iz > iz0) {
                 const int64_t e = ey + (int64_t)gc.EY * (ex + (int64_t)gc.EX * (e0z + (iz - iz0) / S - 1));
                 f[(int64_t)(3 * vtx_of(jy, jx, 0) + oc) * ldk + e] = acc0;
                 f[(int64_t)(3 * vtx_of(jy, jx, 1) + oc) * ldk + e] = acc1;
@@ -587,13 +588,13 @@ __global__ __launch_bounds__(RN_NODES * 24 * (S + 1)) void k_restrict_node(const
     if (t < 24 * RN_NODES) {
         const int o = t / (3 * RN_NODES);
         if (sOn[o][k]) {
-            T acc = 0;
+            T acc = o >> 2 ? sv[o][0][k][c] : (T)0;  // the element's lowest plane has z weight 1 (0 for its upper vertices)
 #pragma unroll
-            for (int pl = 0; pl < S; ++pl) {
+            for (int pl = 1; pl < S; ++pl) {
                 const T tz = (T)pl / S;
                 acc += (o >> 2 ? (T)1 - tz : tz) * sv[o][pl][k][c];
             }
-            if (!(o >> 2)) acc += sv[o][S][k][c];  // the element's top plane has z weight 1 (0 for its lower vertices)
+            if (!(o >> 2)) acc += sv[o][S][k][c];  // its top plane 1 (0 for its lower vertices)
             sf[o][k][c] = acc;
         }
     }
