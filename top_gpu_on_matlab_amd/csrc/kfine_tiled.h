@@ -205,7 +205,7 @@ __global__ __launch_bounds__(256, MF == 3 ? 2 : ((sizeof(T) == 8 || MF != 0) ? 3
     // FP64: diag is the reciprocal diagonal, one value per node (idiag64): the element matrix's diagonal entries are
     // all equal, and fixed DOFs, whose entry is 1, are known from the mask.  A third of the bytes and no divisions:
     // 128x256x128 146 from 165 us with the pre-smoothing, 119 from 133 with the Jacobi step.  (omega r) d and omega (r d)
-    // are equally accurate; the former rounds omega r as the damped step's own (omega (r - v)) / d does.
+    // round equally often, so either would do; whole runs differ between them as between any two roundings.
     constexpr bool ND = sizeof(T) == 8;
     __shared__ T sU[2][3][KT_PN];
     __shared__ uint8_t sM[2][KT_PN];
